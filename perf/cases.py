@@ -281,9 +281,12 @@ def prepare(case, seed):
                     ops.paged_gqa_decode(s["q"][l], s["kc"][l], s["vc"][l], s["table"], s["lens"], HD**-0.5, k_new=s["k"][l],
                                          v_new=s["v"][l], pages_per_split=pps, out=s["o"][l], ws=s["ws"])  # fmt: skip
 
+        # the state never holds both the graph and the closure over it: a cycle would leave the graph to the garbage
+        # collector, which may destroy it while another one is being recorded, an error that ends the process
         if case["graph"]:
             s["graph"] = _graph(layers)
-        s["call"] = layers
+        else:
+            s["call"] = layers
     elif kind == "step":
         d = _step_inputs(case, seed)
         gdn = [x for x in d["layers"] if not x["attn"]]
