@@ -236,3 +236,78 @@ def test_attention_negative_control(dev):
     wrong = O.bf16(O.gqa_decode(d["q"], d["k_cache"], d["v_cache"], d["block_table"], d["seq_lens"] - 1, d["scale"]))
     with pytest.raises(AssertionError):
         assert_attn_output(o, wrong)
+
+
+# Query rows per KV head past one MFMA tile of the rows kernel's ranges: 33 .. 48 and 49 .. 64 in one block of 3 or 4
+# tiles, 65 .. 96 and 97 .. 128 in two blocks; new rows that start a user's cache, end a page, cross pages and splits;
+# one and two page groups; one split, in-range and past the last page.
+@pytest.mark.parametrize(
+    "G,T,lens,pps",
+    [
+        (6, 6, [6, 64, 700], 2),  # 36 rows; the first user holds nothing but its new rows
+        (6, 8, [4099, 68, 1300], 8),  # 48 rows; new rows across pages, an odd page count per split
+        (6, 8, [130], 1),  # one page per split
+        (4, 13, [77, 640], 64),  # 52 rows, one split
+        (8, 8, [8, 1027], 3),  # 64 rows
+        (6, 11, [11, 138, 900], 2),  # 66 rows: two blocks of 3 tiles, 30 of them empty
+        (6, 16, [1040, 16], 1),  # 96 rows; 16 new rows over two pages, each its own split
+        (8, 13, [333], 4),  # 104 rows: two blocks of 4 tiles
+        (8, 16, [72, 1999], 2),  # 128 rows, the most
+    ],
+)
+@pytest.mark.parametrize("mixer", [False, True])
+def test_verify_row_blocks(dev, G, T, lens, pps, mixer):
+    B, nkv = len(lens), 4
+    d = W.attn_layer(B, max(lens), "cpu", seed=G * 100 + T + pps, T=T, num_blocks=512)
+    gen = torch.Generator().manual_seed(G + T)
+    d["q"] = torch.randn(B, T, G * nkv, 256, generator=gen).bfloat16()
+    d["seq_lens"] = torch.tensor(lens, dtype=torch.int32)
+    if not mixer:
+        o1, ref, same1 = run_case(dev, d, pps, fused=True)
+        o2, _, same2 = run_case(dev, d, pps, fused=False)
+        assert same1 and same2
+        assert torch.equal(o1.cpu(), o2.cpu())
+        assert_attn_output(o1, ref)
+        return
+    from conftest import bf16_ulp_mismatch
+
+    gate = torch.randn(d["q"].shape, generator=gen).bfloat16()
+    wq = (1 + 0.1 * torch.randn(256, generator=gen)) / 16.0
+    wk = 1 + 0.1 * torch.randn(256, generator=gen)
+    cos, sin = O.rope_tables((d["seq_lens"] - T)[:, None] + torch.arange(T)[None])
+    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+    o = ops.attn_mixer_decode(g["q"], g["k_new"], g["v_new"], gate.to(dev), wq.to(dev), wk.to(dev), cos.to(dev),
+                              sin.to(dev), g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"],
+                              pages_per_split=pps)  # fmt: skip
+    kc, vc = d["k_cache"].clone(), d["v_cache"].clone()
+    o_ref = O.attn_mixer(d["q"], d["k_new"], d["v_new"], gate, wq, wk, cos, sin, kc, vc, d["block_table"],
+                         d["seq_lens"])  # fmt: skip
+    assert torch.equal(g["v_cache"].cpu(), vc)
+    ulps, frac = bf16_ulp_mismatch(g["k_cache"].cpu(), kc)
+    assert ulps <= 1 and frac < 1e-3, (ulps, frac)
+    assert_attn_output(o, o_ref)
+
+
+def test_verify_row_blocks_idle_and_bad_page(dev):
+    """Two row blocks with an idle user and a page entry outside the pool: the idle user's rows are zero, the bad
+    page is reported and not attended, the others match the oracle."""
+    T, lens = 11, [500, 3, 900]
+    d = W.attn_layer(3, 900, "cpu", seed=7, T=T, num_blocks=64)
+    d["seq_lens"] = torch.tensor(lens, dtype=torch.int32)
+    o_ref = O.bf16(O.gqa_decode(d["q"], d["k_cache"], d["v_cache"], d["block_table"], d["seq_lens"], d["scale"]))
+    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+    g["block_table"][2, 5] = 64
+    st = ops.Status(dev)
+    o = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"],
+                             pages_per_split=2, status=st.word)  # fmt: skip
+    assert st.peek() == ops.STATUS_PAGE
+    assert_attn_output(o[0], o_ref[0])
+    assert int(o[1].count_nonzero()) == 0
+    keep = torch.ones(900, dtype=torch.bool)
+    keep[5 * 64 : 6 * 64] = False
+    rows = d["block_table"][2, :15].long()
+    K, V = (d[n][rows].permute(1, 0, 2, 3).reshape(4, -1, 256)[:, :900].float() for n in ("k_cache", "v_cache"))
+    for t in range(T):
+        seen = keep & (torch.arange(900) <= 900 - T + t)
+        s = (d["q"][2, t].float().view(4, 6, 256) @ K[:, seen].transpose(1, 2)) * d["scale"]
+        assert_attn_output(o[2, t].view(4, 6, 256), O.bf16(s.softmax(-1) @ V[:, seen]))

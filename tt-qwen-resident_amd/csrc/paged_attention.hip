@@ -7,14 +7,13 @@
 //   attn_wave_kernel  up to 16 query rows per KV head (every one-token decode): MFMA scores and P V, each
 //                     wave on its own 16-row slices with no barrier in the page loop, one or two pages in
 //                     flight per workgroup;
-//   attn_mfma_kernel  17 to 32 query rows (verify steps up to T = 5 at G = 6): MFMA, the 4 waves on the same
-//                     page, each wave owning a quarter of the head dims in P V;
-//   attn_kernel       more query rows: VALU dot products, the 4 waves on the same page.
+//   attn_rows_kernel  more query rows (verify steps): MFMA, 4 waves on a page, each wave owning a quarter of the
+//                     head dims in P V, one or two pages in flight, blocks of up to 64 query rows.
 // The step's new rows are loaded with the query rows and attended without a round trip through the pool:
 // the one-token kernel (up to two tokens) holds them in registers and patches them over the page rows they
-// replace (K through a one-row LDS copy when the page goes straight into the score operand), the MFMA kernel
-// (up to 8) stages them in LDS; both store them to the pool after the page loop. With the mixer or more
-// tokens they are appended first, by the wave that reads them back from the pool.
+// replace (K through a one-row LDS copy when the page goes straight into the score operand), the rows kernel
+// stages them in LDS; both store them to the pool after the page loop. The one-token kernel appends them first
+// with the mixer or more than two tokens, by the wave that reads them back from the pool.
 // The splits' partials (m, l, unnormalised O per query row) go to the workspace and are merged in split order
 // (the leader side of the reference: global max, rescale, sum, normalise, kernels/attn_leader_writer.cpp:
 // 86-106 and kernels/attn_leader_compute.cpp:42-79) by the last workgroup of the (user, KV head) to finish
@@ -128,9 +127,8 @@ __device__ __forceinline__ void report_page(const AttnArgs &a) {
     if (a.status) atomicOr(a.status, QS_STATUS_PAGE);
 }
 // Zero output rows of an inactive user for KV head g (all T G query rows; threads of one workgroup).
-template <int G, int NTH = 256>
-__device__ __forceinline__ void zero_rows(const AttnArgs &a, int b, int g, int tid) {
-    for (int idx = tid; idx < a.T * G * 32; idx += NTH) {
+__device__ __forceinline__ void zero_rows(const AttnArgs &a, int G, int b, int g, int tid, int nth) {
+    for (int idx = tid; idx < a.T * G * 32; idx += nth) {
         const int qr = idx >> 5, ch = idx & 31;
         *reinterpret_cast<uint4 *>(a.o + (((size_t)b * a.T + qr / G) * a.NQ + g * G + qr % G) * HD + ch * 8) =
             make_uint4(0, 0, 0, 0);
@@ -191,321 +189,12 @@ __device__ __forceinline__ u32x4 new_chunk(const AttnArgs &a, const uint16_t *ro
     return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
 }
 
-// One workgroup per (user, KV head, split); the 4 waves work on the same page at a time, wave w owning
-// rows 16 w .. 16 w + 15, so a page's K and V (16 KB per wave) are requested in one round trip:
-//   K   lane = (row 16 w + lane / 4, piece c = lane % 4): dims 32 i + 8 c .. + 7 for i < 8, 8 x 16-byte loads
-//   V   lane = head dims 4 lane .. 4 lane + 3, the wave's 16 rows (one 512-byte row per load instruction)
-// and the loaded page is reused for every query token of the group (TT tokens: the verify rows).
-template <int G, int TT, bool MIX>
-__global__ __launch_bounds__(256) void attn_kernel(AttnArgs a) {
-    constexpr int GP = (G + 3) & ~3;
-    const int nwg = a.B * a.NKV * a.nsplit;
-    const int lid = qs::xcd_logical(blockIdx.x, nwg);
-    const int split = lid % a.nsplit;
-    const int g = (lid / a.nsplit) % a.NKV;
-    const int b = lid / (a.nsplit * a.NKV);
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int T = a.T;
-
-    __shared__ __align__(16) uint16_t s_q[TT][G][HD];
-    __shared__ __align__(16) uint16_t s_ql[MIX ? TT : 1][G][HD];  // mixer: bf16 residues of the fp32 q
-    __shared__ __align__(16) uint32_t s_pp[4][8][GP];
-    __shared__ __align__(16) float s_acc[4][G][HD];
-    __shared__ float s_m[4][G], s_l[4][G];
-    __shared__ float s_w[4][G], s_L[G], s_M[G];
-
-    const int n = a.seq_lens[b];
-    if (!user_active(a, n, split == 0 && g == 0 && tid == 0)) {  // uniform over the user's workgroups
-        if (split == 0) zero_rows<G>(a, b, g, tid);
-        return;
-    }
-    const int base = n - T;  // first new position
-    const int npages = (n + BLK - 1) / BLK;
-    const int p0 = split * a.pps;
-    const int p1 = min(npages, p0 + a.pps);
-    const int *bt = a.block_table + (size_t)b * a.max_blocks;
-    // The split's block-table entries (at most 64), one per lane, read once up front: the page walk takes
-    // each page index with a readlane and never waits on a table read (a wait for one load would also
-    // wait for the K/V loads in flight).
-    const int bt_pre = p0 + lane < min(a.max_blocks, p0 + a.pps) ? bt[p0 + lane] : -1;  // issued before n is known
-    auto page_at = [&](int pi) {
-        const int pg = __builtin_amdgcn_readlane(bt_pre, pi - p0);
-        return (pg >= 0 && pg < a.num_blocks) ? pg : -1;
-    };
-    if (tid == 0)
-        for (int pi = p0; pi < p1; ++pi)
-            if (page_at(pi) < 0) report_page(a);
-
-    // Fused append, first: the new rows that fall in this split's pages go into the pools, and the stores
-    // complete before the barrier that precedes the page walk, so the walk reads every row - new ones
-    // included - from the pool. No other workgroup reads these pages.
-    if (a.k_new && p0 <= (n - 1) / BLK && base / BLK < p1) {
-        for (int idx = tid; idx < T * 64; idx += 256) {  // whole waves: T * 64 is a multiple of 64
-            const int t = idx >> 6, kv = (idx >> 5) & 1, ch = idx & 31;
-            const int pos = base + t, pi = pos / BLK;
-            const size_t src = (((size_t)b * T + t) * a.NKV + g) * HD + ch * 8;
-            uint4 u = *reinterpret_cast<const uint4 *>((kv ? a.v_new : a.k_new) + src);
-            if (a.wk) {  // k rows normalised and rotated (all lanes take part in the row reductions)
-                float y[8];
-                const size_t rc = ((size_t)b * T + t) * (a.rot / 2);
-                mixer_chunk(u, ch, a.wk, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
-                if (!kv) u = pack8(y);
-            }
-            if (pi < p0 || pi >= p1) continue;
-            const int pg = bt[pi];  // per thread: the new rows may straddle two pages
-            if (pg < 0 || pg >= a.num_blocks) continue;  // reported with the split's pages above
-            const size_t dst = (((size_t)pg * a.NKV + g) * BLK + (pos % BLK)) * HD + ch * 8;
-            *reinterpret_cast<uint4 *>((kv ? a.v_cache : a.k_cache) + dst) = u;
-        }
-        qs::wait_vmem();
-        __syncthreads();  // the rows are read by the wave that owns their 16-row slice (the branch is uniform)
-    }
-
-    const int kq = lane & 3;               // K: this lane's 16-byte piece of each 64-byte run of the row
-    const int krw = 16 * w + (lane >> 2);  // K: row of the page this lane scores
-    const size_t pstride = (size_t)a.NKV * BLK * HD;  // elements per page
-    const float sl2 = a.scale * 1.4426950408889634f;  // scores in the log2 domain: p = 2^(s scale log2e - m)
-    const int kvo = krw * HD * 2 + kq * 16;           // bytes: this lane's K piece in a head tile
-    const int vvo = 16 * w * HD * 2 + lane * 8;       // bytes: this lane's V dims in the wave's first row
-
-    // Page loads through a buffer descriptor based at the page's head tile (the per-page address work is
-    // scalar). A K buffer holds the wave's 16 K rows (4 lanes per row, 8 x 16 bytes per lane); a V buffer
-    // its 16 V rows, 4 dims per lane, rows 2 j and 2 j + 1 in entry j (.xy, .zw). Loads only issue here.
-    auto load_k = [&](int pg, uint4 (&kb)[8]) {
-        const auto rk = __builtin_amdgcn_make_buffer_rsrc(
-            qs::uniform_ptr(const_cast<uint16_t *>(a.k_cache + (size_t)pg * pstride + (size_t)g * BLK * HD)), (short)0,
-            BLK * HD * 2, 0x00020000);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rk, kvo, i * 64, NT);
-            kb[i] = make_uint4(x[0], x[1], x[2], x[3]);
-        }
-    };
-    auto load_v = [&](int pg, uint4 (&vb)[8]) {
-        const auto rv = __builtin_amdgcn_make_buffer_rsrc(
-            qs::uniform_ptr(const_cast<uint16_t *>(a.v_cache + (size_t)pg * pstride + (size_t)g * BLK * HD)), (short)0,
-            BLK * HD * 2, 0x00020000);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const u32x2 x0 = __builtin_amdgcn_raw_buffer_load_b64(rv, vvo, (2 * j) * HD * 2, NT);
-            const u32x2 x1 = __builtin_amdgcn_raw_buffer_load_b64(rv, vvo, (2 * j + 1) * HD * 2, NT);
-            vb[j] = make_uint4(x0[0], x0[1], x1[0], x1[1]);
-        }
-    };
-
-    for (int tg = 0; tg < T; tg += TT) {
-        const int nt = min(TT, T - tg);
-        const int vend = base + tg + nt;  // rows at or past vend are invalid for every token of the group
-        const int pe = min(p1, (vend + BLK - 1) / BLK);
-        // q of the token group: loaded into registers, then stored to LDS (normalised and rotated for the mixer)
-        constexpr int QCH = (TT * G * 32 + 255) / 256;
-        uint4 qreg[QCH];
-#pragma unroll
-        for (int k = 0; k < QCH; ++k) {
-            const int idx = tid + 256 * k;
-            const int tt = idx / (G * 32), hh = (idx / 32) % G, ch = idx & 31;
-            qreg[k] = make_uint4(0, 0, 0, 0);
-            if (idx < TT * G * 32 && tt < nt)
-                qreg[k] = *reinterpret_cast<const uint4 *>(a.q + (((size_t)b * T + tg + tt) * a.NQ + g * G + hh) * HD + ch * 8);
-        }
-        auto store_q = [&]() {
-            __syncthreads();  // the previous group's readers of s_q are done
-#pragma unroll
-            for (int k = 0; k < QCH; ++k) {
-                const int idx = tid + 256 * k;
-                const int tt = idx / (G * 32), hh = (idx / 32) % G, ch = idx & 31;
-                uint4 u = qreg[k];
-                if constexpr (MIX) {  // normalised and rotated q (all lanes take part in the row reductions)
-                    float y[8];
-                    const size_t rc = ((size_t)b * T + min(tg + tt, T - 1)) * (a.rot / 2);
-                    mixer_chunk(u, ch, a.wq, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
-                    u = pack8(y);
-                    if (idx < TT * G * 32) *reinterpret_cast<uint4 *>(&s_ql[tt][hh][ch * 8]) = pack8_lo(y, u);
-                }
-                if (idx < TT * G * 32) *reinterpret_cast<uint4 *>(&s_q[tt][hh][ch * 8]) = u;
-            }
-            __syncthreads();
-        };
-        store_q();
-
-        // m: running max (log2 domain, wave-uniform); lp: every lane adds its row's rounded probability (so
-        // the wave sum is 4x the row sum), reduced over the wave once per split
-        float m[TT][G], lp[TT][G], acc[TT][G][4];
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                m[tt][h] = -INFINITY;
-                lp[tt][h] = 0.f;
-                acc[tt][h][0] = acc[tt][h][1] = acc[tt][h][2] = acc[tt][h][3] = 0.f;
-            }
-
-        // zero the V rows past every token's window (a stale row times a zero probability could be NaN)
-        auto mask_v = [&](int pi, uint4 (&vb)[8]) {
-            const int rbase = pi * BLK + 16 * w;
-            if (rbase + 15 >= vend) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if (rbase + 2 * j >= vend) vb[j].x = vb[j].y = 0;
-                    if (rbase + 2 * j + 1 >= vend) vb[j].z = vb[j].w = 0;
-                }
-            }
-        };
-        // scores of page pi for token tg + tt, online softmax update, probabilities to s_pp
-        auto scores_tt = [&](int pi, int tt, const uint4 (&kv)[8]) {
-            const int P = pi * BLK + krw;
-            const bool okr = P < base + tg + tt + 1;  // token tg + tt sees positions 0 .. base + tg + tt
-            // this lane's row over its 64 dims, then across the row's 4 lanes (the q reads of the 4 lanes
-            // are 64 contiguous bytes; all 16 rows read the same q)
-            float sc[G];
-#pragma unroll
-            for (int h = 0; h < G; ++h) sc[h] = 0.f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-#pragma unroll
-                for (int h = 0; h < G; ++h) {
-                    const uint4 qv = *reinterpret_cast<const uint4 *>(&s_q[tt][h][i * 32 + kq * 8]);
-                    float d = sc[h];
-                    d = dot2(kv[i].x, qv.x, d);
-                    d = dot2(kv[i].y, qv.y, d);
-                    d = dot2(kv[i].z, qv.z, d);
-                    d = dot2(kv[i].w, qv.w, d);
-                    if constexpr (MIX) {
-                        const uint4 ql = *reinterpret_cast<const uint4 *>(&s_ql[tt][h][i * 32 + kq * 8]);
-                        d = dot2(kv[i].x, ql.x, d);
-                        d = dot2(kv[i].y, ql.y, d);
-                        d = dot2(kv[i].z, ql.z, d);
-                        d = dot2(kv[i].w, ql.w, d);
-                    }
-                    sc[h] = d;
-                }
-            }
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                sc[h] += qs::dpp<0xB1>(sc[h]);
-                sc[h] += qs::dpp<0x4E>(sc[h]);
-            }
-            // online softmax over the wave's 16 rows (log2 domain; the max is taken on the raw scores, the
-            // scale being positive); probabilities rounded to bf16 (the running sum adds the rounded values,
-            // so the normalisation matches what P V uses) and packed two rows per dword for P V
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                const float mn = fmaxf(m[tt][h], qs::wave_max_bcast(okr ? sc[h] : -INFINITY) * sl2);
-                const float e = okr ? __builtin_amdgcn_exp2f(fmaf(sc[h], sl2, -mn)) : 0.f;
-                const uint32_t pk = qs::cvt_pk_bf16(e, qs::dpp<0x104>(e));  // this row | the next row
-                if (mn != m[tt][h]) {  // wave-uniform: rescale only when the running max moved
-                    const float alpha = m[tt][h] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[tt][h] - mn);
-                    lp[tt][h] *= alpha;
-                    acc[tt][h][0] *= alpha;
-                    acc[tt][h][1] *= alpha;
-                    acc[tt][h][2] *= alpha;
-                    acc[tt][h][3] *= alpha;
-                    m[tt][h] = mn;
-                }
-                lp[tt][h] += __uint_as_float(pk << 16);
-                if ((lane & 7) == 0) s_pp[w][lane >> 3][h] = pk;
-            }
-            __builtin_amdgcn_wave_barrier();
-        };
-        // P V of the page for token tg + tt: two rows per v_dot2 (interleaved with v_perm)
-        auto pv_tt = [&](int tt, const uint4 (&vb)[8]) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t x0 = __builtin_amdgcn_perm(vb[j].z, vb[j].x, 0x05040100u);
-                const uint32_t x1 = __builtin_amdgcn_perm(vb[j].z, vb[j].x, 0x07060302u);
-                const uint32_t x2 = __builtin_amdgcn_perm(vb[j].w, vb[j].y, 0x05040100u);
-                const uint32_t x3 = __builtin_amdgcn_perm(vb[j].w, vb[j].y, 0x07060302u);
-                uint32_t pr[GP];
-#pragma unroll
-                for (int h4 = 0; h4 < GP; h4 += 4) {
-                    const uint4 p4 = *reinterpret_cast<const uint4 *>(&s_pp[w][j][h4]);
-                    pr[h4] = p4.x, pr[h4 + 1] = p4.y, pr[h4 + 2] = p4.z, pr[h4 + 3] = p4.w;
-                }
-#pragma unroll
-                for (int h = 0; h < G; ++h) {
-                    acc[tt][h][0] = dot2(pr[h], x0, acc[tt][h][0]);
-                    acc[tt][h][1] = dot2(pr[h], x1, acc[tt][h][1]);
-                    acc[tt][h][2] = dot2(pr[h], x2, acc[tt][h][2]);
-                    acc[tt][h][3] = dot2(pr[h], x3, acc[tt][h][3]);
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        };
-
-        // the accumulators of TT tokens leave no registers for pages in flight
-        for (int pi = p0; pi < pe; ++pi) {
-            const int pg = page_at(pi);
-            if (pg < 0) continue;
-            uint4 X[8], Y[8];
-            load_k(pg, X);
-            load_v(pg, Y);
-            mask_v(pi, Y);
-#pragma unroll
-            for (int tt = 0; tt < TT; ++tt) {
-                if (tt >= nt) break;
-                scores_tt(pi, tt, X);
-                pv_tt(tt, Y);
-            }
-        }
-
-        // ---- merge the 4 waves, token by token; one partial (or the output) per token and split
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-            if (tt >= nt) break;
-            const int t = tg + tt;
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                const float lw = 0.25f * qs::wave_sum_dpp(lp[tt][h]);
-                *reinterpret_cast<float4 *>(&s_acc[w][h][lane * 4]) =
-                    make_float4(acc[tt][h][0], acc[tt][h][1], acc[tt][h][2], acc[tt][h][3]);
-                if (lane == 0) {
-                    s_m[w][h] = m[tt][h];
-                    s_l[w][h] = lw;
-                }
-            }
-            __syncthreads();
-            if (tid < G) {
-                float M = -INFINITY;
-                for (int ww = 0; ww < 4; ++ww) M = fmaxf(M, s_m[ww][tid]);
-                float L = 0.f;
-                for (int ww = 0; ww < 4; ++ww) {
-                    const float e = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[ww][tid] - M);
-                    s_w[ww][tid] = e;
-                    L += e * s_l[ww][tid];
-                }
-                s_M[tid] = M;
-                s_L[tid] = L;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                const float O = s_w[0][h] * s_acc[0][h][tid] + s_w[1][h] * s_acc[1][h][tid] +
-                                s_w[2][h] * s_acc[2][h][tid] + s_w[3][h] * s_acc[3][h][tid];
-                if (a.nsplit == 1) {
-                    const size_t oi = (((size_t)b * T + t) * a.NQ + g * G + h) * HD + tid;
-                    const float gt = a.gate ? sigm(qs::bf2f(a.gate[oi])) : 1.0f;
-                    a.o[oi] = (uint16_t)qs::f2bf(O / s_L[h] * gt);
-                }
-                else
-                    a.part_o[prow(a, G, b, g, split, t * G + h) * HD + tid] = O;
-            }
-            if (a.nsplit > 1 && tid < G) {
-                float *ml = a.part_ml + prow(a, G, b, g, split, t * G + tid) * 2;
-                ml[0] = s_M[tid];
-                ml[1] = s_L[tid];
-            }
-            __syncthreads();
-        }
-    }
-}
-
 // ------------------------------------------------------------------------------ shared by the MFMA kernels
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr int QPAD = HD + 8;   // s_q row pitch (bf16): 16-byte skew between rows
 constexpr int VPAD = HD + 16;  // K / V slice row pitch (bf16): 32-byte skew between rows
-constexpr int PPAD = 16 + 4;   // s_p row pitch (bf16)
 
 // Split merge inside the attention launch (nsplit <= MERGE_MAX). Every workgroup of (user b, KV head g) has
 // stored its partial with agent-coherent stores (sc1: written through the XCD's L2); each thread waits for
@@ -517,8 +206,9 @@ constexpr int PPAD = 16 + 4;   // s_p row pitch (bf16)
 // invalidate is needed because only sc1 accesses touch the shared data. (The leader side of the
 // reference: kernels/attn_leader_writer.cpp:86-106, kernels/attn_leader_compute.cpp:42-79.)
 constexpr int MERGE_MAX = 16;
-template <int G, int NWV = 4>
-__device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int b, int g, int tid) {
+constexpr int MERGE_ROWS = 32;  // query rows per KV head up to which one workgroup merges
+template <int NWV>
+__device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b, int g, int tid) {
     __shared__ int s_last;
     qs::wait_vmem();
     __syncthreads();
@@ -583,217 +273,208 @@ __device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int b, int g,
 }
 
 // ------------------------------------------------------------------------------ MFMA kernel (verify rows)
-// For T query tokens the T * G query rows of a KV head form a dense [T G x 256] x [256 x rows] product, so
-// the multi-token (verify) step runs it on MFMA. One workgroup per (user, KV head, split of pps pages),
-// walking its pages in order. Per page, in two phases separated by a barrier:
-//   scores  wave w takes rows 16 w .. 16 w + 15 (a 16-row slice): S^T [16 rows x 16 q] = K Q^T on 8
-//           v_mfma_f32_16x16x32_bf16 per 16-query-row tile (lane l holds K row l % 16, dims 32 j + 8 (l / 16)
-//           .. + 7: one 16-byte load per j), the slice's own max m_s per query row (log2 domain), P^T =
-//           2^(s - m_s) rounded to bf16 and its row sums l_s into LDS; the slice's V rows into LDS;
-//   P V     every wave adds the 4 slices in order to O^T [its 64 head dims x 16 q] on
-//           v_mfma_f32_16x16x16_bf16 (V^T read from LDS with the transposing ds_read_b64_tr_b16, P^T as
-//           written), scaled by 2^(m_s - M) against the running max M; M moves only when a slice max exceeds
-//           it by 2^8, so the accumulators are rarely rescaled.
-// All waves see the same slice maxima in the same order, so M and the sum L agree across waves, and the
-// 4 waves' head dims are disjoint: the split's partial needs no cross-wave merge.
-template <int G, int QT, bool MIX>
-__global__ __launch_bounds__(256) void attn_mfma_kernel(AttnArgs a) {
-    constexpr int NQR = 16 * QT;
-    const int nwg = a.B * a.NKV * a.nsplit;
+// For T query tokens the T G query rows of a KV head form a dense [T G x 256] x [256 x rows] product. One
+// workgroup per (user, KV head, split of pps pages, block of 16 QT query rows) with WPP groups of 4 waves: group
+// ph walks pages p0 + ph, p0 + ph + WPP, ... (WPP pages in flight), every group in step. Per page, two barriers:
+//   scores  wave w takes rows 16 w .. + 15 of the page: S^T [16 rows x 16 q] = K Q^T on 8
+//           v_mfma_f32_16x16x32_bf16 per query tile (lane l holds K row l % 16, dims 32 j + 8 (l / 16) .. + 7,
+//           loaded in that layout), its rows' max per query row into LDS;                            barrier
+//   softmax the page's max per query row from the 4 waves; the running max M (log2 domain, the same in all 4
+//           waves) moves only when the page exceeds it by 2^8 (the accumulators are then rescaled); P^T =
+//           2^(s - M) as bf16 hi + lo into LDS beside the page's V rows, the fp32 values summed per wave;
+//                                                                                                    barrier
+//   P V     every wave adds the page to O^T [its 64 head dims x 16 q]: four v_mfma_f32_16x16x32_bf16 per tile,
+//           V^T read with the transposing ds_read_b64_tr_b16, accumulated by the MFMA itself.
+// With one max per page fixed before P is formed, P V is a plain accumulation: no per-slice products to scale
+// and add, no branch between the slices' LDS reads. The V rows and P^T are written after the first barrier and
+// read after the second, so one buffer of each serves every page. P keeps its rounding residue: with bf16 alone
+// and no row of the page exactly 1 it is off by 1.6e-3 of the output (0.8e-3 against each 16-row slice's own max),
+// and the second product costs 3% (B 4 / 4100 positions / T 8 / pps 8: 33.7 against 32.5 us a layer).
+// Bound by the chain of a page: about 7000 cycles a page pair (stamps: K requests and scores 2000, maxima and
+// barrier 1500, V and P into LDS 2000, P V 1400), both waves of a SIMD in the same phase; the scores of pages
+// without new rows skip the masks. Measured per layer, G 6: B 4 / 4100 positions ragged / T 8 / pps 8 163 -> 35 us
+// against VALU dot products with two tokens a pass; B 1 / 8192 / T 4 / pps 2 with the mixer 24.9 -> 21.7 us against
+// the pages one at a time with a scaled product per 16-row slice (17.4 us without the mixer either way).
+// The step's new rows (mixer: k normalised and rotated) are requested with the query rows and staged in LDS by
+// the workgroups whose split holds their pages; they take the place of the pool's rows as the page is used (K in
+// the score operand's registers, V as it is staged) and go to the pool after the page loop, so nothing waits for
+// a store, no page is read twice, and the other row blocks of the split never depend on those stores.
+// At the end the WPP groups' O meet in LDS, each group finishing its share of the query tiles.
+constexpr int T_MAX = 16;
+constexpr int PP = BLK + 8;  // s_p row pitch (bf16)
+template <int QT, bool MIX, int WPP>
+struct RowsLds {
+    static constexpr int NQR = 16 * QT, NW = 4 * WPP;
+    static constexpr int TN = QT == 3 && MIX && WPP == 2 ? 8 : T_MAX;  // new tokens a call may bring (the LDS limit)
+    static constexpr int Q = NQR * QPAD * 2, QL = MIX ? Q : 0, V = NW * 16 * VPAD * 2, P = 2 * WPP * NQR * PP * 2;
+    static constexpr int NEW = TN * 2 * HD * 2, ML = NW * NQR * 4;
+    static constexpr int bytes = Q + QL + V + P + NEW + 2 * ML;
+    static_assert(bytes <= 163840, "LDS");
+    static_assert(NQR * HD * 4 <= V || WPP == 1, "the groups' O exchange reuses the V rows");
+};
+template <int QT, bool MIX, int WPP>
+__global__ __launch_bounds__(256 * WPP) void attn_rows_kernel(AttnArgs a, int G, int nrb) {
+    using S = RowsLds<QT, MIX, WPP>;
+    constexpr int NQR = S::NQR, NTH = 256 * WPP;
+    // Q^T fragments in registers for the split where they fit beside the page's rows and the accumulators; else
+    // read from LDS per page (the mixer's residues always)
+    constexpr bool QREG = QT == 2;
+    const int nwg = a.B * a.NKV * a.nsplit * nrb;
     const int lid = qs::xcd_logical(blockIdx.x, nwg);
-    const int split = lid % a.nsplit;
-    const int g = (lid / a.nsplit) % a.NKV;
-    const int b = lid / (a.nsplit * a.NKV);
-    // the wave index through readfirstlane: the compiler then knows the wave's page and slice tests are uniform
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rb = lid % nrb;  // the row blocks of a split are neighbours: its pages come from L2 for all but one
+    const int split = (lid / nrb) % a.nsplit;
+    const int g = (lid / (nrb * a.nsplit)) % a.NKV;
+    const int b = lid / (nrb * a.nsplit * a.NKV);
+    // the wave index through readfirstlane: the compiler then knows the wave's page and row tests are uniform
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int w = wv & 3, ph = wv >> 2;
     const int l16 = lane & 15, lg = lane >> 4;
-    const int T = a.T;
+    const int T = a.T, R = T * G, r0 = rb * NQR;
 
-    __shared__ __align__(16) uint16_t s_q[NQR][QPAD];
-    __shared__ __align__(16) uint16_t s_ql[MIX ? NQR : 1][QPAD];  // mixer: bf16 residues of the fp32 q
-    __shared__ __align__(16) uint16_t s_v[4][16][VPAD];     // the page's V rows, slice by slice
-    __shared__ __align__(16) uint16_t s_p[4][QT][16][PPAD];  // P^T of each slice: [query row][slice row]
-    __shared__ float s_m[4][NQR], s_l[4][NQR];              // slice max (log2 domain) and row sum
-    // Fused append from registers and LDS (up to TN tokens, no mixer): the new rows are requested with the
-    // query rows, staged in LDS with them, written over the page's rows as those are used (K in the registers
-    // of the score operand, V as it is staged) and stored to the pool after the page loop, so nothing waits for
-    // a store and no page is read twice.
-    constexpr int TN = MIX ? 0 : (32 / G < 8 ? 32 / G : 8);
-    __shared__ __align__(16) uint16_t s_new[TN > 0 ? TN : 1][2][HD];  // token t's new K and V rows
+    __shared__ __align__(16) unsigned char s_raw[S::bytes];
+    auto s_q = reinterpret_cast<uint16_t (*)[QPAD]>(s_raw);
+    auto s_ql = reinterpret_cast<uint16_t (*)[QPAD]>(s_raw + S::Q);
+    auto s_v = reinterpret_cast<uint16_t (*)[VPAD]>(s_raw + S::Q + S::QL) + 64 * ph;  // the group's page of V rows
+    auto s_p = reinterpret_cast<uint16_t (*)[PP]>(s_raw + S::Q + S::QL + S::V) + 2 * NQR * ph;  // hi rows, lo rows
+    auto s_new = reinterpret_cast<uint16_t (*)[2][HD]>(s_raw + S::Q + S::QL + S::V + S::P);
+    auto s_m = reinterpret_cast<float (*)[4]>(s_raw + S::Q + S::QL + S::V + S::P + S::NEW) + NQR * ph;  // [row][wave]
+    auto s_l = reinterpret_cast<float (*)[NQR]>(s_raw + S::Q + S::QL + S::V + S::P + S::NEW + S::ML);
+    auto s_o = reinterpret_cast<f32x4_t *>(s_raw + S::Q + S::QL);
 
-    // Issued first, in this order: the split's block-table entries, the user's length and the query rows.
-    // The first page's K / V loads then wait only for the table entries, not for the length.
+    // Issued first, in this order: the split's block-table entries, the user's length, the query rows and the
+    // new rows. The first page's K / V loads then wait only for the table entries, not for the length.
     const int p0 = split * a.pps;
-    const int *bt = a.block_table + (size_t)b * a.max_blocks;
     const int bt_pre = split_entries(a, b, p0, lane);
-    int n = a.seq_lens[b];
-    // query rows qr = t G + hh (zero past T G): loaded into registers now, stored to LDS once the first
-    // page's loads are in flight
-    constexpr int QCH = NQR * 32 / 256;
+    const int n = a.seq_lens[b];
+    constexpr int QCH = NQR * 32 / NTH, NCH = S::TN * 64 / NTH;
     uint4 qreg[QCH];
 #pragma unroll
     for (int k = 0; k < QCH; ++k) {
-        const int idx = tid + 256 * k;
-        qreg[k] = q_chunk(a, G, b, g, idx >> 5, idx & 31);
+        const int idx = tid + NTH * k;
+        qreg[k] = q_chunk(a, G, b, g, r0 + (idx >> 5), idx & 31);
     }
-    // the new rows, chunk tid % 32 of token tid / 32 (zeros past T, or with more than TN tokens)
-    const bool fresh = a.k_new && T <= TN;
-    u32x4 nkc = {0u, 0u, 0u, 0u}, nvc = {0u, 0u, 0u, 0u};
-    if constexpr (TN > 0) {
-        nkc = new_chunk(a, fresh ? a.k_new : nullptr, b, g, tid >> 5, tid & 31);
-        nvc = new_chunk(a, fresh ? a.v_new : nullptr, b, g, tid >> 5, tid & 31);
+    // the new rows of tokens wv, wv + 4 WPP, ...: chunk lane % 32 of the K row (lanes < 32) or the V row (zeros past T)
+    u32x4 nk[NCH], nv[NCH];
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+        nk[k] = new_chunk(a, a.k_new, b, g, wv + 4 * WPP * k, lane < 32 ? lane : -1);
+        nv[k] = new_chunk(a, a.v_new, b, g, wv + 4 * WPP * k, lane < 32 ? -1 : lane - 32);
     }
-
     auto page_at = [&](int pi) {
         const int pg = __builtin_amdgcn_readlane(bt_pre, pi - p0);
         return (pg >= 0 && pg < a.num_blocks) ? pg : -1;
     };
     const size_t pstride = (size_t)a.NKV * BLK * HD;  // elements per page
-
     // a page of -1 is an empty range: the loads still issue (no branch around them, so the compiler's waits
     // stay exact) and read zeros without touching memory
-    auto load_k = [&](int pg, uint4 (&kb)[8]) {
+    auto load_k = [&](int pg, u32x4 (&kb)[8]) {
         const auto rk = __builtin_amdgcn_make_buffer_rsrc(
             qs::uniform_ptr(const_cast<uint16_t *>(a.k_cache + (size_t)max(pg, 0) * pstride + (size_t)g * BLK * HD)),
             (short)0, pg >= 0 ? BLK * HD * 2 : 0, 0x00020000);
         const int off = (16 * w + l16) * HD * 2 + lg * 16;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rk, off, j * 64, NT);
-            kb[j] = make_uint4(x[0], x[1], x[2], x[3]);
-        }
+        for (int j = 0; j < 8; ++j) kb[j] = __builtin_amdgcn_raw_buffer_load_b128(rk, off, j * 64, NT);
     };
-    auto load_v = [&](int pg, uint4 (&vb)[8]) {
+    auto load_v = [&](int pg, u32x4 (&vb)[8]) {
         const auto rv = __builtin_amdgcn_make_buffer_rsrc(
             qs::uniform_ptr(const_cast<uint16_t *>(a.v_cache + (size_t)max(pg, 0) * pstride + (size_t)g * BLK * HD)),
             (short)0, pg >= 0 ? BLK * HD * 2 : 0, 0x00020000);
         const int off = (16 * w + (lane >> 5)) * HD * 2 + (lane & 31) * 16;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rv, off, k * 1024, NT);
-            vb[k] = make_uint4(x[0], x[1], x[2], x[3]);
-        }
+        for (int k = 0; k < 8; ++k) vb[k] = __builtin_amdgcn_raw_buffer_load_b128(rv, off, k * 1024, NT);
     };
 
-    // the first page's rows, before the length is known: a page in the pool's range that turns out to lie
-    // past the user's length is simply not used
-    uint4 KA[8], VA[8];
-    const int pg0 = p0 < a.max_blocks ? page_at(p0) : -1;
-    load_k(pg0, KA);
-    load_v(pg0, VA);
+    // the group's first page, before the length is known: a page in the pool's range that turns out to lie past
+    // the user's length is simply not used
+    u32x4 kb[8], vb[8];
+    const int pf = p0 + ph;
+    const int pg0 = pf < min(a.max_blocks, p0 + a.pps) ? page_at(pf) : -1;
+    load_k(pg0, kb);
+    load_v(pg0, vb);
 
-    if (!user_active(a, n, split == 0 && g == 0 && tid == 0)) {  // uniform over the user's workgroups
-        if (split == 0) zero_rows<G>(a, b, g, tid);
+    if (!user_active(a, n, split == 0 && g == 0 && rb == 0 && tid == 0)) {  // uniform over the user's workgroups
+        if (split == 0 && rb == 0) zero_rows(a, G, b, g, tid, NTH);
         return;
     }
     const int base = n - T;  // first new position
-    const int npages = (n + BLK - 1) / BLK;
-    const int p1 = min(npages, p0 + a.pps);
+    const int p1 = min((n + BLK - 1) / BLK, p0 + a.pps);
     // an entry of the split's pages outside the pool (lane pi - p0 checks entry pi) is reported after the
     // page loop: an atomic here, inside a branch, would make the compiler wait for every load at the next use
     const bool bad_pages = __any(lane < p1 - p0 && (bt_pre < 0 || bt_pre >= a.num_blocks));
+    const bool fresh = a.k_new && base / BLK < p1 && (n - 1) / BLK >= p0;  // new rows in this split (uniform)
 
-    // Fused append otherwise (more tokens, or the mixer's normalised and rotated k rows), first: wave w writes
-    // the new rows of its 16-row slices in this split's pages and waits for them, so its slice loads read them
-    // back from the pool. No other wave reads these slices.
-    if (a.k_new && !fresh && p0 < p1 && base / BLK < p1 && (n - 1) / BLK >= p0) {
-        for (int idx = lane; idx < T * 64; idx += 64) {
-            const int t = idx >> 6, kv = (idx >> 5) & 1, ch = idx & 31;
-            const int pos = base + t, pi = pos / BLK;
-            const size_t src = (((size_t)b * T + t) * a.NKV + g) * HD + ch * 8;
-            uint4 u = *reinterpret_cast<const uint4 *>((kv ? a.v_new : a.k_new) + src);
-            if (a.wk) {  // k rows normalised and rotated (all lanes take part in the row reductions)
+    // query rows (and the mixer's residues) and new rows into LDS
+#pragma unroll
+    for (int k = 0; k < QCH; ++k) {
+        const int idx = tid + NTH * k, row = idx >> 5, ch = idx & 31;
+        uint4 u = qreg[k];
+        if constexpr (MIX) {  // normalised and rotated q (all lanes take part in the row reductions)
+            float y[8];
+            const size_t rc = ((size_t)b * T + min((r0 + row) / G, T - 1)) * (a.rot / 2);
+            mixer_chunk(u, ch, a.wq, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
+            u = pack8(y);
+            *reinterpret_cast<uint4 *>(&s_ql[row][ch * 8]) = pack8_lo(y, u);
+        }
+        *reinterpret_cast<uint4 *>(&s_q[row][ch * 8]) = u;
+    }
+    if (fresh)
+#pragma unroll
+        for (int k = 0; k < NCH; ++k) {
+            const int t = wv + 4 * WPP * k;
+            if (t >= T) break;
+            const u32x4 x = lane < 32 ? nk[k] : nv[k];
+            uint4 u = make_uint4(x[0], x[1], x[2], x[3]);
+            if constexpr (MIX) {  // k rows normalised and rotated; the V lanes take part in the shuffles only
                 float y[8];
                 const size_t rc = ((size_t)b * T + t) * (a.rot / 2);
-                mixer_chunk(u, ch, a.wk, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
-                if (!kv) u = pack8(y);
+                mixer_chunk(u, lane & 31, a.wk, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
+                if (lane < 32) u = pack8(y);
             }
-            if (pi < p0 || pi >= p1 || (pos % BLK) / 16 != w) continue;
-            const int pg = bt[pi];
-            if (pg < 0 || pg >= a.num_blocks) continue;  // reported with the split's pages above
-            const size_t dst = (((size_t)pg * a.NKV + g) * BLK + (pos % BLK)) * HD + ch * 8;
-            *reinterpret_cast<uint4 *>((kv ? a.v_cache : a.k_cache) + dst) = u;
+            *reinterpret_cast<uint4 *>(&s_new[t][lane >> 5][(lane & 31) * 8]) = u;
         }
-        qs::wait_vmem();
-        if (pg0 >= 0 && base / BLK <= p0) {  // new rows landed in the first page: read it again
-            load_k(pg0, KA);
-            load_v(pg0, VA);
-        }
-    }
+    __syncthreads();
+    bf16x8_t qr[QREG ? QT : 1][QREG ? 8 : 1];
+    if constexpr (QREG)
+#pragma unroll
+        for (int nt = 0; nt < QT; ++nt)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                qr[nt][j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(&s_q[16 * nt + l16][32 * j + 8 * lg]));
 
     const float sl2 = a.scale * 1.4426950408889634f;  // log2 domain
-    int lim[QT];  // the lane's causal limit per query-row tile: token qr / G sees positions <= base + token
+    int lim[QT];           // the lane's causal limit per query tile: token qr / G sees positions <= base + token
+    f32x4_t oacc[QT][4];   // O^T of head dims 64 w + 16 dd + 4 lg + i (dd < 4), query row r0 + 16 nt + l16
+    float M[QT], L[QT];    // running max (the same in the group's 4 waves) and this wave's rows' sum
 #pragma unroll
     for (int nt = 0; nt < QT; ++nt) {
-        const int qr = l16 + 16 * nt;
-        lim[nt] = qr < T * G ? base + qr / G : -1;
-    }
-
-    f32x4_t oacc[QT][4];  // O^T of head dims 64 w + 16 dd + 4 lg + i (dd < 4), query row l16 + 16 nt
-    float M[QT], L[QT];
-#pragma unroll
-    for (int nt = 0; nt < QT; ++nt) {
+        const int row = r0 + 16 * nt + l16;
+        lim[nt] = row < R ? base + row / G : -1;
         M[nt] = -INFINITY;
         L[nt] = 0.f;
 #pragma unroll
         for (int dd = 0; dd < 4; ++dd) oacc[nt][dd] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
 
-    // Q^T fragments (query row l16 + 16 nt, dims 32 j + 8 lg .. + 7), held in registers for the split once
-    // the query rows are staged (with the mixer, whose residues double them, they are read from LDS per page)
-    bf16x8_t qbr[MIX ? 1 : QT][MIX ? 1 : 8];
-
-    // one page: scores of this wave's slice into LDS, barrier, every slice's P V into this wave's dims,
-    // barrier. kb / vb hold the page's K and V rows; each is refilled with the next page's rows as soon as
-    // it has been consumed (V after staging, K after the score MFMAs), so one buffer of each suffices.
-    auto page = [&](int pi, uint4 (&kb)[8], uint4 (&vb)[8]) {
-        const int pgn = pi + 1 < p1 ? page_at(pi + 1) : -1;
-        const bool ok = page_at(pi) >= 0;
-        const int r0w = pi * BLK + 16 * w;  // first position of this wave's slice
-        // V rows (zero where the page is invalid or past the user's length: a stale row times a zero
-        // probability could be NaN)
-        // new rows in this wave's slice of the page (uniform): token pos - base at slice row pos - r0w; their
-        // LDS reads are issued together, ahead of the staging
-        const bool has_new = TN > 0 && fresh && ok && r0w + 16 > base && r0w < n;
-        auto stage_v = [&](const u32x4 (&x)[8], bool patch) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int row = 2 * k + (lane >> 5), pos = r0w + row;
-                const bool live = ok && pos < n;
-                u32x4 v = {live ? vb[k].x : 0u, live ? vb[k].y : 0u, live ? vb[k].z : 0u, live ? vb[k].w : 0u};
-                if (patch) v = live && pos >= base ? x[k] : v;
-                *reinterpret_cast<u32x4 *>(&s_v[w][row][(lane & 31) * 8]) = v;
-            }
-        };
-        if (TN > 0 && has_new) {
+    // every group takes the same number of steps (the barriers are the workgroup's); a group past its last page
+    // works on an empty one
+    for (int s0 = p0; s0 < p1; s0 += WPP) {
+        const int pi = s0 + ph;
+        const int pgn = pi + WPP < p1 ? page_at(pi + WPP) : -1;
+        const bool ok = pi < p1 && page_at(pi) >= 0;
+        const int r0w = pi * BLK + 16 * w;  // first position of this wave's rows
+        // new rows among this wave's rows (uniform): token pos - base at row pos - r0w
+        const bool has_new = fresh && ok && r0w + 16 > base && r0w < n;
+        if (has_new) {  // the new K row at this lane's row over the pool's (dims 32 j + 8 lg)
+            const int t = r0w + l16 - base;
+            const bool kp = t >= 0 && t < T;
             u32x4 x[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int t = r0w + 2 * k + (lane >> 5) - base;
-                x[k] = *reinterpret_cast<const u32x4 *>(&s_new[min(max(t, 0), TN > 0 ? TN - 1 : 0)][1][(lane & 31) * 8]);
-            }
-            stage_v(x, true);
-        } else {
-            const u32x4 x[8] = {};
-            stage_v(x, false);
+            for (int j = 0; j < 8; ++j) x[j] = *reinterpret_cast<const u32x4 *>(&s_new[min(max(t, 0), T - 1)][0][32 * j + 8 * lg]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) kb[j][e] = kp ? x[j][e] : kb[j][e];
         }
-        load_v(pgn, vb);
-        if constexpr (TN > 0)
-            if (has_new) {  // the new K row at this lane's row l16 of the slice, over the pool's (dims 32 j + 8 lg)
-                const int t = r0w + l16 - base;
-                const bool kp = t >= 0 && r0w + l16 < n;
-                u32x4 x[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    x[j] = *reinterpret_cast<const u32x4 *>(&s_new[min(max(t, 0), TN - 1)][0][32 * j + 8 * lg]);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    kb[j].x = kp ? x[j][0] : kb[j].x;
-                    kb[j].y = kp ? x[j][1] : kb[j].y;
-                    kb[j].z = kp ? x[j][2] : kb[j].z;
-                    kb[j].w = kp ? x[j][3] : kb[j].w;
-                }
-            }
         f32x4_t sacc[QT];
 #pragma unroll
         for (int nt = 0; nt < QT; ++nt) sacc[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -803,152 +484,217 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
             for (int nt = 0; nt < QT; ++nt) {
                 bf16x8_t bq;
-                if constexpr (MIX)
-                    bq = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(&s_q[l16 + 16 * nt][32 * j + 8 * lg]));
+                if constexpr (QREG)
+                    bq = qr[nt][j];
                 else
-                    bq = qbr[nt][j];
+                    bq = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(&s_q[16 * nt + l16][32 * j + 8 * lg]));
                 sacc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ak, bq, sacc[nt], 0, 0, 0);
                 if constexpr (MIX) {
                     const bf16x8_t bl = __builtin_bit_cast(
-                        bf16x8_t, *reinterpret_cast<const uint4 *>(&s_ql[l16 + 16 * nt][32 * j + 8 * lg]));
+                        bf16x8_t, *reinterpret_cast<const uint4 *>(&s_ql[16 * nt + l16][32 * j + 8 * lg]));
                     sacc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ak, bl, sacc[nt], 0, 0, 0);
                 }
             }
         }
         load_k(pgn, kb);
-#pragma unroll
-        for (int nt = 0; nt < QT; ++nt) {
-            float sc[4];
-            float mx = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                sc[i] = ok && r0w + 4 * lg + i <= lim[nt] ? sacc[nt][i] : -INFINITY;
-                mx = fmaxf(mx, sc[i]);
-            }
-            mx = qs::xor32_max(qs::xor16_max(mx));
-            const float ms = mx * sl2;  // -inf when no row of the slice is visible to this query row
-            float e[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) e[i] = sc[i] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(fmaf(sc[i], sl2, -ms));
-            const uint32_t p01 = qs::cvt_pk_bf16(e[0], e[1]), p23 = qs::cvt_pk_bf16(e[2], e[3]);
-            *reinterpret_cast<uint2 *>(&s_p[w][nt][l16][4 * lg]) = make_uint2(p01, p23);
-            float ls = (qs::bf_lo(p01) + qs::bf_hi(p01)) + (qs::bf_lo(p23) + qs::bf_hi(p23));
-            ls = qs::xor32_sum(qs::xor16_sum(ls));
-            if (lg == 0) {
-                s_m[w][l16 + 16 * nt] = ms;
-                s_l[w][l16 + 16 * nt] = ls;
-            }
-        }
-        __syncthreads();
-        // P V: the 4 slices in order into this wave's head dims
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            i16x4_t av[4];
-#pragma unroll
-            for (int dd = 0; dd < 4; ++dd)
-                av[dd] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t *)&s_v[q][4 * lg + (l16 >> 2)][16 * (4 * w + dd) + 4 * (l16 & 3)]);
+        // every row of the page lies before the step's new rows: no masks, no patches (uniform; query rows past R
+        // then take part unmasked, into outputs that are never stored)
+        const bool full = ok && (pi + 1) * BLK <= base;
+        // the scores in the log2 domain, -inf where masked, and their max over this wave's 16 rows
+        float mx[QT];
+        if (full) {
 #pragma unroll
             for (int nt = 0; nt < QT; ++nt) {
-                const float ms = s_m[q][l16 + 16 * nt], ls = s_l[q][l16 + 16 * nt];
-                const bool move = M[nt] == -INFINITY ? ms != -INFINITY : ms > M[nt] + 8.0f;
-                const float Mn = move ? ms : M[nt];
-                if (__any(move)) {
-                    const float alpha = M[nt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M[nt] - Mn);
-                    L[nt] *= alpha;
+                sacc[nt] *= sl2;
+                mx[nt] = fmaxf(fmaxf(sacc[nt][0], sacc[nt][1]), fmaxf(sacc[nt][2], sacc[nt][3]));
+            }
+        } else {
 #pragma unroll
-                    for (int dd = 0; dd < 4; ++dd) oacc[nt][dd] *= alpha;
-                }
-                M[nt] = Mn;
-                const float es = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - Mn);
-                L[nt] = fmaf(es, ls, L[nt]);
-                const i16x4_t pb = __builtin_bit_cast(i16x4_t, *reinterpret_cast<const uint2 *>(&s_p[q][nt][l16][4 * lg]));
+            for (int nt = 0; nt < QT; ++nt) {
+                mx[nt] = -INFINITY;
 #pragma unroll
-                for (int dd = 0; dd < 4; ++dd) {
-                    const f32x4_t z = {0.f, 0.f, 0.f, 0.f};
-                    const f32x4_t pv = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[dd], pb, z, 0, 0, 0);
-                    oacc[nt][dd] += es * pv;
+                for (int i = 0; i < 4; ++i) {
+                    sacc[nt][i] = ok && r0w + 4 * lg + i <= lim[nt] ? sacc[nt][i] * sl2 : -INFINITY;
+                    mx[nt] = fmaxf(mx[nt], sacc[nt][i]);
                 }
             }
         }
-        __syncthreads();  // the next page's scores overwrite s_v, s_p, s_m, s_l
-    };
-
 #pragma unroll
-    for (int k = 0; k < QCH; ++k) {
-        const int idx = tid + 256 * k, qr = idx >> 5, ch = idx & 31;
-        uint4 u = qreg[k];
-        if constexpr (MIX) {  // normalised and rotated q (all lanes take part in the row reductions)
-            float y[8];
-            const size_t rc = ((size_t)b * T + min(qr / G, T - 1)) * (a.rot / 2);
-            mixer_chunk(u, ch, a.wq, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
-            u = pack8(y);
-            *reinterpret_cast<uint4 *>(&s_ql[qr][ch * 8]) = pack8_lo(y, u);
-        }
-        *reinterpret_cast<uint4 *>(&s_q[qr][ch * 8]) = u;
-    }
-    if constexpr (TN > 0)
-        if (tid < TN * 32) {
-            *reinterpret_cast<u32x4 *>(&s_new[tid >> 5][0][(tid & 31) * 8]) = nkc;
-            *reinterpret_cast<u32x4 *>(&s_new[tid >> 5][1][(tid & 31) * 8]) = nvc;
-        }
-    __syncthreads();
-    if constexpr (!MIX)
+        for (int nt = 0; nt < QT; ++nt) mx[nt] = qs::xor32_max(qs::xor16_max(mx[nt]));
+        if (lg == 0)
 #pragma unroll
-        for (int nt = 0; nt < QT; ++nt)
+            for (int nt = 0; nt < QT; ++nt) s_m[16 * nt + l16][w] = mx[nt];
+        __syncthreads();  // the page's maxima are in LDS, and the previous page's V and P are no longer read
+        f32x4_t pm[QT];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                qbr[nt][j] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(&s_q[l16 + 16 * nt][32 * j + 8 * lg]));
-    for (int pi = p0; pi < p1; ++pi) page(pi, KA, VA);
-    if (bad_pages && tid == 0) report_page(a);
-    if constexpr (TN > 0)
-        if (fresh)  // the new rows of this wave's slices into the pool (lanes < 32 the K row, the others the V row)
+        for (int nt = 0; nt < QT; ++nt) pm[nt] = *reinterpret_cast<const f32x4_t *>(&s_m[16 * nt + l16][0]);
+        // V rows (zero where the page is invalid or past the user's length: a stale row times a zero
+        // probability could be NaN), the new ones over the pool's
+        if (full) {
 #pragma unroll
-            for (int t = 0; t < TN; ++t) {
-                const int pos = base + t, pi = pos / BLK;
-                if (t >= T || pi < p0 || pi >= p1 || (pos % BLK) / 16 != w) continue;
-                const int pg = page_at(pi);
-                if (pg < 0) continue;  // reported with the split's pages
-                const size_t row = (((size_t)pg * a.NKV + g) * BLK + pos % BLK) * HD + (lane & 31) * 8;
-                *reinterpret_cast<u32x4 *>((lane < 32 ? a.k_cache : a.v_cache) + row) =
-                    *reinterpret_cast<const u32x4 *>(&s_new[t][lane >> 5][(lane & 31) * 8]);
+            for (int k = 0; k < 8; ++k) *reinterpret_cast<u32x4 *>(&s_v[16 * w + 2 * k + (lane >> 5)][(lane & 31) * 8]) = vb[k];
+        } else {
+            u32x4 x[8] = {};
+            if (has_new)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int t = r0w + 2 * k + (lane >> 5) - base;
+                    x[k] = *reinterpret_cast<const u32x4 *>(&s_new[min(max(t, 0), T - 1)][1][(lane & 31) * 8]);
+                }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int row = 2 * k + (lane >> 5), pos = r0w + row;
+                const bool live = ok && pos < n, patch = has_new && live && pos >= base;
+                u32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = patch ? x[k][e] : live ? vb[k][e] : 0u;
+                *reinterpret_cast<u32x4 *>(&s_v[16 * w + row][(lane & 31) * 8]) = v;
             }
-
-    // this wave's head dims of the split's partial (or of the output); the partials are written through
-    // to the agent-coherent level (sc1), where another workgroup of this launch or the merge launch reads them
-    const auto rpo = __builtin_amdgcn_make_buffer_rsrc(a.part_o + prow(a, G, b, g, split, 0) * HD, (short)0,
-                                                       T * G * HD * 4, 0x00020000);
-    const auto rpm = __builtin_amdgcn_make_buffer_rsrc(a.part_ml + prow(a, G, b, g, split, 0) * 2, (short)0,
-                                                       T * G * 8, 0x00020000);
+        }
+        load_v(pgn, vb);
+        float Mn[QT];
+        bool move = false;
 #pragma unroll
-    for (int nt = 0; nt < QT; ++nt) {
-        const int qr = l16 + 16 * nt;
-        if (qr >= T * G) continue;
-        const int t = qr / G, hh = qr % G;
-        if (a.nsplit == 1) {
-            const float inv = 1.0f / L[nt];
-            const size_t oi = (((size_t)b * T + t) * a.NQ + g * G + hh) * HD + 64 * w + 4 * lg;
+        for (int nt = 0; nt < QT; ++nt) {
+            const float m4 = fmaxf(fmaxf(pm[nt][0], pm[nt][1]), fmaxf(pm[nt][2], pm[nt][3]));
+            Mn[nt] = m4 > M[nt] + 8.0f ? m4 : M[nt];  // from -inf: to any finite maximum
+            move |= Mn[nt] != M[nt];
+        }
+        if (__any(move))
+#pragma unroll
+            for (int nt = 0; nt < QT; ++nt) {
+                const float alpha = M[nt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M[nt] - Mn[nt]);
+                L[nt] *= alpha;
+#pragma unroll
+                for (int dd = 0; dd < 4; ++dd) oacc[nt][dd] *= alpha;
+                M[nt] = Mn[nt];
+            }
+#pragma unroll
+        for (int nt = 0; nt < QT; ++nt) {
+            const float Ms = M[nt] == -INFINITY ? 0.f : M[nt];  // nothing visible yet: every 2^(-inf - 0) is 0
+            float e[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) e[i] = __builtin_amdgcn_exp2f(sacc[nt][i] - Ms);
+            const uint32_t p01 = qs::cvt_pk_bf16(e[0], e[1]), p23 = qs::cvt_pk_bf16(e[2], e[3]);
+            const uint32_t l01 = qs::cvt_pk_bf16(e[0] - qs::bf_lo(p01), e[1] - qs::bf_hi(p01));
+            const uint32_t l23 = qs::cvt_pk_bf16(e[2] - qs::bf_lo(p23), e[3] - qs::bf_hi(p23));
+            *reinterpret_cast<uint2 *>(&s_p[16 * nt + l16][16 * w + 4 * lg]) = make_uint2(p01, p23);
+            *reinterpret_cast<uint2 *>(&s_p[NQR + 16 * nt + l16][16 * w + 4 * lg]) = make_uint2(l01, l23);
+            L[nt] += (e[0] + e[1]) + (e[2] + e[3]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            bf16x8_t pb[2][QT];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int nt = 0; nt < QT; ++nt)
+                    pb[h][nt] = __builtin_bit_cast(
+                        bf16x8_t, *reinterpret_cast<const uint4 *>(&s_p[h * NQR + 16 * nt + l16][32 * kk + 8 * lg]));
 #pragma unroll
             for (int dd = 0; dd < 4; ++dd) {
-                f32x4_t v = oacc[nt][dd] * inv;
+                i16x4_t av[2];  // V^T: head dim l16 of the tile, page rows 32 kk + 8 lg + 4 h .. + 3
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    av[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t *)&s_v[32 * kk + 8 * lg + 4 * h + (l16 >> 2)][64 * w + 16 * dd + 4 * (l16 & 3)]);
+                const u32x2 a0 = __builtin_bit_cast(u32x2, av[0]), a1 = __builtin_bit_cast(u32x2, av[1]);
+                const bf16x8_t va = __builtin_bit_cast(bf16x8_t, u32x4{a0[0], a0[1], a1[0], a1[1]});
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int nt = 0; nt < QT; ++nt)
+                        oacc[nt][dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[h][nt], oacc[nt][dd], 0, 0, 0);
+            }
+        }
+    }
+
+    if (bad_pages && rb == 0 && tid == 0) report_page(a);
+    if (fresh && rb == 0)  // the new rows into the pool (lanes < 32 the K row, the others the V row)
+        for (int t = wv; t < T; t += 4 * WPP) {
+            const int pos = base + t, pi = pos / BLK;
+            if (pi < p0 || pi >= p1) continue;
+            const int pg = page_at(pi);
+            if (pg < 0) continue;  // reported with the split's pages
+            const size_t row = (((size_t)pg * a.NKV + g) * BLK + pos % BLK) * HD + (lane & 31) * 8;
+            *reinterpret_cast<u32x4 *>((lane < 32 ? a.k_cache : a.v_cache) + row) =
+                *reinterpret_cast<const u32x4 *>(&s_new[t][lane >> 5][(lane & 31) * 8]);
+        }
+
+    // the waves' row sums and the groups' maxima
+#pragma unroll
+    for (int nt = 0; nt < QT; ++nt) {
+        const float ls = qs::xor32_sum(qs::xor16_sum(L[nt]));
+        if (lg == 0) {
+            s_l[wv][16 * nt + l16] = ls;
+            if (w == 0) s_m[16 * nt + l16][0] = M[nt];
+        }
+    }
+    __syncthreads();
+    auto mine = [&](int nt) { return WPP == 1 || (nt < (QT + 1) / 2) == (ph == 0); };  // tiles this group finishes
+    float sc[QT], Mx[QT], Lx[QT];  // this group's scale, and the split's max and sum of each row
+#pragma unroll
+    for (int nt = 0; nt < QT; ++nt) {
+        const int row = 16 * nt + l16;
+        const float lo = ((s_l[4 * ph][row] + s_l[4 * ph + 1][row]) + s_l[4 * ph + 2][row]) + s_l[4 * ph + 3][row];
+        Mx[nt] = M[nt], Lx[nt] = lo, sc[nt] = 1.f;
+        if constexpr (WPP == 2) {
+            const int po = 4 * (1 - ph);
+            const float mo = s_m[(1 - 2 * ph) * NQR + row][0];  // s_m is based at the own group's rows
+            const float l2 = ((s_l[po][row] + s_l[po + 1][row]) + s_l[po + 2][row]) + s_l[po + 3][row];
+            Mx[nt] = fmaxf(M[nt], mo);
+            sc[nt] = M[nt] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M[nt] - Mx[nt]);
+            Lx[nt] = sc[nt] * lo + (mo == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mo - Mx[nt])) * l2;
+            if (!mine(nt))
+#pragma unroll
+                for (int dd = 0; dd < 4; ++dd) s_o[((nt * 4 + w) * 4 + dd) * 64 + lane] = oacc[nt][dd] * sc[nt];
+        }
+    }
+    if constexpr (WPP == 2) __syncthreads();
+
+    // this wave's head dims of the group's tiles of the split's partial (or of the output); the partials are
+    // written through to the agent-coherent level (sc1), where another workgroup of this launch or the merge
+    // launch reads them
+    const auto rpo = __builtin_amdgcn_make_buffer_rsrc(a.part_o + prow(a, G, b, g, split, 0) * HD, (short)0,
+                                                       R * HD * 4, 0x00020000);
+    const auto rpm = __builtin_amdgcn_make_buffer_rsrc(a.part_ml + prow(a, G, b, g, split, 0) * 2, (short)0,
+                                                       R * 8, 0x00020000);
+#pragma unroll
+    for (int nt = 0; nt < QT; ++nt) {
+        const int row = r0 + 16 * nt + l16;
+        if (!mine(nt) || row >= R) continue;
+        f32x4_t v[4];
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd) {
+            v[dd] = oacc[nt][dd] * sc[nt];
+            if constexpr (WPP == 2) v[dd] += s_o[((nt * 4 + w) * 4 + dd) * 64 + lane];
+        }
+        if (a.nsplit == 1) {
+            const float inv = 1.0f / Lx[nt];
+            const size_t oi = (((size_t)b * T + row / G) * a.NQ + g * G + row % G) * HD + 64 * w + 4 * lg;
+#pragma unroll
+            for (int dd = 0; dd < 4; ++dd) {
+                v[dd] *= inv;
                 if (a.gate) {
                     const uint2 gw = *reinterpret_cast<const uint2 *>(a.gate + oi + 16 * dd);
-                    v[0] *= sigm(qs::bf_lo(gw.x)), v[1] *= sigm(qs::bf_hi(gw.x));
-                    v[2] *= sigm(qs::bf_lo(gw.y)), v[3] *= sigm(qs::bf_hi(gw.y));
+                    v[dd][0] *= sigm(qs::bf_lo(gw.x)), v[dd][1] *= sigm(qs::bf_hi(gw.x));
+                    v[dd][2] *= sigm(qs::bf_lo(gw.y)), v[dd][3] *= sigm(qs::bf_hi(gw.y));
                 }
                 *reinterpret_cast<uint2 *>(a.o + oi + 16 * dd) =
-                    make_uint2(qs::cvt_pk_bf16(v[0], v[1]), qs::cvt_pk_bf16(v[2], v[3]));
+                    make_uint2(qs::cvt_pk_bf16(v[dd][0], v[dd][1]), qs::cvt_pk_bf16(v[dd][2], v[dd][3]));
             }
         } else {
 #pragma unroll
             for (int dd = 0; dd < 4; ++dd)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, oacc[nt][dd]), rpo,
-                                                       (qr * HD + 64 * w + 16 * dd + 4 * lg) * 4, 0, qs::CP_SC1);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[dd]), rpo,
+                                                       (row * HD + 64 * w + 16 * dd + 4 * lg) * 4, 0, qs::CP_SC1);
             if (w == 0 && lg == 0)
-                __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(M[nt]), __float_as_uint(L[nt])}, rpm,
-                                                      qr * 8, 0, qs::CP_SC1);
+                __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(Mx[nt]), __float_as_uint(Lx[nt])}, rpm,
+                                                      row * 8, 0, qs::CP_SC1);
         }
     }
-    if (a.nsplit > 1 && a.nsplit <= MERGE_MAX) merge_in_launch<G>(a, b, g, tid);
+    if constexpr (NQR <= MERGE_ROWS)
+        if (a.nsplit > 1 && a.nsplit <= MERGE_MAX) merge_in_launch<NTH / 64>(a, G, b, g, tid);
 }
 
 // ------------------------------------------------------------------- MFMA kernel, independent waves
@@ -1064,7 +810,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
     load_rows(a.v_cache, pg0, VA);
 
     if (!user_active(a, n, split == 0 && g == 0 && tid == 0)) {  // uniform over the user's workgroups
-        if (split == 0) zero_rows<G, NTH>(a, b, g, tid);
+        if (split == 0) zero_rows(a, G, b, g, tid, NTH);
         return;
     }
     const int base = n - T;
@@ -1378,7 +1124,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(Mr), __float_as_uint(Lr)}, rpm, tid * 8, 0,
                                               qs::CP_SC1);
     }
-    if (a.nsplit > 1 && a.nsplit <= MERGE_MAX) merge_in_launch<G, NWV>(a, b, g, tid);
+    if (a.nsplit > 1 && a.nsplit <= MERGE_MAX) merge_in_launch<NWV>(a, G, b, g, tid);
 }
 
 // Merge of the splits of one output row (user, token, query head) in one memory round trip: wave w sums
@@ -1510,52 +1256,47 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
     }
     const dim3 grid(B * NKV * ns);
     hipStream_t st = QS_STREAM(stream);
-    // up to 32 query rows per KV head (every one-token decode, and verify steps with T G <= 32) run on MFMA;
-    // more rows take the VALU kernel, two query tokens per pass over the pages
-    if (T * G <= 32) {
-        const int QT = (T * G + 15) / 16;
-        // two pages in flight per workgroup (8 waves) when the split has more than one page
+    QS_REQUIRE(G == 1 || G == 2 || G == 4 || G == 6 || G == 8, "%s: group size NQ/NKV = %d not in {1, 2, 4, 6, 8}", who, G);
+    const int R = T * G;
+    if (R <= 16) {  // every one-token decode
         const int wpp = attn_wpp(pages_per_split);
-#define QS_WAVE(GG, W, MX) attn_wave_kernel<GG, W, MX><<<grid, 256 * W, 0, st>>>(a)
-#define QS_MFMA_LAUNCH(GG)                                                              \
-    if (a.wq) {                                                                         \
-        if (QT == 1) { if (wpp == 1) QS_WAVE(GG, 1, true); else QS_WAVE(GG, 2, true); }  \
-        else attn_mfma_kernel<GG, 2, true><<<grid, 256, 0, st>>>(a);                    \
-    } else {                                                                            \
-        if (QT == 1) { if (wpp == 1) QS_WAVE(GG, 1, false); else QS_WAVE(GG, 2, false); } \
-        else attn_mfma_kernel<GG, 2, false><<<grid, 256, 0, st>>>(a);                   \
+#define QS_WAVE(GG)                                                              \
+    if (a.wq) {                                                                  \
+        if (wpp == 1) attn_wave_kernel<GG, 1, true><<<grid, 256, 0, st>>>(a);    \
+        else attn_wave_kernel<GG, 2, true><<<grid, 512, 0, st>>>(a);             \
+    } else {                                                                     \
+        if (wpp == 1) attn_wave_kernel<GG, 1, false><<<grid, 256, 0, st>>>(a);   \
+        else attn_wave_kernel<GG, 2, false><<<grid, 512, 0, st>>>(a);            \
     }
         switch (G) {
-            case 1: QS_MFMA_LAUNCH(1) break;
-            case 2: QS_MFMA_LAUNCH(2) break;
-            case 4: QS_MFMA_LAUNCH(4) break;
-            case 6: QS_MFMA_LAUNCH(6) break;
-            case 8: QS_MFMA_LAUNCH(8) break;
-            default: QS_REQUIRE(false, "%s: group size NQ/NKV = %d not in {1, 2, 4, 6, 8}", who, G);
+            case 1: QS_WAVE(1) break;
+            case 2: QS_WAVE(2) break;
+            case 4: QS_WAVE(4) break;
+            case 6: QS_WAVE(6) break;
+            default: QS_WAVE(8) break;
         }
-#undef QS_MFMA_LAUNCH
 #undef QS_WAVE
-        if (int e = qs::launch_status(who)) return e;
-        if (ns > MERGE_MAX) {  // fewer splits are merged inside the attention launch
-            attn_merge_kernel<<<B * T * NKV * G, 256, 0, st>>>(a, G);
-            return qs::launch_status(who);
+    } else {
+        // query rows in blocks of 16 QT, QT the fewest tiles that cover them in as few blocks as 4 tiles would
+        const int nrb = (R + 63) / 64, QT = (R + 16 * nrb - 1) / (16 * nrb);
+        QS_REQUIRE((long)grid.x * nrb < (1L << 31), "%s: grid too large", who);
+        const dim3 rgrid(grid.x * nrb);
+        const bool two = pages_per_split >= 2;
+        // the new rows of more than 8 tokens leave no LDS for the second group of 3 tiles with the mixer's residues
+#define QS_ROWS(Q, MX, W) attn_rows_kernel<Q, MX, W><<<rgrid, 256 * W, 0, st>>>(a, G, nrb)
+        if (a.wq) {  // with 4 tiles and the mixer's residues LDS has room for one page group only
+            if (QT == 2) { if (two) QS_ROWS(2, true, 2); else QS_ROWS(2, true, 1); }
+            else if (QT == 3) { if (two && T <= 8) QS_ROWS(3, true, 2); else QS_ROWS(3, true, 1); }
+            else QS_ROWS(4, true, 1);
+        } else {
+            if (QT == 2) { if (two) QS_ROWS(2, false, 2); else QS_ROWS(2, false, 1); }
+            else if (QT == 3) { if (two) QS_ROWS(3, false, 2); else QS_ROWS(3, false, 1); }
+            else { if (two) QS_ROWS(4, false, 2); else QS_ROWS(4, false, 1); }
         }
-        return QS_OK;
+#undef QS_ROWS
     }
-#define QS_ATTN_LAUNCH(GG)                                \
-    if (a.wq) attn_kernel<GG, 2, true><<<grid, 256, 0, st>>>(a); \
-    else attn_kernel<GG, 2, false><<<grid, 256, 0, st>>>(a);
-    switch (G) {
-        case 1: QS_ATTN_LAUNCH(1) break;
-        case 2: QS_ATTN_LAUNCH(2) break;
-        case 4: QS_ATTN_LAUNCH(4) break;
-        case 6: QS_ATTN_LAUNCH(6) break;
-        case 8: QS_ATTN_LAUNCH(8) break;
-        default: QS_REQUIRE(false, "%s: group size NQ/NKV = %d not in {1, 2, 4, 6, 8}", who, G);
-    }
-#undef QS_ATTN_LAUNCH
     if (int e = qs::launch_status(who)) return e;
-    if (ns > 1) {
+    if (ns > 1 && (ns > MERGE_MAX || R > MERGE_ROWS)) {  // the rest are merged inside the attention launch
         attn_merge_kernel<<<B * T * NKV * G, 256, 0, st>>>(a, G);
         return qs::launch_status(who);
     }
