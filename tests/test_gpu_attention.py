@@ -269,23 +269,43 @@ def test_verify_row_blocks(dev, G, T, lens, pps, mixer):
         assert torch.equal(o1.cpu(), o2.cpu())
         assert_attn_output(o1, ref)
         return
+    check_mixer(dev, d, pps, 64, gen)
+
+
+def check_mixer(dev, d, pps, rot, gen):
+    """The mixer's call against the oracle: appended K rows within one bf16 ulp, V rows bit-exact, the output."""
     from conftest import bf16_ulp_mismatch
 
+    T = d["q"].shape[1]
     gate = torch.randn(d["q"].shape, generator=gen).bfloat16()
     wq = (1 + 0.1 * torch.randn(256, generator=gen)) / 16.0
     wk = 1 + 0.1 * torch.randn(256, generator=gen)
-    cos, sin = O.rope_tables((d["seq_lens"] - T)[:, None] + torch.arange(T)[None])
+    cos, sin = O.rope_tables((d["seq_lens"] - T)[:, None] + torch.arange(T)[None], rot) if rot else (None, None)
     g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
-    o = ops.attn_mixer_decode(g["q"], g["k_new"], g["v_new"], gate.to(dev), wq.to(dev), wk.to(dev), cos.to(dev),
-                              sin.to(dev), g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"],
-                              pages_per_split=pps)  # fmt: skip
+    tab = [t.to(dev) if rot else None for t in (cos, sin)]
+    o = ops.attn_mixer_decode(g["q"], g["k_new"], g["v_new"], gate.to(dev), wq.to(dev), wk.to(dev), *tab, g["k_cache"],
+                              g["v_cache"], g["block_table"], g["seq_lens"], pages_per_split=pps, rot=rot)  # fmt: skip
     kc, vc = d["k_cache"].clone(), d["v_cache"].clone()
+    if not rot:
+        cos, sin = torch.ones(*d["q"].shape[:2], 8), torch.zeros(*d["q"].shape[:2], 8)  # the identity rotation
     o_ref = O.attn_mixer(d["q"], d["k_new"], d["v_new"], gate, wq, wk, cos, sin, kc, vc, d["block_table"],
-                         d["seq_lens"])  # fmt: skip
+                         d["seq_lens"], rot=rot or 16)  # fmt: skip
     assert torch.equal(g["v_cache"].cpu(), vc)
     ulps, frac = bf16_ulp_mismatch(g["k_cache"].cpu(), kc)
     assert ulps <= 1 and frac < 1e-3, (ulps, frac)
     assert_attn_output(o, o_ref)
+
+
+# The mixer's new rows, normalised, rotated and staged before the page loop: one and two tokens (held in LDS), three
+# and more (through the pool, or the rows kernel), each with one and two pages in flight; a user with nothing but its
+# new rows, rows that end, start and cross a page; every rotation width.
+@pytest.mark.parametrize("T,lens,pps", [(1, [1, 64, 65, 700], 8), (1, [65, 128], 1), (2, [2, 65, 333], 4),
+                                        (2, [129, 64], 1), (4, [66, 4], 2), (4, [193], 1)])  # fmt: skip
+@pytest.mark.parametrize("rot", [0, 16, 256])
+def test_mixer_new_rows(dev, T, lens, pps, rot):
+    d = W.attn_layer(len(lens), max(lens), "cpu", seed=T + pps + rot, T=T, num_blocks=64)
+    d["seq_lens"] = torch.tensor(lens, dtype=torch.int32)
+    check_mixer(dev, d, pps, rot, torch.Generator().manual_seed(T + rot))
 
 
 def test_verify_row_blocks_idle_and_bad_page(dev):

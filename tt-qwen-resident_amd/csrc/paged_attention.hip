@@ -11,9 +11,9 @@
 //                     head dims in P V, one or two pages in flight, blocks of up to 64 query rows.
 // The step's new rows are loaded with the query rows and attended without a round trip through the pool:
 // the one-token kernel (up to two tokens) holds them in registers and patches them over the page rows they
-// replace (K through a one-row LDS copy when the page goes straight into the score operand), the rows kernel
-// stages them in LDS; both store them to the pool after the page loop. The one-token kernel appends them first
-// with the mixer or more than two tokens, by the wave that reads them back from the pool.
+// replace (K through a one-row LDS copy when the page goes straight into the score operand), the rows kernel,
+// and with the mixer the one-token kernel, stages them in LDS; both store them to the pool after the page loop. The
+// one-token kernel appends more than two tokens first, by the wave that reads them back from the pool.
 // The splits' partials (m, l, unnormalised O per query row) go to the workspace and are merged in split order
 // (the leader side of the reference: global max, rescale, sum, normalise, kernels/attn_leader_writer.cpp:
 // 86-106 and kernels/attn_leader_compute.cpp:42-79) by the last workgroup of the (user, KV head) to finish
@@ -31,6 +31,7 @@ constexpr int NT = 2;
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c,
@@ -59,12 +60,39 @@ struct AttnArgs {
     float eps;
 };
 
+// The mixer's tables for one 8-element chunk, requested ahead of the page loads: read where they are used they
+// queue behind the launch's first page burst (B 1 / 8192 positions / T 4, stamps: query and new rows staged 12500
+// cycles after the length, 5500 without the mixer). With the new rows attended from LDS too, per layer: B 1 / 8192 /
+// T 4 / pps 2 21.0 -> 19.8 us, B 1 / 4096 / one page per split 15.9 -> 13.2, B 4 / 2000 / T 3 / pps 4 30.3 -> 22.5,
+// B 8 / 4096 / pps 8 29.5 -> 28.7, B 1 / 200 13.2 -> 11.9.
+struct MixChunk {
+    f32x4_t w[2], c[2], s[2];
+};
+// norm weights of dims 8 ch .. + 7
+__device__ __forceinline__ void mix_weights(const float *w, int ch, MixChunk &m) {
+    const auto r = __builtin_amdgcn_make_buffer_rsrc(qs::uniform_ptr(const_cast<float *>(w)), (short)0, HD * 4, 0x00020000);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        m.w[h] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, ch * 32, h * 16, 0));
+}
+// cos / sin of the chunk's dims (halves paired) for row `row` of the tables [rows, rot / 2]; zeros where the chunk
+// is not rotated. Buffer loads: the tables need no more than their 4-byte alignment.
+__device__ __forceinline__ void mix_angles(const AttnArgs &a, int row, int ch, MixChunk &m) {
+    const int half = a.rot / 2, hc = half / 8, bytes = a.B * a.T * half * 4;
+    const auto rc = __builtin_amdgcn_make_buffer_rsrc(qs::uniform_ptr(const_cast<float *>(a.rcos)), (short)0, bytes, 0x00020000);
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(qs::uniform_ptr(const_cast<float *>(a.rsin)), (short)0, bytes, 0x00020000);
+    const int off = ch < 2 * hc ? (row * half + (ch < hc ? ch : ch - hc) * 8) * 4 : 0x7fffffe0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        m.c[h] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rc, off, h * 16, 0));
+        m.s[h] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, off, h * 16, 0));
+    }
+}
 // Mixer prologue of one 8-element chunk (raw bf16 bits, chunk ch of a 256-dim row whose 32 chunks sit in 32
 // consecutive, fully active lanes): y = x * rsqrt(mean(x^2) + eps) * w, then the rotary embedding on the
 // first rot dims with the halves paired as at model.py:135-140 (d < rot/2 with d + rot/2:
 // y_d c - y_{d+h} s and y_{d+h} c + y_d s). fp32 throughout (model.py:86-89, :237-238).
-__device__ __forceinline__ void mixer_chunk(const uint4 raw, int ch, const float *w, const float *cs,
-                                            const float *sn, int rot, float eps, float y[8]) {
+__device__ __forceinline__ void mixer_chunk(const uint4 raw, int ch, const MixChunk &m, int rot, float eps, float y[8]) {
     const uint32_t wd[4] = {raw.x, raw.y, raw.z, raw.w};
     float ss = 0.f;
 #pragma unroll
@@ -80,20 +108,18 @@ __device__ __forceinline__ void mixer_chunk(const uint4 raw, int ch, const float
     ss += qs::dpp<0x128>(ss);
     ss = qs::xor16_sum(ss);  // the 32 lanes of the row
     const float r = rsqrtf(ss * (1.0f / HD) + eps);
-    const float4 w0 = *reinterpret_cast<const float4 *>(w + ch * 8), w1 = *reinterpret_cast<const float4 *>(w + ch * 8 + 4);
-    const float wv[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = y[i] * r * wv[i];
+    for (int i = 0; i < 8; ++i) y[i] = y[i] * r * m.w[i / 4][i % 4];
     if (rot > 0) {
-        const int half = rot / 2, hc = half / 8;  // dims / chunks per half
+        const int hc = rot / 16;  // chunks per half
         float yp[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) yp[i] = __shfl_xor(y[i], hc, 64);
         if (ch < 2 * hc) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const int d = (ch * 8 + i) % half;
-                y[i] = ch < hc ? y[i] * cs[d] - yp[i] * sn[d] : y[i] * cs[d] + yp[i] * sn[d];
+                const float c = m.c[i / 4][i % 4], s = m.s[i / 4][i % 4];
+                y[i] = ch < hc ? y[i] * c - yp[i] * s : y[i] * c + yp[i] * s;
             }
         }
     }
@@ -192,7 +218,6 @@ __device__ __forceinline__ u32x4 new_chunk(const AttnArgs &a, const uint16_t *ro
 // ------------------------------------------------------------------------------ shared by the MFMA kernels
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr int QPAD = HD + 8;   // s_q row pitch (bf16): 16-byte skew between rows
 constexpr int VPAD = HD + 16;  // K / V slice row pitch (bf16): 32-byte skew between rows
 
@@ -360,6 +385,21 @@ __global__ __launch_bounds__(256 * WPP) void attn_rows_kernel(AttnArgs a, int G,
         nk[k] = new_chunk(a, a.k_new, b, g, wv + 4 * WPP * k, lane < 32 ? lane : -1);
         nv[k] = new_chunk(a, a.v_new, b, g, wv + 4 * WPP * k, lane < 32 ? -1 : lane - 32);
     }
+    MixChunk mq[MIX ? QCH : 1], mk[MIX ? NCH : 1];
+    if constexpr (MIX) {
+        mix_weights(a.wq, lane & 31, mq[0]);
+        mix_weights(a.wk, lane & 31, mk[0]);
+#pragma unroll
+        for (int k = 0; k < QCH; ++k) {
+            if (k > 0) mq[k].w[0] = mq[0].w[0], mq[k].w[1] = mq[0].w[1];
+            mix_angles(a, b * T + min((r0 + ((tid + NTH * k) >> 5)) / G, T - 1), lane & 31, mq[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < NCH; ++k) {
+            if (k > 0) mk[k].w[0] = mk[0].w[0], mk[k].w[1] = mk[0].w[1];
+            mix_angles(a, b * T + min(wv + 4 * WPP * k, T - 1), lane & 31, mk[k]);
+        }
+    }
     auto page_at = [&](int pi) {
         const int pg = __builtin_amdgcn_readlane(bt_pre, pi - p0);
         return (pg >= 0 && pg < a.num_blocks) ? pg : -1;
@@ -410,8 +450,7 @@ __global__ __launch_bounds__(256 * WPP) void attn_rows_kernel(AttnArgs a, int G,
         uint4 u = qreg[k];
         if constexpr (MIX) {  // normalised and rotated q (all lanes take part in the row reductions)
             float y[8];
-            const size_t rc = ((size_t)b * T + min((r0 + row) / G, T - 1)) * (a.rot / 2);
-            mixer_chunk(u, ch, a.wq, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
+            mixer_chunk(u, ch, mq[k], a.rot, a.eps, y);
             u = pack8(y);
             *reinterpret_cast<uint4 *>(&s_ql[row][ch * 8]) = pack8_lo(y, u);
         }
@@ -426,8 +465,7 @@ __global__ __launch_bounds__(256 * WPP) void attn_rows_kernel(AttnArgs a, int G,
             uint4 u = make_uint4(x[0], x[1], x[2], x[3]);
             if constexpr (MIX) {  // k rows normalised and rotated; the V lanes take part in the shuffles only
                 float y[8];
-                const size_t rc = ((size_t)b * T + t) * (a.rot / 2);
-                mixer_chunk(u, lane & 31, a.wk, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
+                mixer_chunk(u, lane & 31, mk[k], a.rot, a.eps, y);
                 if (lane < 32) u = pack8(y);
             }
             *reinterpret_cast<uint4 *>(&s_new[t][lane >> 5][(lane & 31) * 8]) = u;
@@ -744,7 +782,9 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
     auto s_kv = reinterpret_cast<uint16_t (*)[16][VPAD]>(s_raw + QB + QLB);
     auto s_o = reinterpret_cast<float (*)[NQR][OPAD]>(s_raw);
     __shared__ float s_ml[NWV][NQR][2];
-    __shared__ __align__(16) uint16_t s_nk[WPP == 1 && !MIX ? 2 : 1][HD];  // WPP = 1: the new K rows, for the score operand
+    // the step's new K / V rows: every one with the mixer (k normalised and rotated), the K rows for the score
+    // operand with WPP = 1
+    __shared__ __align__(16) uint16_t s_nw[MIX || WPP == 1 ? 2 : 1][2][HD];
 
     const int p0 = split * a.pps;
     const int *bt = a.block_table + (size_t)b * a.max_blocks;
@@ -757,15 +797,27 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         const int idx = tid + NTH * k;
         qreg[k] = q_chunk(a, G, b, g, idx >> 5, idx & 31);  // rows past NQR are never staged
     }
-    // The step's new K / V rows (up to TN tokens, which registers allow: two, none with the mixer; more go
-    // through the pool below): token t's chunk lane % 32 of the K row (lanes < 32) or of the V row, requested
-    // before the pages like the query rows
-    constexpr int TN = MIX ? 0 : 2;
-    u32x4 nk[TN > 0 ? TN : 1], nv[TN > 0 ? TN : 1];  // vector types (not uint4): selects stay in registers
+    // The step's new K / V rows (up to TN tokens; more go through the pool below): chunk lane % 32 of the K row
+    // (lanes < 32) or of the V row, requested before the pages like the query rows. Every wave holds all of them
+    // in registers; with the mixer, which leaves none, wave t turns token t's K row and puts both rows in LDS.
+    constexpr int TN = 2, NTK = MIX ? 1 : TN;
+    u32x4 nk[NTK], nv[NTK];  // vector types (not uint4): selects stay in registers
 #pragma unroll
-    for (int t = 0; t < TN; ++t) {
-        nk[t] = new_chunk(a, a.k_new, b, g, t, lane < 32 ? lane : -1);
-        nv[t] = new_chunk(a, a.v_new, b, g, t, lane < 32 ? -1 : lane - 32);
+    for (int t = 0; t < NTK; ++t) {
+        const int tok = MIX ? (w < TN ? w : T) : t;
+        nk[t] = new_chunk(a, a.k_new, b, g, tok, lane < 32 ? lane : -1);
+        nv[t] = new_chunk(a, a.v_new, b, g, tok, lane < 32 ? -1 : lane - 32);
+    }
+    MixChunk mq[MIX ? QCH : 1], mk;
+    if constexpr (MIX) {
+        mix_weights(a.wq, lane & 31, mq[0]);
+        mix_weights(a.wk, lane & 31, mk);
+#pragma unroll
+        for (int k = 0; k < QCH; ++k) {
+            if (k > 0) mq[k].w[0] = mq[0].w[0], mq[k].w[1] = mq[0].w[1];
+            mix_angles(a, b * T + min(((tid + NTH * k) >> 5) / G, T - 1), lane & 31, mq[k]);
+        }
+        mix_angles(a, b * T + min(w, T - 1), lane & 31, mk);
     }
     auto page_at = [&](int pi) {
         const int pg = __builtin_amdgcn_readlane(bt_pre, pi - p0);
@@ -820,7 +872,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
     // page loop: an atomic here, inside a branch, would make the compiler wait for every load at the next use
     const bool bad_pages = __any(lane < p1 - p0 && (bt_pre < 0 || bt_pre >= a.num_blocks));
 
-    // Fused append. Up to TN tokens: the new rows stay in registers (nk, nv), the page loop writes them over
+    // Fused append. Up to TN tokens: the new rows stay in registers (or LDS), the page loop writes them over
     // the staged rows of this wave's slices, and they go to the pool after the loop, so no store is in flight
     // while pages load (the compiler would then wait for every load at each use), nothing waits for the
     // stores, and no page is read twice. More tokens: each wave writes the new rows of its own slices to the
@@ -836,10 +888,10 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
             const int pos = base + t, pi = pos / BLK;
             const size_t src = (((size_t)b * T + t) * a.NKV + g) * HD + ch * 8;
             uint4 u = *reinterpret_cast<const uint4 *>((kv ? a.v_new : a.k_new) + src);
-            if (a.wk) {
+            if constexpr (MIX) {
                 float y[8];
-                const size_t rc = ((size_t)b * T + t) * (a.rot / 2);
-                mixer_chunk(u, ch, a.wk, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
+                mix_angles(a, b * T + t, ch, mk);
+                mixer_chunk(u, ch, mk, a.rot, a.eps, y);
                 if (!kv) u = pack8(y);
             }
             if (!owned(pos)) continue;
@@ -863,18 +915,33 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         uint4 u = qreg[k];
         if constexpr (MIX) {
             float y[8];
-            const size_t rc = ((size_t)b * T + min(qr / G, T - 1)) * (a.rot / 2);
-            mixer_chunk(u, ch, a.wq, a.rcos + rc, a.rsin + rc, a.rot, a.eps, y);
+            mixer_chunk(u, ch, mq[k], a.rot, a.eps, y);
             u = pack8(y);
             *reinterpret_cast<uint4 *>(&s_ql[qr][ch * 8]) = pack8_lo(y, u);
         }
         *reinterpret_cast<uint4 *>(&s_q[qr][ch * 8]) = u;
     }
-    if constexpr (WPP == 1 && TN > 0)
+    if constexpr (MIX) {
+        if (fresh && w < T) {
+            uint4 u = make_uint4(nk[0][0], nk[0][1], nk[0][2], nk[0][3]);
+            float y[8];
+            mixer_chunk(u, lane & 31, mk, a.rot, a.eps, y);
+            if (lane < 32) u = pack8(y);
+            *reinterpret_cast<u32x4 *>(&s_nw[w][lane >> 5][(lane & 31) * 8]) = lane < 32 ? u32x4{u.x, u.y, u.z, u.w} : nv[0];
+        }
+    } else if constexpr (WPP == 1) {
         if (w == 0 && lane < 32)
 #pragma unroll
-            for (int t = 0; t < TN; ++t) *reinterpret_cast<u32x4 *>(&s_nk[t][lane * 8]) = nk[t];
+            for (int t = 0; t < TN; ++t) *reinterpret_cast<u32x4 *>(&s_nw[t][0][lane * 8]) = nk[t];
+    }
     __syncthreads();
+    // token t's new K row (kv 0, lanes < 32) or V row (kv 1, lanes >= 32), this lane's chunk
+    auto new_row = [&](int t, int kv) -> u32x4 {
+        if constexpr (MIX)
+            return *reinterpret_cast<const u32x4 *>(&s_nw[t][kv][(lane & 31) * 8]);
+        else
+            return kv ? nv[t] : nk[t];
+    };
     // Q^T fragments, held in registers for the split
     bf16x8_t qb[QT][8], qlo[QT][MIX ? 8 : 1];
 #pragma unroll
@@ -906,13 +973,13 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         const int r0w = pi * BLK + 16 * sl;
         f32x4_t sacc[QT];
         if constexpr (WPP == 1) {  // K already in the operand's layout; the new rows patched from LDS
-            if (TN > 0 && fresh && base + T > r0w && base < r0w + 16) {  // new rows in this slice (uniform)
+            if (fresh && base + T > r0w && base < r0w + 16) {  // new rows in this slice (uniform)
                 const int t = r0w + l16 - base;
                 const bool kp = t >= 0 && t < T;
                 u32x4 x[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
-                    x[j] = *reinterpret_cast<const u32x4 *>(&s_nk[min(max(t, 0), TN > 0 ? TN - 1 : 0)][32 * j + 8 * lg]);
+                    x[j] = *reinterpret_cast<const u32x4 *>(&s_nw[min(max(t, 0), TN - 1)][0][32 * j + 8 * lg]);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     KA[j].x = kp ? x[j][0] : KA[j].x;
@@ -943,7 +1010,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
 #pragma unroll
             for (int t = 0; t < TN; ++t)
                 if (t < T && base + t >= r0w && base + t < r0w + 16 && lane < 32)
-                    *reinterpret_cast<u32x4 *>(&s_kv[w][base + t - r0w][lane * 8]) = nk[t];
+                    *reinterpret_cast<u32x4 *>(&s_kv[w][base + t - r0w][lane * 8]) = new_row(t, 0);
         load_rows(a.k_cache, pgn, KA);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         // K fragments (row l16, dims 32 j + 8 lg .. + 7), each used by every query tile
@@ -979,7 +1046,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
 #pragma unroll
             for (int t = 0; t < TN; ++t)
                 if (t < T && base + t >= r0w && base + t < r0w + 16 && lane >= 32)
-                    *reinterpret_cast<u32x4 *>(&s_kv[w][base + t - r0w][(lane - 32) * 8]) = nv[t];
+                    *reinterpret_cast<u32x4 *>(&s_kv[w][base + t - r0w][(lane - 32) * 8]) = new_row(t, 1);
         load_rows(a.v_cache, pgn, VA);
         i16x4_t pb[QT];
 #pragma unroll
@@ -1030,7 +1097,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
             const int pg = page_at(pos / BLK);
             if (pg < 0) continue;  // reported with the split's pages
             const size_t dst = (((size_t)pg * a.NKV + g) * BLK + (pos % BLK)) * HD + (lane & 31) * 8;
-            *reinterpret_cast<u32x4 *>((lane < 32 ? a.k_cache : a.v_cache) + dst) = lane < 32 ? nk[t] : nv[t];
+            *reinterpret_cast<u32x4 *>((lane < 32 ? a.k_cache : a.v_cache) + dst) = lane < 32 ? new_row(t, 0) : new_row(t, 1);
         }
     // the waves' (max, sum) per query row; the barrier also frees the q and K / V bytes for the O rows
     if (lg == 0)
