@@ -311,7 +311,7 @@ int qs_mx_gemv(const uint16_t *h, const uint8_t *w, float *y, void *workspace, i
  * (9: MXINT8, the reference's 8-bit precision; 8: MXFP8);
  * x, x_out [B, H] fp32 (may alias), gamma [H] fp32 or null when the norm weight is already folded into the
  * rows of gate and up (the reference's weights.py:107-112 does so); H % 128 == 0, I % 64 == 0. Two launches for one row
- * with H <= 5120 (the gate | up workgroups normalise the row themselves), three otherwise. The workspace
+ * with H <= 6144 (the gate | up workgroups normalise the row themselves), three otherwise. The workspace
  * (qs_mlp_decode_workspace_bytes, zeroed once) holds arrival counters, h, z and the K-split partials.
  * Replaces the streamers' MLP phase and its residual (kernels/streamer_compute.cpp:452-464,
  * mlp_hub.cpp:309-364 all-reduce on one device; torch pattern tests/bench_resident_mlp.py:98-105). */
