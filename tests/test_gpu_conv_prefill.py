@@ -68,6 +68,17 @@ def test_conv_prefill_fresh_in_place_and_split(dev):
     assert torch.equal(whole, xg[-3:].t())
 
 
+def test_conv_prefill_pieces_equal_the_whole(dev):
+    """3073 tokens (8 per thread) equal, bit for bit, their pieces of 3071 and 2 (4 per thread)."""
+    xp, cs, taps = prompt(3073, seed=6)
+    xg, tg, csg = xp.to(dev)[:, :C], taps.to(dev), cs.to(dev)
+    q, k, v, whole = ops.causal_conv1d_prefill(xg, tg, csg)
+    a = ops.causal_conv1d_prefill(xg[:3071], tg, csg)
+    b = ops.causal_conv1d_prefill(xg[3071:], tg, a[3])
+    assert torch.equal(torch.cat([qkv_cat(*a[:3]), qkv_cat(*b[:3])]), qkv_cat(q, k, v))
+    assert torch.equal(b[3], whole)
+
+
 def test_conv_prefill_8192_tokens(dev):
     """The prompt length of the prefill workload: 8192 tokens of the 10240 q | k | v channels."""
     T = 8192

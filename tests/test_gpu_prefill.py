@@ -34,6 +34,18 @@ def test_prefill_matches_recurrence(dev, T):
     assert_bf16_output(o, O.bf16(o_ref.float()))
 
 
+@pytest.mark.parametrize("T,cut", [(1345, 1344), (1600, 320)])
+def test_prefill_pieces_equal_the_whole(dev, T, cut):
+    """A prompt whose prep takes a key head's value heads in turn (more than 1024 chunks x value heads) equals, bit for
+    bit, its pieces cut at a chunk, whose preps run a workgroup per value head (1344 tokens are the most)."""
+    d = {k: v.to(dev) for k, v in W.prefill(T, "cpu", seed=9).items()}
+    o, S = run(dev, d, T)
+    rows = ("q", "k", "v", "g", "beta")
+    o0, S0 = run(dev, {n: d[n][:cut] if n in rows else d[n] for n in d}, cut)
+    o1, S1 = run(dev, {n: d[n][cut:].contiguous() if n in rows else S0 for n in d}, T - cut)
+    assert torch.equal(torch.cat([o0, o1]), o) and torch.equal(S1, S)
+
+
 @pytest.mark.parametrize("nk,nv", [(4, 4), (4, 8), (2, 8)])
 def test_prefill_head_ratios(dev, nk, nv):
     """1, 2 and 4 value heads per key head (the prep forms K K^T and Q K^T once per key head and takes the

@@ -21,7 +21,6 @@ namespace {
 
 constexpr int KC = 4;  // conv taps
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-constexpr int R = 8;  // tokens per thread (4, 16, 24, 32, or 4 blocks of 16 in sequence measured slower)
 
 struct ConvPrefillArgs {
     const uint16_t *x;       // [T, ldx], conv channels in columns [0, 2 CQ + CV)
@@ -37,6 +36,7 @@ __device__ __forceinline__ uint32_t half_of(const uint4 &r, int c) {
     return (c & 1) ? w >> 16 : w & 0xffffu;
 }
 
+template <int R>  // tokens per thread
 __global__ __launch_bounds__(256) void conv_prefill_kernel(ConvPrefillArgs a) {
     // workgroup = 64 channel groups (lanes) x 4 consecutive token blocks (waves): the 3 rows before the
     // block of waves 1-3 are rows the wave before loads, so only wave 0's come from another workgroup;
@@ -160,9 +160,18 @@ extern "C" int qs_conv1d_prefill(const uint16_t *x, int ldx, const uint16_t *con
                "qs_conv1d_prefill: every buffer must be 16-byte aligned");
     ConvPrefillArgs a{};
     a.x = x, a.st_in = conv_state_in, a.taps = taps, a.q = q, a.k = k, a.v = v, a.st_out = conv_state_out;
-    a.ldx = ldx, a.T = T, a.CQ = CQ, a.CV = CV, a.ngroups = C / 8, a.ntb = T > 0 ? (T + R - 1) / R : 1;
+    a.ldx = ldx, a.T = T, a.CQ = CQ, a.CV = CV, a.ngroups = C / 8;
+    // tokens per thread: 8, or 4 for prompts too short to fill the chip with blocks of 8 (the carry's rows reach 3
+    // tokens into the prompt and only the first block may read them, so not fewer). 10240 channels, 8 -> 4: 16 tokens
+    // 8.8 -> 6.0 us, 200 9.2 -> 6.4, 1000 13.5 -> 13.0, 3000 30.0 -> 28.1, 4096 37.6 -> 37.5, 8192 67.2 -> 68.8
+    // (16, 24, 32 and 4 blocks of 16 in sequence measured slower than 8 there)
+    const int R = T <= 3072 ? 4 : 8;
+    a.ntb = T > 0 ? (T + R - 1) / R : 1;
     const long wgs = (long)((a.ngroups + 63) / 64) * ((a.ntb + 3) / 4);
     QS_REQUIRE(wgs < (1L << 31), "qs_conv1d_prefill: T = %d tokens are too many for one launch", T);
-    conv_prefill_kernel<<<(unsigned)wgs, 256, 0, QS_STREAM(stream)>>>(a);
+    if (R == 4)
+        conv_prefill_kernel<4><<<(unsigned)wgs, 256, 0, QS_STREAM(stream)>>>(a);
+    else
+        conv_prefill_kernel<8><<<(unsigned)wgs, 256, 0, QS_STREAM(stream)>>>(a);
     return qs::launch_status("qs_conv1d_prefill");
 }

@@ -11,7 +11,8 @@
 //   S  = gamma_C S0 + K^T diag(r_k gamma_C / gamma) d
 // (the chunked gated delta rule of Yang et al., "Gated Delta Networks", as FLA's chunk_gated_delta_rule
 // computes it). Two kernels:
-//   chunk_prep  one workgroup per (chunk, key head), fully parallel: the row norms, K K^T and Q K^T on MFMA
+//   chunk_prep  one workgroup per (chunk, key head), or per value head for short prompts, fully parallel: the row
+//               norms, K K^T and Q K^T on MFMA
 //               from the raw bf16 rows (exact products, fp32 sums) once for the key head, then for each of its
 //               value heads in turn A and P from the accumulators, the triangular inverse Tm (16 x 16
 //               diagonal blocks by forward substitution, then the 32 x 32 and 64 x 64 levels of the block
@@ -88,6 +89,7 @@ struct PrefillArgs {
     uint16_t *KQ;               // workspace [nch, NK, 2, 64 x 128] bf16: the chunk's k and q rows, fragment order
     float *sc;                  // workspace [nch, NV, 5, 64]: beta | beta gamma r_k | gamma r_q | r_k gamma_C/gamma | gamma_C
     int T, NK, NV, nch;
+    int prep_heads;             // value heads per prep workgroup: a key head's, or one
     float scale, eps;
 };
 
@@ -108,11 +110,12 @@ __device__ __forceinline__ void put16(float *D, int ds, f32x4 c, int lane) {
 }
 
 __global__ __launch_bounds__(256, 4) void chunk_prep_kernel(PrefillArgs a) {
-    // one workgroup per (chunk, key head): the k, q rows, their norms, K K^T and Q K^T are shared by the rep
-    // value heads of the key head, which then take turns for A, P and Tm
-    const int lid = qs::xcd_logical(blockIdx.x, a.nch * a.NK);
-    const int c = lid / a.NK, kh = lid % a.NK;
-    const int rep = a.NV / a.NK;
+    // one workgroup per (chunk, key head, group of `heads` of its value heads): the k, q rows, their norms, K K^T
+    // and Q K^T are shared by the group, whose heads then take turns for A, P and Tm
+    const int rep = a.NV / a.NK, heads = a.prep_heads, groups = rep / heads;
+    const int lid = qs::xcd_logical(blockIdx.x, a.nch * a.NK * groups);
+    const int c = lid / (a.NK * groups), kh = lid / groups % a.NK;
+    const int h0 = kh * rep + lid % groups * heads;
     const int t0 = c * CH, nval = min(CH, a.T - t0);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int fr = lane & 15, g = lane >> 4;
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(256, 4) void chunk_prep_kernel(PrefillArgs a) {
     static_assert(2 * CH * DK * 2 <= 2 * CH * FP * 4, "the K / Q images must fit in the A / Tm space");
 
     // 1. the chunk's raw k, q rows of key head kh into swizzled LDS images (zeros past the sequence); the
-    //    gates of value head kh rep + w (waves w < rep: lane = token, g = 0 and beta = 0 past the sequence)
+    //    gates of value head h0 + w (waves w < heads: lane = token, g = 0 and beta = 0 past the sequence)
     {
         const size_t krow = (size_t)a.NK * DK * 2;  // bytes per token
         const auto rk = rsrc(a.k + (size_t)t0 * a.NK * DK, (int)(nval * krow));
@@ -143,15 +146,15 @@ __global__ __launch_bounds__(256, 4) void chunk_prep_kernel(PrefillArgs a) {
         }
     }
     float gi = 0.f, bi = 0.f;
-    if (w < rep && lane < nval) {
-        gi = a.g[(size_t)(t0 + lane) * a.NV + kh * rep + w];
-        bi = a.beta[(size_t)(t0 + lane) * a.NV + kh * rep + w];
+    if (w < heads && lane < nval) {
+        gi = a.g[(size_t)(t0 + lane) * a.NV + h0 + w];
+        bi = a.beta[(size_t)(t0 + lane) * a.NV + h0 + w];
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
     // 2. row norms (4 lanes per row; the sum runs over the row's chunks in stored order); cumulative log
-    //    decay of each value head (waves w < rep, inclusive scan over the 64 tokens)
+    //    decay of each value head (waves w < heads, inclusive scan over the 64 tokens)
     {
         const int r = tid >> 2, part = tid & 3;
         float kk = 0.f, qq = 0.f;
@@ -177,7 +180,7 @@ __global__ __launch_bounds__(256, 4) void chunk_prep_kernel(PrefillArgs a) {
             s_rq[r] = rsqrtf(qq + a.eps) * a.scale;
         }
     }
-    if (w < rep) {
+    if (w < heads) {
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const float up = __shfl_up(gi, d, 64);
@@ -187,8 +190,8 @@ __global__ __launch_bounds__(256, 4) void chunk_prep_kernel(PrefillArgs a) {
         s_b[w][lane] = bi;
     }
 
-    // 2b. the chunk's k and q rows in fragment order for the walk
-    {
+    // 2b. the chunk's k and q rows in fragment order for the walk, once per key head
+    if (h0 == kh * rep) {
         uint16_t *dst = a.KQ + ((size_t)c * a.NK + kh) * 2 * CH * DK;
 #pragma unroll
         for (int m = 0; m < 8; ++m) {
@@ -229,8 +232,8 @@ __global__ __launch_bounds__(256, 4) void chunk_prep_kernel(PrefillArgs a) {
     __syncthreads();  // every read of the K / Q images is done before A overwrites them
 
 #pragma unroll 1
-    for (int hv = 0; hv < rep; ++hv) {
-        const int h = kh * rep + hv;
+    for (int hv = 0; hv < heads; ++hv) {
+        const int h = h0 + hv;
         const float *sG = s_G[hv], *sB = s_b[hv];
         // 4. A (strictly lower) and P (lower with the diagonal, bf16 hi and lo planes) from the accumulators into
         //    LDS; P is staged in the space Tm takes later and leaves in 16-byte rows
@@ -747,7 +750,13 @@ extern "C" int qs_gdn_chunk_prefill(const uint16_t *q, const uint16_t *k, const 
     a.KQ = reinterpret_cast<uint16_t *>(ws + L.kq);
     a.T = T, a.NK = NK, a.NV = NV, a.nch = (T + CH - 1) / CH, a.scale = scale, a.eps = eps;
     hipStream_t st = QS_STREAM(stream);
-    chunk_prep_kernel<<<a.nch * NK, 256, 0, st>>>(a);
+    // A value head's turn is a ~6 us chain (A, P, the block inverse with its barriers) after ~4 us for the rows and
+    // their products: with few chunks each head gets a workgroup of its own, as long as all of them are resident at
+    // once (4 per CU; above that the repeated rows cost more than the shorter chain saves). 16 key / 48 value heads,
+    // the rule alone, one workgroup per key head -> per value head: 16 tokens 27.2 -> 17.9 us, 200 36.2 -> 26.7,
+    // 1000 61.7 -> 54.4, 1344 71.7 -> 64.9, 2048 92.6 -> 92.6, 4096 164.6 -> 171.9.
+    a.prep_heads = (long)a.nch * NV <= 4 * 256 ? 1 : NV / NK;
+    chunk_prep_kernel<<<a.nch * NV / a.prep_heads, 256, 0, st>>>(a);
     if (int e = qs::launch_status("qs_gdn_chunk_prefill (prep)")) return e;
     chunk_walk_kernel<<<NV * NSLAB, WALK_THREADS, 0, st>>>(a);
     return qs::launch_status("qs_gdn_chunk_prefill (walk)");
