@@ -94,7 +94,7 @@ def lib():
 
 def call(name, *args):
     """Call ``name``; raise ValueError (invalid argument) or QSError (HIP error) on a non-zero status."""
-    rc = getattr(lib(), name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != 0:
         msg = lib().qs_last_error().decode()
         if rc == -1:

@@ -5,8 +5,6 @@ shapes, dtypes, devices and contiguity (ValueError on a mismatch, like the refer
 enqueues HIP kernels on the current torch stream. Tensors are caller-owned; state arguments are updated in
 place as in the reference. Nothing here computes on the CPU.
 """
-import ctypes
-
 import torch
 
 from ._lib import call, lib
@@ -18,15 +16,24 @@ BLOCK = 64  # vLLM block size, tt-model.yaml:41
 EPS = 1e-6  # model.py:264-267
 
 
+# A directly called op of a short prompt or a single layer is bound by the host: pointers and streams go to the
+# library as plain integers (its argument types convert them), and an argument that is as it should be is accepted
+# on one chain of attribute reads.
+
+
 def _p(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+    return None if t is None else t.data_ptr()
 
 
 def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    """The current stream's handle on ``dev`` (a tensor's device), without a Stream object around it."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def _chk(t, name, dtype, shape=None, dev=None):
+    if (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda and t.is_contiguous()
+            and (shape is None or t.shape == shape) and (dev is None or t.device == dev)):  # fmt: skip
+        return t
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a tensor")
     if not t.is_cuda:
@@ -52,8 +59,9 @@ def workspace(kind, nbytes, device):
 
     The kernels leave their counters zeroed again, so the buffer is reused by every later call on the
     same stream. It must exist before a HIP graph capture starts (warm the op up once first)."""
-    device = torch.device(device)
-    key = (kind, device, torch.cuda.current_stream(device).cuda_stream)
+    if not isinstance(device, torch.device) or device.index is None:
+        device = torch.empty(0, device=device).device
+    key = (kind, device, _stream(device))
     ws = _WS.get(key)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
@@ -425,7 +433,7 @@ def paged_fill_cache(cache, x, page_table, batch_idx=0):
     _chk(x, "x", torch.bfloat16, (1, nkv, T, hd), dev)
     _chk(page_table, "page_table", torch.int32, None, dev)
     row = page_table[batch_idx]
-    call("qs_paged_kv_fill", _p(x), None, _p(cache), None, ctypes.c_void_p(row.data_ptr()), T, 0, nkv, hd, block,
+    call("qs_paged_kv_fill", _p(x), None, _p(cache), None, _p(row), T, 0, nkv, hd, block,
          row.shape[0], nb, _stream(dev))  # fmt: skip
 
 
@@ -544,11 +552,12 @@ def chunk_gated_delta_rule(q, k, v, g, beta, *, scale=None, initial_state=None, 
     dev = q.device
     T = q.shape[0]
     nv = g.shape[1]
-    q3 = q.reshape(T, -1, DK)
+    heads = lambda t, d: t if t.dim() == 3 and t.shape[2] == d else t.reshape(T, -1, d)  # noqa: E731
+    q3 = heads(q, DK)
     nk = q3.shape[1]
     _chk(q3, "q", torch.bfloat16, (T, nk, DK), dev)
-    _chk(k.reshape(T, -1, DK), "k", torch.bfloat16, (T, nk, DK), dev)
-    _chk(v.reshape(T, -1, DV), "v", torch.bfloat16, (T, nv, DV), dev)
+    _chk(heads(k, DK), "k", torch.bfloat16, (T, nk, DK), dev)
+    _chk(heads(v, DV), "v", torch.bfloat16, (T, nv, DV), dev)
     _chk(g, "g", torch.float32, (T, nv), dev)
     _chk(beta, "beta", torch.float32, (T, nv), dev)
     if initial_state is None:
