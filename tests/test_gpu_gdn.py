@@ -215,7 +215,7 @@ def test_gdn_decode_fused_gated_norm(dev, B):
     274-275, kernels/gdn_head_compute.cpp:320-346): o = bf16(rmsnorm(o) norm_w silu(z)) per value head, from
     the fp32 o as the reference normalises it, against the oracle's gdn_gated_norm(gdn_step(...)) at rtol 2e-2
     (the oracle fed the kernel's own conv output); z is read as a strided slice of a wider projection row.
-    Batch 1 and 3 (a head's 4 slabs on 4 waves each, 16 waves per workgroup) and 8 (one wave per slab). The
+    Batch 1 and 3 (a head's 4 slabs on 2 waves each, 8 waves per workgroup) and 8 (one wave per slab). The
     state and conv state are bit-identical to the plain fused launch, whose o rounded to bf16 and then put
     through the separate epilogue lands within two bf16 ulps of the fused result."""
     d = inputs(B, seed=40 + B)

@@ -193,7 +193,7 @@ __device__ __forceinline__ const float *sp_of_t(const GdnArgs &a, size_t user, i
 // w * RW + rg + RG i (i < RPL), columns 4 cg .. 4 cg + 3. NW = 1 at large batch (each wave streams a
 // 16 KB slab); NW = 4 when one wave per slab would leave the chip underfilled (small batch), which also
 // spreads the conv prologue over three waves and cuts the serial work per token by 4, for one LDS
-// exchange per token.
+// exchange per token; NW = 2 with the epilogue, where a workgroup holds a whole head (8 waves instead of 16).
 // Per token both column reductions are taken from the state before the update, in one pass:
 //     p_v = sum_k k_k S_kv,  r_v = sum_k q_k S_kv,  delta_v = beta (v_v - e^g p_v)
 //     S'_kv = e^g S_kv + k_k delta_v,  o_v = q^T S'_v = e^g r_v + (q . k) delta_v
@@ -221,13 +221,17 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     constexpr int RPL = RW / RG;   // rows per lane
     static_assert(RPL >= 1 && RW % RG == 0 && (VERIFY || TM == 1), "slab shape");
     static_assert(!NORM || (!VERIFY && WPG == NSLAB && CG <= 16), "the epilogue needs whole heads per workgroup");
-    // conv roles by wave of the workgroup: q channels on wave 0, k on wave 1 (when there is one), the slab's v
-    // channels on wave 2 (NW = 4) or on every wave for its own slab (NW = 1)
-    constexpr int WK = (NW >= 4 || WPG >= 2) ? 1 : 0;
+    // conv roles by wave of the workgroup: q channels on wave 0, k on wave 1 (when there is one; NW = 2: wave 2), the
+    // slab's v channels on wave 2 (NW = 4), each slab's wave 1 (NW = 2) or every wave for its own slab (NW = 1)
+    constexpr int WK = NW == 2 && WPG >= 2 ? 2 : (NW >= 4 || WPG >= 2) ? 1 : 0;
     constexpr int WV = NW >= 4 ? 2 : NW - 1;
     // the wave that writes o (and forms each token's q . k for it): the slab's last wave, which reaches each
     // token's exchange first; wave 0, which also runs the q conv, was the last with o on its path as well
-    constexpr int WO = NW - 1;
+    // (NORM: the slab's first wave, 293 against 282 us for the 48 layers below; the last also runs the v conv)
+    constexpr int WO = NORM ? 0 : NW - 1;
+    // The column sums of the forms with several waves per slab are taken over 32-row blocks, 4 to a slab, and added in
+    // row order, so that 2 and 4 waves per slab give the same bits
+    constexpr int NB = NW > 1 ? 4 / NW : 1;  // row blocks per wave
     // The one-wave-per-slab form: the load addresses' kernel arguments, requested with the first batch of
     // argument loads (the compiler would otherwise request them after the index arithmetic below, a second
     // round trip before the first load; the other forms already request them in one batch, and the fence
@@ -273,7 +277,7 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     __shared__ __align__(16) float s_kn[TM][DK];
     __shared__ __align__(16) float s_v_[WPG][TM][SLAB];
     auto &s_v = s_v_[gw];
-    __shared__ __align__(16) f32x4 s_red_[NW > 1 ? 2 : 1][WPG][NW][2][CG];  // per token parity: wave column sums
+    __shared__ __align__(16) f32x4 s_red_[NW > 1 ? 2 : 1][WPG][NW * NB][2][CG];  // per token parity: row blocks' column sums
     __shared__ float s_nrm[2][WPG];  // NORM, per token parity: the slabs' sums of o^2
     __shared__ float s_qk_[WPG][TM];  // q . k of every token of the unit
 
@@ -332,6 +336,19 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
         if (isk) ink = conv_load<TM>(a, conv_b, b, ck, T);
         if (isv) inv = conv_load<TM>(a, conv_b, b, cv, T);
     }
+    // NORM: the epilogue's z and norm_w of the lane's 4 columns. Requested and read before any store leaves (read
+    // after the last token they waited for the state stores too: 271 against 281 us for the 48 layers below), ahead of
+    // the state with several waves per slab (250 us), behind it with one (batch 8, 12 layers: 130.0 us behind, 137.6
+    // ahead, 136.5 read after the token)
+    uint2 z4 = make_uint2(0, 0);
+    float4 w4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load_z = [&]() {
+        if (NORM && w == WO && lane < CG) {
+            z4 = *reinterpret_cast<const uint2 *>(a.z + (size_t)b * a.ldz + h * DV + s * SLAB + cg * 4);
+            w4 = *reinterpret_cast<const float4 *>(a.norm_w + s * SLAB + cg * 4);
+        }
+    };
+    if constexpr (NW > 1) load_z();
     const size_t head = (size_t)(b * a.NV + h) * DK * DV;
     const float *sp = sp_of_t<SLAB>(a, user_in, h, s, cg, w * RW + rg);
     f32x4 S[RPL];  // streamed once per step: nontemporal loads and stores keep it from thrashing L2 / MALL
@@ -345,13 +362,7 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
         gdec[t] = a.g[gi];
         gbeta[t] = a.beta[gi];
     }
-    // NORM: the epilogue's z and norm_w of the lane's 4 columns, requested now (used after the last token)
-    uint2 z4 = make_uint2(0, 0);
-    float4 w4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (NORM && w == WO && lane < CG) {
-        z4 = *reinterpret_cast<const uint2 *>(a.z + (size_t)b * a.ldz + h * DV + s * SLAB + cg * 4);
-        w4 = *reinterpret_cast<const float4 *>(a.norm_w + s * SLAB + cg * 4);
-    }
+    if constexpr (NW == 1) load_z();
     // An idle slot keeps its state, conv history and output as they are. The check comes once the loads are
     // requested (they only read, within the buffers), so the length's round trip overlaps them, and waits for
     // the length alone (requested first); nothing has been stored or counted yet. The workgroup's units belong
@@ -423,6 +434,11 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
         const float2 k2 = *reinterpret_cast<const float2 *>(&s_kn[t][2 * lane]);
         s_qk_[gw][t] = qs::wave_sum_dpp(q2.x * k2.x + q2.y * k2.y);
     }
+    float sz[4] = {0.f, 0.f, 0.f, 0.f};  // NORM: silu(z)
+    if (NORM && w == WO) {
+        sz[0] = qs::silu(qs::bf_lo(z4.x)), sz[1] = qs::silu(qs::bf_hi(z4.x));
+        sz[2] = qs::silu(qs::bf_lo(z4.y)), sz[3] = qs::silu(qs::bf_hi(z4.y));
+    }
     // 3. Delta rule, token by token, on the rows held in registers.
     for (int t = 0; t < T; ++t) {
         const int gi = ((b * T) + t) * a.NV + h;
@@ -444,41 +460,50 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
             }
         }
         const float4 v4 = *reinterpret_cast<const float4 *>(&s_v[t][cg * 4]);
-        float p[4] = {0.f, 0.f, 0.f, 0.f}, r[4] = {0.f, 0.f, 0.f, 0.f};
+        float p[4], r[4];
+        auto block_sums = [&](int i0) {  // over the lane's rows i0 .. i0 + RPL / NB - 1
 #pragma unroll
-        for (int i = 0; i < RPL; ++i) {
-            p[0] = fmaf(kn[i], S[i].x, p[0]);
-            p[1] = fmaf(kn[i], S[i].y, p[1]);
-            p[2] = fmaf(kn[i], S[i].z, p[2]);
-            p[3] = fmaf(kn[i], S[i].w, p[3]);
-            r[0] = fmaf(qn[i], S[i].x, r[0]);
-            r[1] = fmaf(qn[i], S[i].y, r[1]);
-            r[2] = fmaf(qn[i], S[i].z, r[2]);
-            r[3] = fmaf(qn[i], S[i].w, r[3]);
-        }
+            for (int j = 0; j < 4; ++j) p[j] = 0.f, r[j] = 0.f;
+#pragma unroll
+            for (int i = i0; i < i0 + RPL / NB; ++i) {
+                p[0] = fmaf(kn[i], S[i].x, p[0]);
+                p[1] = fmaf(kn[i], S[i].y, p[1]);
+                p[2] = fmaf(kn[i], S[i].z, p[2]);
+                p[3] = fmaf(kn[i], S[i].w, p[3]);
+                r[0] = fmaf(qn[i], S[i].x, r[0]);
+                r[1] = fmaf(qn[i], S[i].y, r[1]);
+                r[2] = fmaf(qn[i], S[i].z, r[2]);
+                r[3] = fmaf(qn[i], S[i].w, r[3]);
+            }
+        };
         if constexpr (NW == 1) {
+            block_sums(0);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 p[j] = sum_row_groups<CG>(p[j]);
                 r[j] = sum_row_groups<CG>(r[j]);
             }
         } else {
-            // the wave's column sums, one column component per lane (scatter_sums8), then the waves' sums
-            // added in wave order by every wave (bit-identical everywhere); two buffers by token parity, so one
+            // the row blocks' column sums, one column component per lane (scatter_sums8), then all of the slab's
+            // added in row order by every wave (bit-identical everywhere); two buffers by token parity, so one
             // barrier per token suffices
             static_assert(NW == 1 || CG == 8, "the reduce-scatter takes 8 column groups");
-            float ps, rs;
-            scatter_sums8(p, r, ps, rs);
             auto &red = s_red_[t & 1][gw];
-            if (((lane >> 3) & 1) == 0) {
-                const int c = ((lane >> 5) & 1) * 2 + ((lane >> 4) & 1);
-                reinterpret_cast<float *>(&red[w][0][cg])[c] = ps;
-                reinterpret_cast<float *>(&red[w][1][cg])[c] = rs;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                float ps, rs;
+                block_sums(nb * (RPL / NB));
+                scatter_sums8(p, r, ps, rs);
+                if (((lane >> 3) & 1) == 0) {
+                    const int c = ((lane >> 5) & 1) * 2 + ((lane >> 4) & 1);
+                    reinterpret_cast<float *>(&red[w * NB + nb][0][cg])[c] = ps;
+                    reinterpret_cast<float *>(&red[w * NB + nb][1][cg])[c] = rs;
+                }
             }
             __syncthreads();
             f32x4 P = red[0][0][cg], R = red[0][1][cg];
 #pragma unroll
-            for (int ww = 1; ww < NW; ++ww) {
+            for (int ww = 1; ww < NW * NB; ++ww) {
                 P += red[ww][0][cg];
                 R += red[ww][1][cg];
             }
@@ -537,10 +562,10 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
                 for (int u = 1; u < WPG; ++u) tot += s_nrm[t & 1][u];
                 const float rn = rsqrtf(tot * (1.0f / DV) + a.eps);
                 const int d0 = s * SLAB + cg * 4;
-                const float y0 = po[0] * rn * w4.x * qs::silu(qs::bf_lo(z4.x));
-                const float y1 = po[1] * rn * w4.y * qs::silu(qs::bf_hi(z4.x));
-                const float y2 = po[2] * rn * w4.z * qs::silu(qs::bf_lo(z4.y));
-                const float y3 = po[3] * rn * w4.w * qs::silu(qs::bf_hi(z4.y));
+                const float y0 = po[0] * rn * w4.x * sz[0];
+                const float y1 = po[1] * rn * w4.y * sz[1];
+                const float y2 = po[2] * rn * w4.z * sz[2];
+                const float y3 = po[3] * rn * w4.w * sz[3];
                 *reinterpret_cast<uint2 *>(a.o + (size_t)gi * DV + d0) =
                     make_uint2(qs::cvt_pk_bf16(y0, y1), qs::cvt_pk_bf16(y2, y3));
             }
@@ -691,12 +716,13 @@ void launch_gdn_tm(const GdnArgs &a, hipStream_t st) {
     const int per_key_head = (a.NV / a.NK) * (DV / 32);  // consecutive slab units sharing one key head
     if constexpr (!VERIFY) {
         // with the gated RMSNorm epilogue a workgroup holds one value head: its 4 slabs on one wave each at
-        // large batch, on 4 waves each (16 waves) below
+        // large batch, on 2 waves each below (batch 1, 48 layers: 250 us, with 4 waves each 293; batch 8, where 2
+        // waves each take 148 us for 12 layers, 137 with one)
         if (a.z) {
             if (units >= 1024)
                 gdn_kernel<CONV, VERIFY, TM, 32, 1, 4, true><<<units / 4, 256, 0, st>>>(a);
             else
-                gdn_kernel<CONV, VERIFY, TM, 32, 4, 4, true><<<units / 4, 1024, 0, st>>>(a);
+                gdn_kernel<CONV, VERIFY, TM, 32, 2, 4, true><<<units / 4, 512, 0, st>>>(a);
             return;
         }
     }
