@@ -219,7 +219,9 @@ int qs_paged_kv_gather(const uint16_t *k_cache, const uint16_t *v_cache, const i
  *   When k_new/v_new [B, T, NKV, HD] are non-null the T new rows are also appended (a5 fused): the
  *   workgroup owning a new row's page writes it first and waits for the store, then reads it back with the
  *   page, so no call sees a half-written row.
- *   pages_per_split (1..64): pages one workgroup walks (the split-K grain); the workspace holds the partials.
+ *   pages_per_split (1..64): most pages one workgroup walks (the split-K grain); with a workspace, a launch that would
+ *   leave CUs idle walks fewer. The workspace holds the partials; one sized for B users, a table of max_blocks and T
+ *   tokens serves calls of fewer of each.
  *   A user with seq_lens[b] < T is an idle slot: nothing is appended or attended and its output rows are
  *   zero. A user with seq_lens[b] > max_blocks * block is treated the same and reported (QS_STATUS_LENGTH);
  *   a page entry outside [0, num_blocks) is not attended and is reported (QS_STATUS_PAGE).

@@ -85,6 +85,19 @@ def test_workspace_sizes():
     assert L.qs_paged_attention_workspace_bytes(1, 1, 24, 4, 128, 512, 8) == 0
 
 
+def test_attention_workspace_serves_smaller_calls():
+    """A workspace sized for a call holds the partials of every call of fewer users, tokens or table entries, though a
+    smaller grid is cut into more splits."""
+    size = lambda B, T, mb, pps: Q.lib().qs_paged_attention_workspace_bytes(B, T, 24, 4, 256, mb, pps)  # noqa: E731
+    for pps in (1, 2, 8, 16, 64):
+        for T in (1, 4, 16):
+            for B in (1, 3, 8, 70):
+                for mb in (1, 7, 64, 500):
+                    whole = size(B, T, mb, pps)
+                    assert all(size(b, t, m, pps) <= whole
+                               for b in (1, B // 2 + 1, B) for t in (1, T) for m in (1, mb // 3 + 1, mb) if b <= B and m <= mb)  # fmt: skip
+
+
 def test_ops_validate_before_calling():
     cpu = torch.zeros(1, 16, 128, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="GPU"):

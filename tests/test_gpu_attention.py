@@ -64,6 +64,20 @@ def test_attention_ragged_users(dev):
     torch.testing.assert_close(o[0, 0].cpu().float(), d["v_new"][0, 0].float().repeat_interleave(6, 0), rtol=0, atol=0)
 
 
+# The pages a workgroup walks follow the grid: 8 users of 8 pages at 2 pages per split are cut to one page (256
+# workgroups), 9 users keep two (288 would be past them); 64 users keep one split of 5 pages each, 70 users two splits of
+# up to 4 pages, walked two at a time, at 1, 4 and 8 tokens (6, 24 and 48 query rows per KV head)
+@pytest.mark.parametrize("B,pages,T,pps", [(8, 8, 1, 2), (9, 8, 1, 2), (64, 5, 1, 8), (70, 5, 1, 4), (70, 5, 4, 4),
+                                           (70, 5, 8, 4), (1, 20, 1, 7), (2, 30, 5, 16)])  # fmt: skip
+def test_attention_walked_pages(dev, B, pages, T, pps):
+    d = W.attn_layer(B, pages * 64, "cpu", seed=B + T, T=T, num_blocks=B * pages + 8)
+    gen = torch.Generator().manual_seed(B)
+    d["seq_lens"] = torch.randint(T, pages * 64 + 1, (B,), generator=gen).to(torch.int32)
+    o, o_ref, same = run_case(dev, d, pps)
+    assert same
+    assert_attn_output(o, o_ref)
+
+
 def test_attention_unfused_equals_fused(dev):
     d = W.attn_layer(2, 1000, "cpu", seed=5, T=2, num_blocks=64)
     o1, ref, _ = run_case(dev, d, pps=4, fused=True)

@@ -18,6 +18,8 @@
 // (the leader side of the reference: global max, rescale, sum, normalise, kernels/attn_leader_writer.cpp:
 // 86-106 and kernels/attn_leader_compute.cpp:42-79) by the last workgroup of the (user, KV head) to finish
 // when there are at most 16 splits, else by a separate merge launch, so results are identical run to run.
+#include <algorithm>
+
 #include "qs_common.h"
 
 namespace {
@@ -221,7 +223,7 @@ typedef short i16x4_t __attribute__((ext_vector_type(4)));
 constexpr int QPAD = HD + 8;   // s_q row pitch (bf16): 16-byte skew between rows
 constexpr int VPAD = HD + 16;  // K / V slice row pitch (bf16): 32-byte skew between rows
 
-// Split merge inside the attention launch (nsplit <= MERGE_MAX). Every workgroup of (user b, KV head g) has
+// Split merge inside the attention launch (nsplit <= MERGE_MAX, at most MERGE_ROWS query rows per KV head). Every workgroup of (user b, KV head g) has
 // stored its partial with agent-coherent stores (sc1: written through the XCD's L2); each thread waits for
 // its stores to complete, then one thread counts the workgroup in (the count wraps to zero at the last
 // arrival). The workgroup that completes the count merges: wave w of NWV takes query rows w, w + NWV, ...
@@ -231,7 +233,10 @@ constexpr int VPAD = HD + 16;  // K / V slice row pitch (bf16): 32-byte skew bet
 // invalidate is needed because only sc1 accesses touch the shared data. (The leader side of the
 // reference: kernels/attn_leader_writer.cpp:86-106, kernels/attn_leader_compute.cpp:42-79.)
 constexpr int MERGE_MAX = 16;
-constexpr int MERGE_ROWS = 32;  // query rows per KV head up to which one workgroup merges
+// Steps of more query rows leave the merge to its own launch: one workgroup would read their partials in several round
+// trips (per layer, batch 1 / 3 tokens at 100 positions, 2 splits: 14.8 us in its own launch, 16.5 in the same; batch
+// 1 / 4 tokens at 1000, 16 splits: 15.2 and 21.3).
+constexpr int MERGE_ROWS = 16;
 template <int NWV>
 __device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b, int g, int tid) {
     __shared__ int s_last;
@@ -731,8 +736,6 @@ __global__ __launch_bounds__(256 * WPP) void attn_rows_kernel(AttnArgs a, int G,
                                                       row * 8, 0, qs::CP_SC1);
         }
     }
-    if constexpr (NQR <= MERGE_ROWS)
-        if (a.nsplit > 1 && a.nsplit <= MERGE_MAX) merge_in_launch<NTH / 64>(a, G, b, g, tid);
 }
 
 // ------------------------------------------------------------------- MFMA kernel, independent waves
@@ -1202,6 +1205,9 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
 // rescale, sum, normalise, kernels/attn_leader_writer.cpp:86-106, kernels/attn_leader_compute.cpp:42-79.)
 constexpr int MAX_SPLITS = 1024;
 constexpr int MCH = 16;  // splits per wave per batch of loads (64 splits in one round trip)
+// MLR: 64-split groups of (m, l) pairs read. Up to 64 splits take 1, whose maxima also weight the partials: 31 fewer
+// loads per wave (two layers at batch 1 / 32768, 64 splits: 61.9 -> 61.0 us).
+template <int MLR>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
     __shared__ float4 s_part[4][64];
     const int rowh = blockIdx.x;  // ((b * T + t) * NKV + g) * G + h
@@ -1223,7 +1229,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
     auto load_split = [&](int sp, float4 &v, float &m) {  // sp wave-uniform, < ns
         const u32x4 u = __builtin_amdgcn_raw_buffer_load_b128(rpo, lane * 16, sp * sbytes, 0);
         v = make_float4(__uint_as_float(u[0]), __uint_as_float(u[1]), __uint_as_float(u[2]), __uint_as_float(u[3]));
-        m = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rml, 0, sp * R * 8, 0));
+        if constexpr (MLR > 1) m = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rml, 0, sp * R * 8, 0));
     };
     float4 x[MCH];
     float mw[MCH];
@@ -1231,9 +1237,9 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
     for (int k = 0; k < MCH; ++k) load_split(min(w + 4 * k, ns - 1), x[k], mw[k]);
     // global max and sum over all splits: lane l covers splits l, l + 64, ...
     float M = -INFINITY;
-    float2 mg[MAX_SPLITS / 64];
+    float2 mg[MLR];
 #pragma unroll
-    for (int j = 0; j < MAX_SPLITS / 64; ++j) {
+    for (int j = 0; j < MLR; ++j) {
         const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(rml, (lane + 64 * j) * R * 8, 0, 0);
         mg[j] = lane + 64 * j < ns ? make_float2(__uint_as_float(u[0]), __uint_as_float(u[1]))
                                    : make_float2(-INFINITY, 0.f);
@@ -1247,7 +1253,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
     M = qs::wave_max_bcast(M);
     float L = 0.f;
 #pragma unroll
-    for (int j = 0; j < MAX_SPLITS / 64; ++j)
+    for (int j = 0; j < MLR; ++j)
         if (mg[j].x != -INFINITY) L += __builtin_amdgcn_exp2f(mg[j].x - M) * mg[j].y;
     L = qs::wave_sum_dpp(L);
     float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1258,12 +1264,14 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
         }
     };
 #pragma unroll
-    for (int k = 0; k < MCH; ++k) acc(w + 4 * k, x[k], mw[k]);
-    for (int s0 = 4 * MCH; s0 < ns; s0 += 4 * MCH) {  // further splits, a batch of loads at a time
+    for (int k = 0; k < MCH; ++k) acc(w + 4 * k, x[k], MLR > 1 ? mw[k] : qs::lane_val(mg[0].x, w + 4 * k));
+    if constexpr (MLR > 1) {
+        for (int s0 = 4 * MCH; s0 < ns; s0 += 4 * MCH) {  // further splits, a batch of loads at a time
 #pragma unroll
-        for (int k = 0; k < MCH; ++k) load_split(min(s0 + w + 4 * k, ns - 1), x[k], mw[k]);
+            for (int k = 0; k < MCH; ++k) load_split(min(s0 + w + 4 * k, ns - 1), x[k], mw[k]);
 #pragma unroll
-        for (int k = 0; k < MCH; ++k) acc(s0 + w + 4 * k, x[k], mw[k]);
+            for (int k = 0; k < MCH; ++k) acc(s0 + w + 4 * k, x[k], mw[k]);
+        }
     }
     s_part[w][lane] = O;
     __syncthreads();
@@ -1282,6 +1290,20 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
 }
 
 int nsplit_of(int max_blocks, int pps) { return (max_blocks + pps - 1) / pps; }
+// Pages a workgroup walks: the caller's, or half of them, and so on, while the whole launch stays within one workgroup
+// per CU. A page takes its waves ~2 us of dependent latency (load, scores, softmax, P V), so a grid that leaves CUs
+// idle is cut finer; past 256 workgroups the partials cost more than the shorter walks save. Per layer with the mixer,
+// the caller's pages -> the rule's: batch 1, 8 pages: 200 positions 13.0 -> 11.4 us (4 workgroups -> 16), 1000 19.1
+// -> 12.3, 4096 19.7 -> 13.2; 16 pages, 2000: 26.4 -> 11.0; batch 4, 8 pages, ragged 1000: 19.3 -> 13.7; batch 1 / 4
+// tokens, 8 pages, 1000: 29.5 -> 15.2. One step finer than the rule: batch 1 / 8192 18.6 against 16.1, batch 4 / 4096
+// 26.4 against 20.4, batch 8 / 2048 27.7 against 18.6. Only sizes known to the host enter the rule, so a user's result
+// depends on no other user's length.
+constexpr int FINE_WGS = 256;
+int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps) {
+    const int nrb = (T * G + 63) / 64;  // row blocks of attn_rows_kernel (1 in attn_wave_kernel)
+    while (pps > 1 && (long)B * NKV * nrb * nsplit_of(max_blocks, (pps + 1) / 2) <= FINE_WGS) pps = (pps + 1) / 2;
+    return pps;
+}
 // Pages a workgroup of the independent-wave kernel walks at once (4 waves each): two when the split has more
 // than one page (batch 8 at 4096 positions: 26.8 against 27.7 us; batch 1 at 32768: 29.8 against 30.4).
 int attn_wpp(int pps) { return pps >= 2 ? 2 : 1; }
@@ -1291,12 +1313,15 @@ int attn_wpp(int pps) { return pps >= 2 ? 2 : 1; }
 extern "C" size_t qs_paged_attention_workspace_bytes(int B, int T, int NQ, int NKV, int HDa, int max_blocks,
                                                      int pages_per_split) {
     if (B <= 0 || T <= 0 || NKV <= 0 || NQ % NKV || HDa != HD || max_blocks <= 0 || pages_per_split <= 0) return 0;
-    const int ns = nsplit_of(max_blocks, pages_per_split);
-    return ws_layout(B, T, NKV, NQ / NKV, ns).total;
+    const int G = NQ / NKV, ns = nsplit_of(max_blocks, walk_pages(B, T, NKV, G, max_blocks, pages_per_split));
+    // at least FINE_WGS partials, which no smaller call of the same T exceeds (a smaller batch or a narrower table is
+    // cut finer): a workspace sized for the largest call serves them all
+    return ws_layout(std::max(B * NKV * ns, FINE_WGS), T, 1, G, 1).total;
 }
 
 static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const char *who, void *stream) {
-    const int B = a.B, T = a.T, NQ = a.NQ, NKV = a.NKV, max_blocks = a.max_blocks, pages_per_split = a.pps;
+    const int B = a.B, T = a.T, NQ = a.NQ, NKV = a.NKV, max_blocks = a.max_blocks;
+    int pages_per_split = a.pps;
     QS_REQUIRE(a.q && a.k_cache && a.v_cache && a.block_table && a.seq_lens && a.o, "%s: null pointer", who);
     QS_REQUIRE((a.k_new == nullptr) == (a.v_new == nullptr), "%s: give both k_new and v_new or neither", who);
     QS_REQUIRE(HDa == HD, "%s: HD must be %d (got %d)", who, HD, HDa);
@@ -1307,12 +1332,16 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
     QS_REQUIRE(pages_per_split > 0 && pages_per_split <= 64, "%s: pages_per_split must be in [1, 64] (got %d)", who,
                pages_per_split);
     const int G = NQ / NKV;
-    const int ns = nsplit_of(max_blocks, pages_per_split);
+    int ns = nsplit_of(max_blocks, pages_per_split);
     QS_REQUIRE(ns == 1 || workspace, "%s: %d splits need a workspace", who, ns);
     QS_REQUIRE(ns <= MAX_SPLITS, "%s: %d splits exceed %d (raise pages_per_split)", who, ns, MAX_SPLITS);
     QS_REQUIRE((long)B * NKV * ns < (1L << 31), "%s: grid too large", who);
     QS_REQUIRE((size_t)B * NKV * sizeof(int) <= CNT_BYTES, "%s: B NKV = %d exceeds %d", who, B * NKV,
                (int)(CNT_BYTES / sizeof(int)));
+    if (workspace) {
+        pages_per_split = a.pps = walk_pages(B, T, NKV, G, max_blocks, pages_per_split);
+        ns = nsplit_of(max_blocks, pages_per_split);
+    }
     a.nsplit = ns;
     if (workspace) {
         const WsLayout L = ws_layout(B, T, NKV, G, ns);
@@ -1364,7 +1393,10 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
     }
     if (int e = qs::launch_status(who)) return e;
     if (ns > 1 && (ns > MERGE_MAX || R > MERGE_ROWS)) {  // the rest are merged inside the attention launch
-        attn_merge_kernel<<<B * T * NKV * G, 256, 0, st>>>(a, G);
+        if (ns <= 64)
+            attn_merge_kernel<1><<<B * T * NKV * G, 256, 0, st>>>(a, G);
+        else
+            attn_merge_kernel<MAX_SPLITS / 64><<<B * T * NKV * G, 256, 0, st>>>(a, G);
         return qs::launch_status(who);
     }
     return QS_OK;
