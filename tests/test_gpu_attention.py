@@ -66,9 +66,11 @@ def test_attention_ragged_users(dev):
 
 # The pages a workgroup walks follow the grid: 8 users of 8 pages at 2 pages per split are cut to one page (256
 # workgroups), 9 users keep two (288 would be past them); 64 users keep one split of 5 pages each, 70 users two splits of
-# up to 4 pages, walked two at a time, at 1, 4 and 8 tokens (6, 24 and 48 query rows per KV head)
+# up to 4 pages, walked two at a time, at 1, 4 and 8 tokens (6, 24 and 48 query rows per KV head); 4 users of 65 pages
+# walk 6 of the caller's 8, 5 users of 50 the caller's 5
 @pytest.mark.parametrize("B,pages,T,pps", [(8, 8, 1, 2), (9, 8, 1, 2), (64, 5, 1, 8), (70, 5, 1, 4), (70, 5, 4, 4),
-                                           (70, 5, 8, 4), (1, 20, 1, 7), (2, 30, 5, 16)])  # fmt: skip
+                                           (70, 5, 8, 4), (1, 20, 1, 7), (2, 30, 5, 16), (4, 65, 8, 8),
+                                           (5, 50, 1, 5)])  # fmt: skip
 def test_attention_walked_pages(dev, B, pages, T, pps):
     d = W.attn_layer(B, pages * 64, "cpu", seed=B + T, T=T, num_blocks=B * pages + 8)
     gen = torch.Generator().manual_seed(B)

@@ -1290,19 +1290,21 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
 }
 
 int nsplit_of(int max_blocks, int pps) { return (max_blocks + pps - 1) / pps; }
-// Pages a workgroup walks: the caller's, or half of them, and so on, while the whole launch stays within one workgroup
-// per CU. A page takes its waves ~2 us of dependent latency (load, scores, softmax, P V), so a grid that leaves CUs
-// idle is cut finer; past 256 workgroups the partials cost more than the shorter walks save. Per layer with the mixer,
-// the caller's pages -> the rule's: batch 1, 8 pages: 200 positions 13.0 -> 11.4 us (4 workgroups -> 16), 1000 19.1
-// -> 12.3, 4096 19.7 -> 13.2; 16 pages, 2000: 26.4 -> 11.0; batch 4, 8 pages, ragged 1000: 19.3 -> 13.7; batch 1 / 4
-// tokens, 8 pages, 1000: 29.5 -> 15.2. One step finer than the rule: batch 1 / 8192 18.6 against 16.1, batch 4 / 4096
-// 26.4 against 20.4, batch 8 / 2048 27.7 against 18.6. Only sizes known to the host enter the rule, so a user's result
-// depends on no other user's length.
+// Pages a workgroup walks: the caller's, or as few as keep the whole launch within one workgroup per CU (an even number
+// past one, for the two pages in flight). A page takes its waves ~2 us of dependent latency (load, scores, softmax,
+// P V), so a grid that leaves CUs idle is cut finer; past 256 workgroups the partials cost more than the shorter walks
+// save. Per layer with the mixer, the caller's pages -> the rule's: batch 1, 8 pages: 200 positions 13.0 -> 11.4 us (4
+// workgroups -> 16), 1000 19.1 -> 12.3, 4096 19.7 -> 13.2; 16 pages, 2000: 26.4 -> 11.0; batch 4, 8 pages, ragged
+// 1000: 19.3 -> 13.7; batch 1 / 4 tokens, 8 pages, 1000: 29.5 -> 15.2. One step finer than the rule: batch 1 / 8192
+// 18.6 against 16.1, batch 4 / 4096 26.4 against 20.4, batch 8 / 2048 27.7 against 18.6. Only sizes known to the host
+// enter the rule, so a user's result depends on no other user's length.
 constexpr int FINE_WGS = 256;
 int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps) {
     const int nrb = (T * G + 63) / 64;  // row blocks of attn_rows_kernel (1 in attn_wave_kernel)
-    while (pps > 1 && (long)B * NKV * nrb * nsplit_of(max_blocks, (pps + 1) / 2) <= FINE_WGS) pps = (pps + 1) / 2;
-    return pps;
+    const long most = FINE_WGS / ((long)B * NKV * nrb);  // splits per user and KV head
+    if (most == 0) return pps;
+    const int p = (int)((max_blocks + most - 1) / most);
+    return std::min(pps, p > 1 ? (p + 1) & ~1 : 1);
 }
 // Pages a workgroup of the independent-wave kernel walks at once (4 waves each): two when the split has more
 // than one page (batch 8 at 4096 positions: 26.8 against 27.7 us; batch 1 at 32768: 29.8 against 30.4).
