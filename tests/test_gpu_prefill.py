@@ -101,6 +101,21 @@ def test_prefill_then_decode_continues(dev):
     assert_bf16_output(o1[0], o2[129])
 
 
+def test_prefill_fresh_prompts_start_from_zero(dev):
+    """Without an initial state every call starts from zeros, also after calls whose final state was written in place and
+    with other head counts in between."""
+    d = {k: v.to(dev) for k, v in W.prefill(70, "cpu", seed=11).items()}
+    rows = [d[n] for n in ("q", "k", "v", "g", "beta")]
+    few = [t[:, :n].contiguous() for t, n in zip(rows, (4, 4, 8, 8, 8))]
+    o, S = ops.chunk_gated_delta_rule(*rows, initial_state=torch.zeros_like(d["S0"]))
+    o4, S4 = ops.chunk_gated_delta_rule(*few, initial_state=torch.zeros_like(d["S0"][:8]))
+    for _ in range(2):
+        o1, S1 = ops.chunk_gated_delta_rule(*rows, final_state=torch.empty_like(S))
+        o2, S2 = ops.chunk_gated_delta_rule(*few)
+        assert torch.equal(o1, o) and torch.equal(S1, S) and torch.equal(o2, o4) and torch.equal(S2, S4)
+        S1.fill_(7.0), S2.fill_(7.0)  # the outputs are the caller's
+
+
 def test_prefill_repeatable(dev):
     d = W.prefill(300, "cpu", seed=7)
     a = run(dev, d, 300)

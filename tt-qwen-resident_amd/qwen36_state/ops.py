@@ -512,6 +512,15 @@ def causal_conv1d_prefill(x, taps, conv_state=None, conv_state_out=None, nk=NK, 
     return q, k, v, conv_state_out
 
 
+def _zero_state(nv, dev):
+    """The zero start state of a fresh prompt, only ever read: a workspace of its own size, cleared once per stream
+    instead of by a launch per call (3 MB at 48 heads; a 200-token prompt's conv, rule and fill 38.3 -> 36.1 us). A
+    captured call clears one inside its graph, which then depends on no buffer kept here."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.zeros(nv, DK, DV, dtype=torch.float32, device=dev)
+    return workspace(("zero state", nv), 4 * nv * DK * DV, dev).view(torch.float32).view(nv, DK, DV)
+
+
 def chunk_gated_delta_rule(q, k, v, g, beta, *, scale=None, initial_state=None, output_final_state=True,
                            chunk_size=64, output_head_major=False, memory_config=None, eye=None, tril=None,
                            ones=None, masks=None, eps=EPS, ws=None, final_state=None):  # fmt: skip
@@ -561,7 +570,7 @@ def chunk_gated_delta_rule(q, k, v, g, beta, *, scale=None, initial_state=None, 
     _chk(g, "g", torch.float32, (T, nv), dev)
     _chk(beta, "beta", torch.float32, (T, nv), dev)
     if initial_state is None:
-        initial_state = torch.zeros(nv, DK, DV, dtype=torch.float32, device=dev)
+        initial_state = _zero_state(nv, dev)
     _chk(initial_state, "initial_state", torch.float32, (nv, DK, DV), dev)
     scale = DK**-0.5 if scale is None else scale
     o = torch.empty(T, nv, DV, dtype=torch.bfloat16, device=dev)
