@@ -80,7 +80,11 @@ def test_gdn_decode_from_x(dev, B, nk, nv, seed):
     assert_bf16_output(o, O.bf16(o_y))
 
 
-@pytest.mark.parametrize("B,T,nk,nv,seed", [(1, 4, 16, 48, 10), (2, 3, 16, 48, 11), (12, 2, 16, 32, 12)])
+# batch 1 and 2, and more than 4 tokens below batch 6: the conv spread over the slab's waves (2, 5, 6 and 8 tokens: a
+# last part that is empty, short or full); (3, 4): not spread
+@pytest.mark.parametrize("B,T,nk,nv,seed", [(1, 4, 16, 48, 10), (2, 3, 16, 48, 11), (12, 2, 16, 32, 12), (1, 2, 16, 48, 14),
+                                            (1, 5, 16, 48, 15), (2, 8, 16, 48, 16), (3, 6, 16, 48, 17),
+                                            (3, 4, 16, 48, 18)])  # fmt: skip
 def test_gdn_verify_from_x(dev, B, T, nk, nv, seed):
     """T tokens from x through the verify kernel against T sequential oracle decode steps from the same x."""
     d = layer(B, nk, nv, seed, T=T)

@@ -149,6 +149,59 @@ __device__ __forceinline__ void conv_commit(const GdnArgs &a, const ConvPair<TM>
     }
 }
 
+// N consecutive tokens of the pair, off .. off + N - 1 (off a multiple of N; a lane's own or the wave's): their inputs
+// s[e][i], i < N + 3, and outputs, the same arithmetic as conv_run.
+template <int N>
+struct ConvPart {
+    uint32_t s[2][N + 3], yb[N];
+};
+template <int TM, int N>
+__device__ __forceinline__ void conv_part(const ConvPair<TM> &in, int off, ConvPart<N> &p, float y[2][N]) {
+    float sv[2][N];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+#pragma unroll
+        for (int i = 0; i < N + 3; ++i) {
+            p.s[e][i] = conv_seq(in, e, i);
+#pragma unroll
+            for (int o = N; o < TM; o += N) p.s[e][i] = off == o ? conv_seq(in, e, i + o) : p.s[e][i];
+        }
+        const uint32_t tw0 = e ? in.tw.z : in.tw.x, tw1 = e ? in.tw.w : in.tw.y;
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            float acc = qs::bf2f(p.s[e][n]) * qs::bf_lo(tw0);
+            acc = acc + qs::bf2f(p.s[e][n + 1]) * qs::bf_hi(tw0);
+            acc = acc + qs::bf2f(p.s[e][n + 2]) * qs::bf_lo(tw1);
+            acc = acc + qs::bf2f(p.s[e][n + 3]) * qs::bf_hi(tw1);
+            sv[e][n] = qs::silu(acc);
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        p.yb[n] = qs::cvt_pk_bf16(sv[0][n], sv[1][n]);
+        y[0][n] = qs::bf_lo(p.yb[n]);
+        y[1][n] = qs::bf_hi(p.yb[n]);
+    }
+}
+// A verify part's global outputs: the conv outputs and the windows after its tokens, as conv_commit writes them
+template <int N>
+__device__ __forceinline__ void commit_part(const GdnArgs &a, const ConvPart<N> &p, int off, int b, int c, int T, bool write) {
+    const int ybytes = a.y_out ? a.B * T * a.C * 2 : 0, sbytes = T * a.B * a.C * (KC - 1) * 2;
+    const auto ry = __builtin_amdgcn_make_buffer_rsrc(a.y_out, (short)0, ybytes, 0x00020000);
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(a.conv_out, (short)0, sbytes, 0x00020000);
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const int t = off + n;
+        const bool w = write && t < T;
+        u32x3 win;
+        win.x = p.s[0][n + 1] | (p.s[0][n + 2] << 16);
+        win.y = p.s[0][n + 3] | (p.s[1][n + 1] << 16);
+        win.z = p.s[1][n + 2] | (p.s[1][n + 3] << 16);
+        __builtin_amdgcn_raw_buffer_store_b32(p.yb[n], ry, w ? ((b * T + t) * a.C + c) * 2 : ybytes, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b96(win, rs, w ? ((t * a.B + b) * a.C + c) * (KC - 1) * 2 : sbytes, 0, 0);
+    }
+}
+
 // Sum over the row groups of a slab wave (lane bits log2(CG) .. 5) as a butterfly in a fixed order: every
 // lane ends with bit-identical sums of its column group.
 template <int CG>
@@ -212,7 +265,7 @@ __device__ __forceinline__ const float *sp_of_t(const GdnArgs &a, size_t user, i
 // the mixer (model.py:274-275, the head cores' steps 7-8, kernels/gdn_head_compute.cpp:320-346) on the fp32 o
 // of the head: the slabs' sums of squares meet in LDS (one barrier per token) and o receives
 // bf16(o rsqrt(mean(o^2) + eps) norm_w silu(z)).
-template <bool CONV, bool VERIFY, int TM, int SLAB, int NW, int WPG, bool NORM = false>
+template <bool CONV, bool VERIFY, int TM, int SLAB, int NW, int WPG, bool NORM = false, bool SPLITC = false>
 __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     constexpr int NSLAB = DV / SLAB;
     constexpr int CG = SLAB / 4;   // column groups of 4 (lane % CG)
@@ -221,7 +274,7 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     constexpr int RPL = RW / RG;   // rows per lane
     static_assert(RPL >= 1 && RW % RG == 0 && (VERIFY || TM == 1), "slab shape");
     static_assert(!NORM || (!VERIFY && WPG == NSLAB && CG <= 16), "the epilogue needs whole heads per workgroup");
-    // conv roles by wave of the workgroup: q channels on wave 0, k on wave 1 (when there is one; NW = 2: wave 2), the
+    // conv roles by wave of the workgroup (SPLITC below: otherwise): q channels on wave 0, k on wave 1 (when there is one; NW = 2: wave 2), the
     // slab's v channels on wave 2 (NW = 4), each slab's wave 1 (NW = 2) or every wave for its own slab (NW = 1)
     constexpr int WK = NW == 2 && WPG >= 2 ? 2 : (NW >= 4 || WPG >= 2) ? 1 : 0;
     constexpr int WV = NW >= 4 ? 2 : NW - 1;
@@ -232,6 +285,11 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     // The column sums of the forms with several waves per slab are taken over 32-row blocks, 4 to a slab, and added in
     // row order, so that 2 and 4 waves per slab give the same bits
     constexpr int NB = NW > 1 ? 4 / NW : 1;  // row blocks per wave
+    // SPLITC (verify, 4 waves per slab): the conv of a step's tokens spread over the waves, q on waves 0 and 2, k on 1 and
+    // 3, half the tokens each, the slab's v channels on wave 2 with a quarter of the tokens per 16 lanes (on one wave
+    // each for q, k and v the chain begins with T x 2 SiLUs and T norms in a row)
+    static_assert(!SPLITC || (CONV && VERIFY && NW == 4), "the spread conv is the small-batch verify's");
+    constexpr int NH = SPLITC ? TM / 2 : 1, NV4 = SPLITC ? TM / 4 : 1;
     // The one-wave-per-slab form: the load addresses' kernel arguments, requested with the first batch of
     // argument loads (the compiler would otherwise request them after the index arithmetic below, a second
     // round trip before the first load; the other forms already request them in one batch, and the fence
@@ -315,7 +373,7 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
         }
         return;
     }
-    ConvPair<TM> inq, ink, inv;
+    ConvPair<TM> inq, ink, inv;  // SPLITC: inq holds the wave's q or k pair
     // Decode + conv: the waves holding the q/k channels count themselves in once their history is consumed.
     // Every wave issues the same buffer atomic, out of range on every lane but lane 0 of the q and k waves, so
     // no branch surrounds it and the compiler's waits for the state loads leave it in flight (a conditional
@@ -331,7 +389,10 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
         const int off = (lane == 0 && (isq || isk)) ? (isq ? 0 : 4) : 8;
         return __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(kq_owner ? 1 - rep * NSLAB / WPG : 1, rc, off, 0, 0);
     };
-    if (CONV) {
+    if constexpr (SPLITC) {
+        inq = conv_load<TM>(a, conv_b, b, (w & 1) ? ck : cq, T);
+        if (isv) inv = conv_load<TM>(a, conv_b, b, cv, T);
+    } else if (CONV) {
         if (isq) inq = conv_load<TM>(a, conv_b, b, cq, T);
         if (isk) ink = conv_load<TM>(a, conv_b, b, ck, T);
         if (isv) inv = conv_load<TM>(a, conv_b, b, cv, T);
@@ -375,7 +436,30 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     // 2. q, k (rows 2 lane, 2 lane + 1) and the v slab for every token; L2 norms (q times scale).
     float qv[2][TM], kv[2][TM], vv[2][TM];
     uint32_t yq[TM], yk[TM], yv[TM];
-    if (CONV) {
+    ConvPart<NH> part;
+    ConvPart<NV4> vpart;
+    const int hoff = (w >> 1) * NH, voff = (lane >> 4) * NV4;  // SPLITC: the wave's first token, the lane's for v
+    if constexpr (SPLITC) {
+        float y[2][NH], yv4[2][NV4];
+        conv_part<TM, NH>(inq, hoff, part, y);
+        const int r0 = 2 * lane, rr = r0 % RW;
+        const int p0 = (r0 / RW) * RW + (rr % RG) * RPL + rr / RG;  // stored position of row r0 (+ RPL: r0 + 1)
+#pragma unroll
+        for (int n = 0; n < NH; ++n) {
+            if (hoff + n >= T) break;
+            const float rn = rsqrtf(qs::wave_sum_dpp(y[0][n] * y[0][n] + y[1][n] * y[1][n]) + a.eps) * ((w & 1) ? 1.f : a.scale);
+            float *row = (w & 1) ? s_kn[hoff + n] : s_qn[hoff + n];
+            row[p0] = y[0][n] * rn;
+            row[p0 + RPL] = y[1][n] * rn;
+        }
+        if (isv) {
+            conv_part<TM, NV4>(inv, voff, vpart, yv4);
+#pragma unroll
+            for (int n = 0; n < NV4; ++n)
+                if (voff + n < T)
+                    *reinterpret_cast<float2 *>(&s_v[voff + n][2 * (lane & 15)]) = make_float2(yv4[0][n], yv4[1][n]);
+        }
+    } else if (CONV) {
         if (isq) conv_run<TM>(inq, T, qv, yq);
         if (isk) conv_run<TM>(ink, T, kv, yk);
         if (isv) conv_run<TM>(inv, T, vv, yv);
@@ -400,7 +484,7 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
             }
         }
     }
-    {
+    if constexpr (!SPLITC) {
         const int r0 = 2 * lane, rr = r0 % RW;
         const int p0 = (r0 / RW) * RW + (rr % RG) * RPL + rr / RG;  // stored position of row r0 (+ RPL: r0 + 1)
 #pragma unroll
@@ -516,9 +600,14 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
             // the rep * NSLAB workgroups of key head kh, which in decode count themselves in (q and k
             // separately when different waves hold them): the last to arrive writes the shifted state at the
             // end, where the count's return is waited for.
-            if (isv) conv_commit<VERIFY, TM>(a, inv, yv, b, cv, T, lane < SLAB / 2, lane < SLAB / 2);
-            if (isq) conv_commit<VERIFY, TM>(a, inq, yq, b, cq, T, kq_owner, VERIFY && kq_owner);
-            if (isk) conv_commit<VERIFY, TM>(a, ink, yk, b, ck, T, kq_owner, VERIFY && kq_owner);
+            if constexpr (SPLITC) {
+                commit_part(a, part, hoff, b, (w & 1) ? ck : cq, T, kq_owner);
+                if (isv) commit_part(a, vpart, voff, b, cv, T, true);
+            } else {
+                if (isv) conv_commit<VERIFY, TM>(a, inv, yv, b, cv, T, lane < SLAB / 2, lane < SLAB / 2);
+                if (isq) conv_commit<VERIFY, TM>(a, inq, yq, b, cq, T, kq_owner, VERIFY && kq_owner);
+                if (isk) conv_commit<VERIFY, TM>(a, ink, yk, b, ck, T, kq_owner, VERIFY && kq_owner);
+            }
             if constexpr (!VERIFY && NW == 1) arrived = count_in();
         }
         float dl[4];
@@ -733,8 +822,20 @@ void launch_gdn_tm(const GdnArgs &a, hipStream_t st) {
         gdn_kernel<CONV, VERIFY, TM, 32, 1, 6><<<units / 6, 384, 0, st>>>(a);
     else if (units >= 1024)
         gdn_kernel<CONV, VERIFY, TM, 32, 1, 4><<<units / 4, 256, 0, st>>>(a);
-    else
-        gdn_kernel<CONV, VERIFY, TM, 32, 4, 1><<<units, 256, 0, st>>>(a);
+    else {
+        // verify: the conv spread over the slab's waves for every step of more than 4 tokens, for shorter ones up to two
+        // workgroups per CU (more of them hide each other's chains, and the q and k inputs are then loaded twice for
+        // nothing). One wave each -> spread, us: batch 1, 12 layers of 2 tokens 69.2 -> 65.8, of 4 88.0 -> 84.9, 6 of 8
+        // 77.4 -> 67.1; batch 2, 6 layers of 3 49.1 -> 46.9; batch 3, 6 layers of 2 50.2 -> 59.3, 4 of 4 49.1 -> 48.6, 2
+        // of 8 46.9 -> 44.5; batch 5, 3 layers of 3 42.9 -> 51.2, 1 of 8 36.6 -> 32.5
+        if constexpr (VERIFY) {
+            if (TM > 4 || units <= 512) {
+                gdn_kernel<CONV, VERIFY, TM, 32, 4, 1, false, true><<<units, 256, 0, st>>>(a);
+                return;
+            }
+        }
+        if constexpr (!VERIFY || TM <= 4) gdn_kernel<CONV, VERIFY, TM, 32, 4, 1><<<units, 256, 0, st>>>(a);
+    }
 }
 template <bool CONV, bool VERIFY>
 void launch_gdn(const GdnArgs &a, hipStream_t st) {
