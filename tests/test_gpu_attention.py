@@ -347,3 +347,25 @@ def test_verify_row_blocks_idle_and_bad_page(dev):
         seen = keep & (torch.arange(900) <= 900 - T + t)
         s = (d["q"][2, t].float().view(4, 6, 256) @ K[:, seen].transpose(1, 2)) * d["scale"]
         assert_attn_output(o[2, t].view(4, 6, 256), O.bf16(s.softmax(-1) @ V[:, seen]))
+
+
+# A step of 3 or more tokens with at most 16 query rows per KV head stores its new rows first and reads the pages they
+# lie in again. A grid of at most 256 workgroups walks one page each whatever the caller asks for (2 users x 4 KV heads
+# x 4 pages), where K is read in the score operand's layout; 66 users x 4 KV heads are past that and walk the caller's
+# two pages at a time. The new rows cross a page, end one, fill a user's cache or start it.
+@pytest.mark.parametrize("G,T", [(4, 3), (4, 4), (2, 3), (2, 8), (1, 3), (1, 16)])
+@pytest.mark.parametrize("B,pps", [(2, 1), (2, 8), (66, 2)])
+@pytest.mark.parametrize("mixer", [False, True])
+def test_few_rows_append(dev, G, T, B, pps, mixer):
+    gen = torch.Generator().manual_seed(G * 100 + T + B)
+    d = W.attn_layer(B, 256, "cpu", seed=G * 100 + T + pps, T=T, num_blocks=B * 4 + 8)
+    d["q"] = torch.randn(B, T, G * 4, 256, generator=gen).bfloat16()
+    d["seq_lens"] = torch.tensor(([130, 256] + [T, 64, 65, 192] * 16)[:B], dtype=torch.int32)
+    assert d["block_table"].shape[1] == 4
+    if mixer:
+        return check_mixer(dev, d, pps, 64, gen)
+    o1, ref, same1 = run_case(dev, d, pps, fused=True)
+    o2, _, same2 = run_case(dev, d, pps, fused=False)
+    assert same1 and same2
+    assert torch.equal(o1.cpu(), o2.cpu())
+    assert_attn_output(o1, ref)

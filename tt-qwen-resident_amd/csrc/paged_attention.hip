@@ -905,7 +905,10 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         }
         qs::wait_vmem();
         if (pg0 >= 0 && base / BLK <= pf) {  // new rows landed in this wave's first page: read it again
-            load_rows(a.k_cache, pg0, KA);
+            if constexpr (WPP == 1)
+                load_kfrag(pg0, KA);
+            else
+                load_rows(a.k_cache, pg0, KA);
             load_rows(a.v_cache, pg0, VA);
         }
     }
