@@ -12,6 +12,25 @@ pytestmark = pytest.mark.gpu
 CNT_BYTES = 65536  # the fixed counter block at the head of an attention workspace
 
 
+def plan(B, T, G, width, pps, nkv=4):
+    """How a call with a workspace is cut (the rules of the library's launch): pages a workgroup walks, splits, and
+    whether the attention launch merges them itself. The tests below choose their shapes by it."""
+    R = T * G
+    most = 256 // (B * nkv * -(-R // 64))
+    p = -(-width // most) if most else pps
+    p = min(pps, p if p <= 1 or not most else p + p % 2)
+    ns = -(-width // p)
+    return p, ns, 1 < ns and R <= 16 and (ns <= 4 or ns <= 8 and R <= (16 if p > 1 else 8))
+
+
+def split_rows(ws):
+    """The rows of split partials a call wrote (every split holding pages) into a workspace whose bytes past the counters
+    were 0xFF, from the first float that is still a NaN: 2 floats (m, l) a row, padded to 256 bytes, then 256 of O."""
+    nan = ws[CNT_BYTES:].view(torch.float32).isnan().cpu()
+    n = int(nan.float().argmax()) if bool(nan.any()) else len(nan)
+    return n // 2 if n % 64 else n // 258
+
+
 def run_case(dev, d, pps, fused=True):
     """Attention (+ append) on the GPU and the same step through the oracle; returns (o_gpu, o_ref,
     pools equal)."""
@@ -163,30 +182,58 @@ def test_attn_mixer(dev, B, ctx, T, pps):
 
 
 def test_in_launch_merge_counters_rearm(dev):
-    """Up to 16 splits are merged inside the attention launch by the last workgroup to arrive. The arrival
-    counters at the workspace head read zero after every call, so one workspace serves repeated calls and
-    calls of other shapes (here batch 8 one token, then batch 3 four verify rows, twice each): outputs repeat
-    bit-exactly and match the oracle."""
+    """Few splits are merged inside the attention launch by the last workgroup to arrive. The arrival counters at the
+    workspace head read zero after every call, so one workspace serves repeated calls and calls of other shapes (here
+    8, 5 and 4 splits of batch 8, 3 and 6, one and two tokens, twice each): outputs repeat bit-exactly and match the
+    oracle."""
     L = ops.lib()
-    ws = torch.zeros(L.qs_paged_attention_workspace_bytes(8, 4, 24, 4, 256, 64, 4), dtype=torch.uint8, device=dev)
-    cases = [(8, 4096, 1), (3, 2000, 4)]
-    data = [W.attn_layer(B, ctx, "cpu", seed=B + T, T=T, num_blocks=1024) for B, ctx, T in cases]
+    cases = [(8, 4096, 1, 8, 8), (3, 300, 1, 4, 5), (6, 250, 2, 2, 4)]  # users, positions, tokens, pages, splits
+    assert all(plan(B, T, 6, -(-ctx // 64), pps)[1:] == (ns, True) for B, ctx, T, pps, ns in cases)
+    nbytes = max(L.qs_paged_attention_workspace_bytes(B, T, 24, 4, 256, -(-ctx // 64), pps) for B, ctx, T, pps, _ in cases)
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+    data = [W.attn_layer(B, ctx, "cpu", seed=B + T, T=T, num_blocks=1024) for B, ctx, T, _, _ in cases]
     outs = []
     for rep in range(2):
-        for d in data:
+        for d, (_, _, _, pps, _) in zip(data, cases):
             g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
             o = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"],
-                                     pages_per_split=4, ws=ws)  # fmt: skip
+                                     pages_per_split=pps, ws=ws)  # fmt: skip
             torch.cuda.synchronize()
             assert int(ws[:CNT_BYTES].view(torch.int32).abs().sum()) == 0, "counters not re-armed"
             outs.append(o.cpu())
-    assert torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[3])
+    n = len(cases)
+    assert all(torch.equal(outs[i], outs[i + n]) for i in range(n))
     for d, o in zip(data, outs):
         ref = O.gqa_decode(d["q"], d["k_cache"], d["v_cache"], d["block_table"], d["seq_lens"], d["scale"])
         assert_attn_output(o, O.bf16(ref))
 
 
-# More than 16 splits go through the separate merge launch (one workgroup per output row, the partials merged in
+# Where the merge moves between the launches: 4 and 5 splits of 12 rows and 8 and 9 of 6 on one page per workgroup, 8 and
+# 9 of 12 rows on two pages, 2 splits of 16 rows (group size 8) and of 18. The partials written show the split count.
+@pytest.mark.parametrize("B,G,T,width,pps,splits,merged", [
+    (6, 6, 2, 4, 2, 4, True), (2, 6, 2, 5, 2, 5, False), (2, 6, 1, 8, 8, 8, True), (2, 6, 1, 9, 8, 9, False),
+    (8, 6, 2, 16, 2, 8, True), (7, 6, 2, 18, 8, 9, False), (64, 8, 2, 5, 4, 2, True), (64, 6, 3, 5, 4, 2, False),
+])  # fmt: skip
+def test_merge_split_counts(dev, B, G, T, width, pps, splits, merged):
+    assert plan(B, T, G, width, pps)[1:] == (splits, merged)
+    d = W.attn_layer(B, width * 64, "cpu", seed=B + T + width, T=T, num_blocks=B * width + 8)
+    gen = torch.Generator().manual_seed(width)
+    d["q"] = torch.randn(B, T, G * 4, 256, generator=gen).bfloat16()
+    d["seq_lens"] = torch.randint((width - 1) * 64 + T, width * 64 + 1, (B,), generator=gen).to(torch.int32)
+    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+    ws = torch.zeros(ops.lib().qs_paged_attention_workspace_bytes(B, T, G * 4, 4, 256, width, pps), dtype=torch.uint8,
+                     device=dev)  # fmt: skip
+    ws[CNT_BYTES:] = 0xFF
+    o = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"],
+                             k_new=g["k_new"], v_new=g["v_new"], pages_per_split=pps, ws=ws)  # fmt: skip
+    assert split_rows(ws) == B * 4 * splits * T * G
+    assert int(ws[:CNT_BYTES].view(torch.int32).abs().sum()) == 0, "counters not re-armed"
+    kc, vc = d["k_cache"].clone(), d["v_cache"].clone()
+    O.paged_append(kc, vc, d["k_new"], d["v_new"], d["block_table"], d["seq_lens"] - T)
+    assert_attn_output(o, O.bf16(O.gqa_decode(d["q"], kc, vc, d["block_table"], d["seq_lens"], d["scale"])))
+
+
+# More splits go through the separate merge launch (one workgroup per output row, the partials merged in
 # split order): 18, 64, 512 and 1024 splits, verify rows on the MFMA kernel at 64, 32 and 18 splits, batch 3 with
 # an idle user at 32 and 18 splits. Three calls give the same bits, match the oracle, leave the in-launch counters
 # at zero and report nothing.

@@ -17,7 +17,7 @@
 // The splits' partials (m, l, unnormalised O per query row) go to the workspace and are merged in split order
 // (the leader side of the reference: global max, rescale, sum, normalise, kernels/attn_leader_writer.cpp:
 // 86-106 and kernels/attn_leader_compute.cpp:42-79) by the last workgroup of the (user, KV head) to finish
-// when there are at most 16 splits, else by a separate merge launch, so results are identical run to run.
+// when there are few (AttnArgs::merge), else by a separate merge launch, so results are identical run to run.
 #include <algorithm>
 
 #include "qs_common.h"
@@ -52,6 +52,7 @@ struct AttnArgs {
     int *cnt;                           // [B, NKV] arrival counters of the in-launch merge (kept zero)
     int *status;                        // nullable: QS_STATUS_* bits of invalid lengths / table entries
     int B, T, NQ, NKV, max_blocks, num_blocks, pps, nsplit;
+    int merge;                          // the splits are merged inside the attention launch
     float scale;
     // mixer edges (qs_attn_mixer_decode; null / 0 for plain attention): q and the new k rows are
     // RMS-normalised times wq / wk [HD] and rotated on their first rot dims with rcos / rsin
@@ -223,20 +224,21 @@ typedef short i16x4_t __attribute__((ext_vector_type(4)));
 constexpr int QPAD = HD + 8;   // s_q row pitch (bf16): 16-byte skew between rows
 constexpr int VPAD = HD + 16;  // K / V slice row pitch (bf16): 32-byte skew between rows
 
-// Split merge inside the attention launch (nsplit <= MERGE_MAX, at most MERGE_ROWS query rows per KV head). Every workgroup of (user b, KV head g) has
+// Split merge inside the attention launch (AttnArgs::merge). Every workgroup of (user b, KV head g) has
 // stored its partial with agent-coherent stores (sc1: written through the XCD's L2); each thread waits for
 // its stores to complete, then one thread counts the workgroup in (the count wraps to zero at the last
 // arrival). The workgroup that completes the count merges: wave w of NWV takes query rows w, w + NWV, ...
-// (two at a time), lane l owns head dims 4 l .. 4 l + 3, and every split's partial and (m, l) are read with agent-coherent loads in one round
-// trip. Global max M (log2 domain) and sum L over the splits, weights 2^(m_s - M), O = sum_s w_s O_s / L in
-// split order, so the result does not depend on which workgroup finished last. No L2-wide writeback or
+// (two at a time), lane l owns head dims 4 l .. 4 l + 3, and every split's partial and (m, l) are read with agent-coherent
+// loads in one round trip. Global max M (log2 domain) and sum L over the splits, weights 2^(m_s - M), O = sum_s w_s O_s / L
+// in split order, so the result does not depend on which workgroup finished last. No L2-wide writeback or
 // invalidate is needed because only sc1 accesses touch the shared data. (The leader side of the
 // reference: kernels/attn_leader_writer.cpp:86-106, kernels/attn_leader_compute.cpp:42-79.)
-constexpr int MERGE_MAX = 16;
-// Steps of more query rows leave the merge to its own launch: one workgroup would read their partials in several round
-// trips (per layer, batch 1 / 3 tokens at 100 positions, 2 splits: 14.8 us in its own launch, 16.5 in the same; batch
-// 1 / 4 tokens at 1000, 16 splits: 15.2 and 21.3).
-constexpr int MERGE_ROWS = 16;
+// Up to 4 splits, or 8 where 2 rows per wave cover the user's query rows, are merged there; more, and every verify step
+// of the rows kernel, in a launch of their own. Per layer, in the launch against in its own: one token (6 rows), a page
+// per workgroup (4 waves), 2 / 4 / 8 / 16 splits at batch 1 8.8, 9.0, 9.5, 10.3 against 9.7, 9.7, 10.0, 10.0 us and at
+// batch 4 9.2, 9.4, 10.5, 12.8 against 10.2, 10.1, 10.3, 10.6; two tokens (12 rows) at batch 1 9.8, 10.1, 10.8, 12.3
+// against 9.9, 9.9, 10.0, 10.0 and 4 splits at batch 8 10.5 against 10.9; two pages (8 waves), 8 splits 11.2 against 11.2.
+constexpr int MERGE_MAX = 8, MERGE_ANY = 4;
 template <int NWV>
 __device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b, int g, int tid) {
     __shared__ int s_last;
@@ -1197,7 +1199,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(Mr), __float_as_uint(Lr)}, rpm, tid * 8, 0,
                                               qs::CP_SC1);
     }
-    if (a.nsplit > 1 && a.nsplit <= MERGE_MAX) merge_in_launch<NWV>(a, G, b, g, tid);
+    if (a.merge) merge_in_launch<NWV>(a, G, b, g, tid);
 }
 
 // Merge of the splits of one output row (user, token, query head) in one memory round trip: wave w sums
@@ -1348,6 +1350,7 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
         ns = nsplit_of(max_blocks, pages_per_split);
     }
     a.nsplit = ns;
+    a.merge = ns > 1 && T * G <= 16 && (ns <= MERGE_ANY || (ns <= MERGE_MAX && T * G <= 8 * attn_wpp(pages_per_split)));
     if (workspace) {
         const WsLayout L = ws_layout(B, T, NKV, G, ns);
         char *ws = static_cast<char *>(workspace);
@@ -1397,7 +1400,7 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
 #undef QS_ROWS
     }
     if (int e = qs::launch_status(who)) return e;
-    if (ns > 1 && (ns > MERGE_MAX || R > MERGE_ROWS)) {  // the rest are merged inside the attention launch
+    if (ns > 1 && !a.merge) {
         if (ns <= 64)
             attn_merge_kernel<1><<<B * T * NKV * G, 256, 0, st>>>(a, G);
         else
