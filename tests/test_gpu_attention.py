@@ -12,10 +12,22 @@ pytestmark = pytest.mark.gpu
 CNT_BYTES = 65536  # the fixed counter block at the head of an attention workspace
 
 
-def plan(B, T, G, width, pps, nkv=4):
+def pairs(T, G, mixer):
+    """Whether a verify step (more than 16 query rows per KV head) can walk two pages at once."""
+    R = T * G
+    nrb = -(-R // 64)
+    tiles = -(-R // (16 * nrb))
+    return not mixer or tiles == 2 or (tiles == 3 and T <= 8)
+
+
+def plan(B, T, G, width, pps, mixer=False, nkv=4):
     """How a call with a workspace is cut (the rules of the library's launch): pages a workgroup walks, splits, and
     whether the attention launch merges them itself. The tests below choose their shapes by it."""
     R = T * G
+    few = B * nkv <= 16
+    whole = (3 if few and not mixer else 2) if R <= 8 else (4 if few else 3) if R <= 16 else 2 if pairs(T, G, mixer) else 1
+    if width <= min(whole, pps):
+        return width, 1, False
     most = 256 // (B * nkv * -(-R // 64))
     p = -(-width // most) if most else pps
     p = min(pps, p if p <= 1 or not most else p + p % 2)
@@ -209,28 +221,42 @@ def test_in_launch_merge_counters_rearm(dev):
 
 
 # Where the merge moves between the launches: 4 and 5 splits of 12 rows and 8 and 9 of 6 on one page per workgroup, 8 and
-# 9 of 12 rows on two pages, 2 splits of 16 rows (group size 8) and of 18. The partials written show the split count.
+# 9 of 12 rows on two pages, 2 splits of 16 rows (group size 8) and of 18; and where a table stays whole: 2 and 3 pages of
+# 6 rows at batch 4, 2 but not 3 at batch 5, 4 but not 5 of 12 rows at batch 4, 3 but not 4 at batch 5, 2 but not 3 of 24.
+# The partials written show the split count.
 @pytest.mark.parametrize("B,G,T,width,pps,splits,merged", [
     (6, 6, 2, 4, 2, 4, True), (2, 6, 2, 5, 2, 5, False), (2, 6, 1, 8, 8, 8, True), (2, 6, 1, 9, 8, 9, False),
     (8, 6, 2, 16, 2, 8, True), (7, 6, 2, 18, 8, 9, False), (64, 8, 2, 5, 4, 2, True), (64, 6, 3, 5, 4, 2, False),
+    (4, 6, 1, 1, 8, 1, False), (4, 6, 1, 2, 2, 1, False), (4, 6, 1, 3, 8, 1, False), (4, 6, 1, 3, 2, 3, True),
+    (5, 6, 1, 2, 8, 1, False), (5, 6, 1, 3, 8, 3, True), (4, 6, 2, 4, 8, 1, False), (4, 6, 2, 5, 8, 5, False),
+    (5, 6, 2, 3, 8, 1, False), (5, 6, 2, 4, 8, 4, True), (1, 6, 4, 2, 8, 1, False), (1, 6, 4, 3, 8, 3, False),
+    (1, 6, 8, 2, 8, 1, False), (1, 6, 11, 2, 8, 1, False), (1, 6, 11, 3, 8, 3, False),
 ])  # fmt: skip
-def test_merge_split_counts(dev, B, G, T, width, pps, splits, merged):
-    assert plan(B, T, G, width, pps)[1:] == (splits, merged)
+@pytest.mark.parametrize("mixer", [False, True])
+def test_split_plans(dev, B, G, T, width, pps, splits, merged, mixer):
+    if mixer and (B, T, width, pps) == (4, 1, 3, 8):
+        splits, merged = 3, True  # the mixer's launch keeps 2 pages whole, not 3
+    if mixer and (T, width) == (11, 2):
+        splits = 2  # and of 11 tokens, whose rows it walks a page at a time, none
+    assert plan(B, T, G, width, pps, mixer)[1:] == (splits, merged)
     d = W.attn_layer(B, width * 64, "cpu", seed=B + T + width, T=T, num_blocks=B * width + 8)
     gen = torch.Generator().manual_seed(width)
     d["q"] = torch.randn(B, T, G * 4, 256, generator=gen).bfloat16()
     d["seq_lens"] = torch.randint((width - 1) * 64 + T, width * 64 + 1, (B,), generator=gen).to(torch.int32)
-    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
     ws = torch.zeros(ops.lib().qs_paged_attention_workspace_bytes(B, T, G * 4, 4, 256, width, pps), dtype=torch.uint8,
                      device=dev)  # fmt: skip
     ws[CNT_BYTES:] = 0xFF
-    o = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"],
-                             k_new=g["k_new"], v_new=g["v_new"], pages_per_split=pps, ws=ws)  # fmt: skip
-    assert split_rows(ws) == B * 4 * splits * T * G
+    if mixer:
+        check_mixer(dev, d, pps, 64, gen, ws=ws)
+    else:
+        g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+        o = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"],
+                                 k_new=g["k_new"], v_new=g["v_new"], pages_per_split=pps, ws=ws)  # fmt: skip
+        kc, vc = d["k_cache"].clone(), d["v_cache"].clone()
+        O.paged_append(kc, vc, d["k_new"], d["v_new"], d["block_table"], d["seq_lens"] - T)
+        assert_attn_output(o, O.bf16(O.gqa_decode(d["q"], kc, vc, d["block_table"], d["seq_lens"], d["scale"])))
+    assert split_rows(ws) == (B * 4 * splits * T * G if splits > 1 else 0)
     assert int(ws[:CNT_BYTES].view(torch.int32).abs().sum()) == 0, "counters not re-armed"
-    kc, vc = d["k_cache"].clone(), d["v_cache"].clone()
-    O.paged_append(kc, vc, d["k_new"], d["v_new"], d["block_table"], d["seq_lens"] - T)
-    assert_attn_output(o, O.bf16(O.gqa_decode(d["q"], kc, vc, d["block_table"], d["seq_lens"], d["scale"])))
 
 
 # More splits go through the separate merge launch (one workgroup per output row, the partials merged in
@@ -335,7 +361,7 @@ def test_verify_row_blocks(dev, G, T, lens, pps, mixer):
     check_mixer(dev, d, pps, 64, gen)
 
 
-def check_mixer(dev, d, pps, rot, gen):
+def check_mixer(dev, d, pps, rot, gen, ws=None):
     """The mixer's call against the oracle: appended K rows within one bf16 ulp, V rows bit-exact, the output."""
     from conftest import bf16_ulp_mismatch
 
@@ -347,7 +373,7 @@ def check_mixer(dev, d, pps, rot, gen):
     g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
     tab = [t.to(dev) if rot else None for t in (cos, sin)]
     o = ops.attn_mixer_decode(g["q"], g["k_new"], g["v_new"], gate.to(dev), wq.to(dev), wk.to(dev), *tab, g["k_cache"],
-                              g["v_cache"], g["block_table"], g["seq_lens"], pages_per_split=pps, rot=rot)  # fmt: skip
+                              g["v_cache"], g["block_table"], g["seq_lens"], pages_per_split=pps, rot=rot, ws=ws)  # fmt: skip
     kc, vc = d["k_cache"].clone(), d["v_cache"].clone()
     if not rot:
         cos, sin = torch.ones(*d["q"].shape[:2], 8), torch.zeros(*d["q"].shape[:2], 8)  # the identity rotation
@@ -397,18 +423,18 @@ def test_verify_row_blocks_idle_and_bad_page(dev):
 
 
 # A step of 3 or more tokens with at most 16 query rows per KV head stores its new rows first and reads the pages they
-# lie in again. A grid of at most 256 workgroups walks one page each whatever the caller asks for (2 users x 4 KV heads
+# lie in again. A grid of at most 256 workgroups walks one page each though the caller allows two (2 users x 4 KV heads
 # x 4 pages), where K is read in the score operand's layout; 66 users x 4 KV heads are past that and walk the caller's
 # two pages at a time. The new rows cross a page, end one, fill a user's cache or start it.
 @pytest.mark.parametrize("G,T", [(4, 3), (4, 4), (2, 3), (2, 8), (1, 3), (1, 16)])
-@pytest.mark.parametrize("B,pps", [(2, 1), (2, 8), (66, 2)])
+@pytest.mark.parametrize("B,pps", [(2, 1), (2, 2), (66, 2)])
 @pytest.mark.parametrize("mixer", [False, True])
 def test_few_rows_append(dev, G, T, B, pps, mixer):
     gen = torch.Generator().manual_seed(G * 100 + T + B)
     d = W.attn_layer(B, 256, "cpu", seed=G * 100 + T + pps, T=T, num_blocks=B * 4 + 8)
     d["q"] = torch.randn(B, T, G * 4, 256, generator=gen).bfloat16()
     d["seq_lens"] = torch.tensor(([130, 256] + [T, 64, 65, 192] * 16)[:B], dtype=torch.int32)
-    assert d["block_table"].shape[1] == 4
+    assert plan(B, T, G, 4, pps, mixer)[0] == (2 if B == 66 else 1)
     if mixer:
         return check_mixer(dev, d, pps, 64, gen)
     o1, ref, same1 = run_case(dev, d, pps, fused=True)

@@ -1294,6 +1294,15 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
     *reinterpret_cast<uint2 *>(a.o + oi) = make_uint2(qs::cvt_pk_bf16(o0, o1), qs::cvt_pk_bf16(o2, o3));
 }
 
+// The rows kernel's query tiles per block for R rows: the fewest that cover them in as few blocks as 4 tiles would.
+int rows_tiles(int R) {
+    const int nrb = (R + 63) / 64;
+    return (R + 16 * nrb - 1) / (16 * nrb);
+}
+// Whether its LDS holds two page groups: the mixer's residues leave no room for the second with 3 tiles and more than 8
+// new tokens, or with 4 tiles.
+bool rows_pairs(int R, int T, bool mixer) { return !mixer || rows_tiles(R) == 2 || (rows_tiles(R) == 3 && T <= 8); }
+
 int nsplit_of(int max_blocks, int pps) { return (max_blocks + pps - 1) / pps; }
 // Pages a workgroup walks: the caller's, or as few as keep the whole launch within one workgroup per CU (an even number
 // past one, for the two pages in flight). A page takes its waves ~2 us of dependent latency (load, scores, softmax,
@@ -1303,9 +1312,19 @@ int nsplit_of(int max_blocks, int pps) { return (max_blocks + pps - 1) / pps; }
 // 1000: 19.3 -> 13.7; batch 1 / 4 tokens, 8 pages, 1000: 29.5 -> 15.2. One step finer than the rule: batch 1 / 8192
 // 18.6 against 16.1, batch 4 / 4096 26.4 against 20.4, batch 8 / 2048 27.7 against 18.6. Only sizes known to the host
 // enter the rule, so a user's result depends on no other user's length.
+// A table of few pages stays whole (if the caller's pages allow it): two pages are walked at once, and without a second
+// split there is no merge. One split against a page per split: one token, batch 1, 2 / 3 / 4 pages 7.8, 8.7, 9.5 against
+// 8.8, 8.9, 8.8 us, 3 pages at batch 8 9.8 against 9.4, with the mixer 10.6 against 10.4; two tokens, batch 1, 2 / 3 / 4
+// pages 7.9, 8.9, 9.7 against 9.8, 9.9, 10.0, 4 pages at batch 8 10.9 against 10.5; four tokens (rows kernel) 2 / 3 pages
+// 9.7, 12.0 against 11.2, 11.2; where the rows kernel walks one page at a time (rows_pairs), 11 tokens with the mixer, 2
+// pages 20.8 against 18.4.
 constexpr int FINE_WGS = 256;
-int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps) {
-    const int nrb = (T * G + 63) / 64;  // row blocks of attn_rows_kernel (1 in attn_wave_kernel)
+int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps, bool mixer) {
+    const int R = T * G;
+    const bool few = B * NKV <= 16;
+    const int whole = R <= 8 ? (few && !mixer ? 3 : 2) : R <= 16 ? (few ? 4 : 3) : rows_pairs(R, T, mixer) ? 2 : 1;
+    if (max_blocks <= std::min(whole, pps)) return max_blocks;
+    const int nrb = (R + 63) / 64;  // row blocks of attn_rows_kernel (1 in attn_wave_kernel)
     const long most = FINE_WGS / ((long)B * NKV * nrb);  // splits per user and KV head
     if (most == 0) return pps;
     const int p = (int)((max_blocks + most - 1) / most);
@@ -1320,9 +1339,9 @@ int attn_wpp(int pps) { return pps >= 2 ? 2 : 1; }
 extern "C" size_t qs_paged_attention_workspace_bytes(int B, int T, int NQ, int NKV, int HDa, int max_blocks,
                                                      int pages_per_split) {
     if (B <= 0 || T <= 0 || NKV <= 0 || NQ % NKV || HDa != HD || max_blocks <= 0 || pages_per_split <= 0) return 0;
-    const int G = NQ / NKV, ns = nsplit_of(max_blocks, walk_pages(B, T, NKV, G, max_blocks, pages_per_split));
-    // at least FINE_WGS partials, which no smaller call of the same T exceeds (a smaller batch or a narrower table is
-    // cut finer): a workspace sized for the largest call serves them all
+    const int G = NQ / NKV, ns = nsplit_of(max_blocks, walk_pages(B, T, NKV, G, max_blocks, pages_per_split, false));
+    // at least FINE_WGS partials, which no smaller call of the same T exceeds (a smaller batch, a narrower table or the
+    // mixer's call may be cut finer): a workspace sized for the largest call serves them all
     return ws_layout(std::max(B * NKV * ns, FINE_WGS), T, 1, G, 1).total;
 }
 
@@ -1346,7 +1365,7 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
     QS_REQUIRE((size_t)B * NKV * sizeof(int) <= CNT_BYTES, "%s: B NKV = %d exceeds %d", who, B * NKV,
                (int)(CNT_BYTES / sizeof(int)));
     if (workspace) {
-        pages_per_split = a.pps = walk_pages(B, T, NKV, G, max_blocks, pages_per_split);
+        pages_per_split = a.pps = walk_pages(B, T, NKV, G, max_blocks, pages_per_split, a.wq);
         ns = nsplit_of(max_blocks, pages_per_split);
     }
     a.nsplit = ns;
@@ -1381,16 +1400,14 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
         }
 #undef QS_WAVE
     } else {
-        // query rows in blocks of 16 QT, QT the fewest tiles that cover them in as few blocks as 4 tiles would
-        const int nrb = (R + 63) / 64, QT = (R + 16 * nrb - 1) / (16 * nrb);
+        const int nrb = (R + 63) / 64, QT = rows_tiles(R);  // query rows in blocks of 16 QT
         QS_REQUIRE((long)grid.x * nrb < (1L << 31), "%s: grid too large", who);
         const dim3 rgrid(grid.x * nrb);
-        const bool two = pages_per_split >= 2;
-        // the new rows of more than 8 tokens leave no LDS for the second group of 3 tiles with the mixer's residues
+        const bool two = pages_per_split >= 2 && rows_pairs(R, T, a.wq);
 #define QS_ROWS(Q, MX, W) attn_rows_kernel<Q, MX, W><<<rgrid, 256 * W, 0, st>>>(a, G, nrb)
-        if (a.wq) {  // with 4 tiles and the mixer's residues LDS has room for one page group only
+        if (a.wq) {
             if (QT == 2) { if (two) QS_ROWS(2, true, 2); else QS_ROWS(2, true, 1); }
-            else if (QT == 3) { if (two && T <= 8) QS_ROWS(3, true, 2); else QS_ROWS(3, true, 1); }
+            else if (QT == 3) { if (two) QS_ROWS(3, true, 2); else QS_ROWS(3, true, 1); }
             else QS_ROWS(4, true, 1);
         } else {
             if (QT == 2) { if (two) QS_ROWS(2, false, 2); else QS_ROWS(2, false, 1); }
