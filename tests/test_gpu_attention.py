@@ -442,3 +442,23 @@ def test_few_rows_append(dev, G, T, B, pps, mixer):
     assert same1 and same2
     assert torch.equal(o1.cpu(), o2.cpu())
     assert_attn_output(o1, ref)
+
+
+# The rows kernel's forms for up to 8 new tokens and for up to 16, 2, 3 and 4 query tiles each side of 8: 32 and 18 rows,
+# 48 and 36, 64 and 54 (the longest call of 8 tokens, the shortest past it). A table of 5 pages is walked a page per
+# workgroup, one of 2 pages whole (both at once where there is room); new rows fill a user's cache, cross a page, end one.
+@pytest.mark.parametrize("G,T", [(4, 8), (2, 9), (6, 8), (4, 9), (8, 8), (6, 9)])
+@pytest.mark.parametrize("width", [5, 2])
+@pytest.mark.parametrize("mixer", [False, True])
+def test_verify_token_forms(dev, G, T, width, mixer):
+    lens = [T, 64 + T // 2, width * 64]
+    assert plan(3, T, G, width, 8, mixer)[0] == (2 if width == 2 and pairs(T, G, mixer) else 1)
+    d = W.attn_layer(3, width * 64, "cpu", seed=G + T, T=T, num_blocks=32)
+    gen = torch.Generator().manual_seed(G + T)
+    d["q"] = torch.randn(3, T, G * 4, 256, generator=gen).bfloat16()
+    d["seq_lens"] = torch.tensor(lens, dtype=torch.int32)
+    if mixer:
+        return check_mixer(dev, d, 8, 64, gen)
+    o, ref, same = run_case(dev, d, 8)
+    assert same
+    assert_attn_output(o, ref)
