@@ -462,3 +462,35 @@ def test_verify_token_forms(dev, G, T, width, mixer):
     o, ref, same = run_case(dev, d, 8)
     assert same
     assert_attn_output(o, ref)
+
+
+# A table wider than its users: the splits past a user's pages write no partial, and the merges read none of theirs (the
+# workspace holds NaNs); table entries past a user's pages are not looked at. Merged in the launch (4 and 8 splits) and in
+# one of their own (16 to 24, and 65, past one load of every split's maximum); users of one page, of all, idle.
+@pytest.mark.parametrize("B,T,width,pps,merged", [(16, 1, 16, 4, True), (8, 2, 16, 2, True), (3, 1, 128, 8, False),
+                                                  (5, 2, 24, 1, False), (4, 4, 64, 8, False), (3, 8, 130, 2, False),
+                                                  (3, 11, 40, 2, False)])  # fmt: skip
+@pytest.mark.parametrize("mixer", [False, True])
+def test_wide_tables(dev, B, T, width, pps, merged, mixer):
+    assert plan(B, T, 6, width, pps, mixer)[2] == merged
+    d = W.attn_layer(B, width * 64, "cpu", seed=B + T + width, T=T, num_blocks=B * width + 8)
+    idle = 0 if not mixer else T  # the oracle's mixer has no idle users
+    d["seq_lens"] = torch.tensor(([T, width * 64, idle, 65, 64] + [128 + T] * B)[:B], dtype=torch.int32)
+    for b in range(B):
+        d["block_table"][b, -(-int(d["seq_lens"][b]) // 64) :] = -1
+    ws = torch.zeros(ops.lib().qs_paged_attention_workspace_bytes(B, T, 24, 4, 256, width, pps), dtype=torch.uint8,
+                     device=dev)  # fmt: skip
+    ws[CNT_BYTES:] = 0xFF
+    if mixer:
+        check_mixer(dev, d, pps, 64, torch.Generator().manual_seed(width), ws=ws)
+    else:
+        g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+        st = ops.Status(dev)
+        o = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"],
+                                 pages_per_split=pps, ws=ws, status=st.word)  # fmt: skip
+        assert st.peek() == 0
+        live = [b for b in range(B) if b != 2]
+        ref = O.gqa_decode(d["q"][live], d["k_cache"], d["v_cache"], d["block_table"][live], d["seq_lens"][live], d["scale"])
+        assert_attn_output(o[live], O.bf16(ref))
+        assert int(o[2].count_nonzero()) == 0
+    assert int(ws[:CNT_BYTES].view(torch.int32).abs().sum()) == 0, "counters not re-armed"

@@ -152,6 +152,18 @@ __device__ __forceinline__ bool user_active(const AttnArgs &a, int n, bool repor
     }
     return n >= a.T;
 }
+// Whether split sp of a user of length n holds pages. A table is as wide as its longest user may get: a shorter user's
+// other splits have nothing to do. Their workgroups request no page, write no partial and leave, and the merges count and
+// read only those that hold pages. At 8 pages a split and a 512-page table, with every split requesting its first pages,
+// storing partials and being merged -> this: 200 positions, batch 8, one token 66.2 -> 22.6 us a layer, four 84.4 -> 34.8,
+// batch 1, one token 16.3 -> 13.2; 64-page table, batch 4 at 200, one token 16.1 -> 13.5.
+__device__ __forceinline__ bool split_live(const AttnArgs &a, int n, int sp) { return sp * a.pps * BLK < n; }
+// How many do (whole waves; FEW: at most 64 splits, counted without a division)
+template <bool FEW>
+__device__ __forceinline__ int live_splits(const AttnArgs &a, int n, int lane) {
+    if constexpr (FEW) return __builtin_popcountll(__ballot(lane < a.nsplit && split_live(a, n, lane)));
+    return ((n + BLK - 1) / BLK + a.pps - 1) / a.pps;
+}
 __device__ __forceinline__ void report_page(const AttnArgs &a) {
     if (a.status) atomicOr(a.status, QS_STATUS_PAGE);
 }
@@ -188,7 +200,7 @@ __device__ __forceinline__ size_t prow(const AttnArgs &a, int G, int b, int g, i
 
 // The MFMA kernels' first requests, each one buffer load with no branch around it (lanes outside the range
 // read zeros without a memory access), so the compiler's waits stay exact: the first page's loads, issued
-// next, need only the block-table entries, and nothing waits for the query rows until they are staged.
+// next, need only the block-table entries and the user's length, and nothing waits for the query rows until they are staged.
 // Block-table entry p0 + lane of user b (zero past the split or the table; only entries below
 // min(max_blocks, p0 + pps) are ever read back).
 __device__ __forceinline__ int split_entries(const AttnArgs &a, int b, int p0, int lane) {
@@ -240,21 +252,23 @@ constexpr int VPAD = HD + 16;  // K / V slice row pitch (bf16): 32-byte skew bet
 // against 9.9, 9.9, 10.0, 10.0 and 4 splits at batch 8 10.5 against 10.9; two pages (8 waves), 8 splits 11.2 against 11.2.
 constexpr int MERGE_MAX = 8, MERGE_ANY = 4;
 template <int NWV>
-__device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b, int g, int tid) {
+__device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b, int g, int tid, int n) {
     __shared__ int s_last;
+    const int ns = live_splits<true>(a, n, tid & 63);
     qs::wait_vmem();
     __syncthreads();
     if (tid == 0) {
-        // an increment modulo the splits: the last arrival leaves the count at zero for the next launch
+        // an increment modulo the splits that arrive (those holding pages): the last one leaves the count at zero for
+        // the next launch
         unsigned *c = reinterpret_cast<unsigned *>(a.cnt) + (size_t)b * a.NKV + g;
-        const unsigned ns1 = (unsigned)a.nsplit - 1;
+        const unsigned ns1 = (unsigned)ns - 1;
         s_last = __builtin_amdgcn_atomic_inc32(c, ns1, __ATOMIC_RELAXED, "agent") == ns1;
     }
     __syncthreads();
     if (!s_last) return;
     asm volatile("" ::: "memory");
     const int lane = tid & 63, w = tid >> 6;
-    const int T = a.T, R = T * G, ns = a.nsplit;
+    const int T = a.T, R = T * G;
     const auto ro = __builtin_amdgcn_make_buffer_rsrc(qs::uniform_ptr(a.part_o + prow(a, G, b, g, 0, 0) * HD),
                                                       (short)0, ns * R * HD * 4, 0x00020000);
     const auto rm = __builtin_amdgcn_make_buffer_rsrc(qs::uniform_ptr(a.part_ml + prow(a, G, b, g, 0, 0) * 2),
@@ -373,7 +387,7 @@ __global__ __launch_bounds__(256 * WPP, 2) void attn_rows_kernel(AttnArgs a, int
     auto s_o = reinterpret_cast<f32x4_t *>(s_raw + S::Q + S::QL);
 
     // Issued first, in this order: the split's block-table entries, the user's length, the query rows and the
-    // new rows. The first page's K / V loads then wait only for the table entries, not for the length.
+    // new rows. The first page's K / V loads then wait only for the table entries and the length.
     const int p0 = split * a.pps;
     const int bt_pre = split_entries(a, b, p0, lane);
     const int n = a.seq_lens[b];
@@ -430,11 +444,10 @@ __global__ __launch_bounds__(256 * WPP, 2) void attn_rows_kernel(AttnArgs a, int
         for (int k = 0; k < 8; ++k) vb[k] = __builtin_amdgcn_raw_buffer_load_b128(rv, off, k * 1024, NT);
     };
 
-    // the group's first page, before the length is known: a page in the pool's range that turns out to lie past
-    // the user's length is simply not used
+    // the group's first page, if the user's length reaches it (the length was requested with the table's entries)
     u32x4 kb[8], vb[8];
     const int pf = p0 + ph;
-    const int pg0 = pf < min(a.max_blocks, p0 + a.pps) ? page_at(pf) : -1;
+    const int pg0 = pf < min(a.max_blocks, p0 + a.pps) && pf * BLK < n ? page_at(pf) : -1;
     load_k(pg0, kb);
     load_v(pg0, vb);
 
@@ -442,6 +455,7 @@ __global__ __launch_bounds__(256 * WPP, 2) void attn_rows_kernel(AttnArgs a, int
         if (split == 0 && rb == 0) zero_rows(a, G, b, g, tid, NTH);
         return;
     }
+    if (!split_live(a, n, split)) return;
     const int base = n - T;  // first new position
     const int p1 = min((n + BLK - 1) / BLK, p0 + a.pps);
     // an entry of the split's pages outside the pool (lane pi - p0 checks entry pi) is reported after the
@@ -857,8 +871,8 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         }
     };
     uint4 KA[8], VA[8];
-    const int pf = p0 + ph;  // this wave's first page
-    const int pg0 = pf < min(a.max_blocks, p0 + a.pps) ? page_at(pf) : -1;
+    const int pf = p0 + ph;  // this wave's first page, if the user's length reaches it
+    const int pg0 = pf < min(a.max_blocks, p0 + a.pps) && pf * BLK < n ? page_at(pf) : -1;
     if constexpr (WPP == 1)
         load_kfrag(pg0, KA);
     else
@@ -869,6 +883,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         if (split == 0) zero_rows(a, G, b, g, tid, NTH);
         return;
     }
+    if (!split_live(a, n, split)) return;
     const int base = n - T;
     const int npages = (n + BLK - 1) / BLK;
     const int p1 = min(npages, p0 + a.pps);
@@ -1198,7 +1213,7 @@ __global__ __launch_bounds__(256 * WPP, WPP == 1 ? 2 : 1) void attn_wave_kernel(
         __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(Mr), __float_as_uint(Lr)}, rpm, tid * 8, 0,
                                               qs::CP_SC1);
     }
-    if (a.merge) merge_in_launch<NWV>(a, G, b, g, tid);
+    if (a.merge) merge_in_launch<NWV>(a, G, b, g, tid, n);
 }
 
 // Merge of the splits of one output row (user, token, query head) in one memory round trip: wave w sums
@@ -1219,7 +1234,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
     const int g = row % a.NKV, bt = row / a.NKV;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ns = a.nsplit, R = a.T * G;
-    const int n = a.seq_lens[bt / a.T];
+    const int n = a.seq_lens[bt / a.T], live = live_splits<MLR == 1>(a, n, lane);
     // The row's partials are requested before the length is checked: their addresses do not depend on it and
     // lie in the workspace either way, so the launch waits for one round trip, not two. Buffer loads, with a
     // wave's split offset in a scalar register and the lane's 16 bytes as the vector offset, need no per-load
@@ -1245,7 +1260,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
 #pragma unroll
     for (int j = 0; j < MLR; ++j) {
         const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(rml, (lane + 64 * j) * R * 8, 0, 0);
-        mg[j] = lane + 64 * j < ns ? make_float2(__uint_as_float(u[0]), __uint_as_float(u[1]))
+        mg[j] = lane + 64 * j < live ? make_float2(__uint_as_float(u[0]), __uint_as_float(u[1]))
                                    : make_float2(-INFINITY, 0.f);
         M = fmaxf(M, mg[j].x);
     }
@@ -1262,7 +1277,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
     L = qs::wave_sum_dpp(L);
     float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
     auto acc = [&](int sp, const float4 &v, float m) {
-        if (sp < ns && m != -INFINITY) {
+        if (sp < live && m != -INFINITY) {
             const float e = __builtin_amdgcn_exp2f(m - M);
             O.x += e * v.x, O.y += e * v.y, O.z += e * v.z, O.w += e * v.w;
         }
@@ -1270,7 +1285,7 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a, int G) {
 #pragma unroll
     for (int k = 0; k < MCH; ++k) acc(w + 4 * k, x[k], MLR > 1 ? mw[k] : qs::lane_val(mg[0].x, w + 4 * k));
     if constexpr (MLR > 1) {
-        for (int s0 = 4 * MCH; s0 < ns; s0 += 4 * MCH) {  // further splits, a batch of loads at a time
+        for (int s0 = 4 * MCH; s0 < live; s0 += 4 * MCH) {  // further splits, a batch of loads at a time
 #pragma unroll
             for (int k = 0; k < MCH; ++k) load_split(min(s0 + w + 4 * k, ns - 1), x[k], mw[k]);
 #pragma unroll
