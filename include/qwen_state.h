@@ -217,11 +217,16 @@ int qs_paged_kv_gather(const uint16_t *k_cache, const uint16_t *v_cache, const i
  *   q [B, T, NQ, HD] bf16; seq_lens [B] = positions valid after this step's T tokens; query t of user b
  *   attends positions 0 .. seq_lens[b] - T + t (causal among the T new rows); o [B, T, NQ, HD] bf16.
  *   When k_new/v_new [B, T, NKV, HD] are non-null the T new rows are also appended (a5 fused): the
- *   workgroup owning a new row's page writes it first and waits for the store, then reads it back with the
- *   page, so no call sees a half-written row.
- *   pages_per_split (1..64): most pages one workgroup walks (the split-K grain); with a workspace, a launch that would
- *   leave CUs idle walks fewer. The workspace holds the partials; one sized for B users, a table of max_blocks and T
- *   tokens serves calls of fewer of each.
+ *   workgroup owning a new row's page attends it without reading the pool and stores it after its pages (3 and
+ *   more tokens of at most 16 query rows per KV head: stores it first, waits, and reads it back with the page),
+ *   so no call sees a half-written row.
+ *   pages_per_split (1..64): pages one workgroup walks (the split-K grain); the workspace holds the partials (one split,
+ *   ceil(max_blocks / pages_per_split) == 1, needs none and leaves it alone).
+ *   qs_paged_attention_walk_pages: the grain, at most the caller's, with which a call of these sizes is fastest: fewer
+ *   pages where the launch would leave CUs idle (mixer: 1 for qs_attn_mixer_decode). A workspace of
+ *   qs_paged_attention_workspace_bytes at the caller's pages_per_split holds that grain's partials too, and one sized for
+ *   B users, a table of max_blocks and T tokens serves calls of fewer of each. The grain decides how the sums are grouped,
+ *   so a user's output bits follow it, and through it the batch size and the table's width, not other users' lengths.
  *   A user with seq_lens[b] < T is an idle slot: nothing is appended or attended and its output rows are
  *   zero. A user with seq_lens[b] > max_blocks * block is treated the same and reported (QS_STATUS_LENGTH);
  *   a page entry outside [0, num_blocks) is not attended and is reported (QS_STATUS_PAGE).
@@ -230,6 +235,7 @@ int qs_paged_kv_gather(const uint16_t *k_cache, const uint16_t *v_cache, const i
  * kernels/attn_common.hpp:139-154; torch model.py:239-246). HD == 256, block == 64, NQ / NKV <= 8. */
 size_t qs_paged_attention_workspace_bytes(int B, int T, int NQ, int NKV, int HD, int max_blocks,
                                           int pages_per_split);
+int qs_paged_attention_walk_pages(int B, int T, int NQ, int NKV, int max_blocks, int pages_per_split, int mixer);
 int qs_paged_gqa_decode(const uint16_t *q, const uint16_t *k_new, const uint16_t *v_new, uint16_t *k_cache,
                         uint16_t *v_cache, const int *block_table, const int *seq_lens, uint16_t *o,
                         void *workspace, int B, int T, int NQ, int NKV, int HD, int block, int max_blocks,

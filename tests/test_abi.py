@@ -98,6 +98,25 @@ def test_attention_workspace_serves_smaller_calls():
                                for b in (1, B // 2 + 1, B) for t in (1, T) for m in (1, mb // 3 + 1, mb) if b <= B and m <= mb)  # fmt: skip
 
 
+def test_attention_walk_pages():
+    """The grain suggested for a call: never more pages than the caller's, its partials fit a workspace sized at the
+    caller's grain (and so do the plain call's and the mixer's), and arguments the launch refuses come back as they are."""
+    L = Q.lib()
+    for pps in (1, 2, 8, 16, 64):
+        for T in (1, 2, 3, 4, 8, 11, 16):
+            for B in (1, 3, 8, 33, 70, 300):
+                for mb in (1, 2, 3, 4, 5, 7, 64, 500):
+                    rows = T * 6
+                    size = L.qs_paged_attention_workspace_bytes(B, T, 24, 4, 256, mb, pps)
+                    for mixer in (0, 1):
+                        walk = L.qs_paged_attention_walk_pages(B, T, 24, 4, mb, pps, mixer)
+                        assert 1 <= walk <= pps
+                        parts = B * 4 * -(-mb // walk) * rows
+                        assert 65536 + -(-parts * 8 // 256) * 256 + parts * 1024 <= size
+    for pps, mb, nq in ((0, 64, 24), (-3, 64, 24), (65, 64, 24), (1, 1025, 24), (8, 64, 23), (8, 0, 24)):
+        assert L.qs_paged_attention_walk_pages(1, 1, nq, 4, mb, pps, 0) == pps
+
+
 def test_ops_validate_before_calling():
     cpu = torch.zeros(1, 16, 128, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="GPU"):

@@ -494,3 +494,29 @@ def test_wide_tables(dev, B, T, width, pps, merged, mixer):
         assert_attn_output(o[live], O.bf16(ref))
         assert int(o[2].count_nonzero()) == 0
     assert int(ws[:CNT_BYTES].view(torch.int32).abs().sum()) == 0, "counters not re-armed"
+
+
+# A call that fits one split needs no workspace: the library writes nothing to one that is given (here full of 0xFF, where
+# counters would have to be zero), and the ops take one too small for finer splits as they take none.
+@pytest.mark.parametrize("T", [1, 4])
+def test_one_split_leaves_the_workspace(dev, T):
+    import ctypes
+
+    d = W.attn_layer(2, 4 * 64, "cpu", seed=T, T=T, num_blocks=16)
+    g = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in d.items()}
+    L = ops.lib()
+    nbytes = L.qs_paged_attention_workspace_bytes(2, T, 24, 4, 256, 4, 8)
+    ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=dev)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    o = torch.empty_like(g["q"])
+    assert L.qs_paged_gqa_decode(p(g["q"]), None, None, p(g["k_cache"]), p(g["v_cache"]), p(g["block_table"]),
+                                 p(g["seq_lens"]), p(o), p(ws), 2, T, 24, 4, 256, 64, 4, 16, 8, d["scale"], None,
+                                 torch.cuda.current_stream().cuda_stream) == 0  # fmt: skip
+    ref = O.bf16(O.gqa_decode(d["q"], d["k_cache"], d["v_cache"], d["block_table"], d["seq_lens"], d["scale"]))
+    assert_attn_output(o, ref)
+    assert int((ws != 0xFF).sum()) == 0
+    o2 = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"], ws=ws[:256])
+    none = ops.paged_gqa_decode(g["q"], g["k_cache"], g["v_cache"], g["block_table"], g["seq_lens"], d["scale"])
+    assert torch.equal(o2, o) and torch.equal(none, o)
+    check_mixer(dev, d, 8, 64, torch.Generator().manual_seed(T), ws=ws[:256])
+    assert int((ws != 0xFF).sum()) == 0

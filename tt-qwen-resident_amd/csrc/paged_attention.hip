@@ -1318,7 +1318,7 @@ int rows_tiles(int R) {
 bool rows_pairs(int R, int T, bool mixer) { return !mixer || rows_tiles(R) == 2 || (rows_tiles(R) == 3 && T <= 8); }
 
 int nsplit_of(int max_blocks, int pps) { return (max_blocks + pps - 1) / pps; }
-// Pages a workgroup walks: the caller's, or as few as keep the whole launch within one workgroup per CU (an even number
+// Pages a workgroup is best given to walk: the caller's, or as few as keep the whole launch within one workgroup per CU (an even number
 // past one, for the two pages in flight). A page takes its waves ~2 us of dependent latency (load, scores, softmax,
 // P V), so a grid that leaves CUs idle is cut finer; past 256 workgroups the partials cost more than the shorter walks
 // save. Per layer with the mixer, the caller's pages -> the rule's: batch 1, 8 pages: 200 positions 13.0 -> 11.4 us (4
@@ -1359,9 +1359,17 @@ extern "C" size_t qs_paged_attention_workspace_bytes(int B, int T, int NQ, int N
     return ws_layout(std::max(B * NKV * ns, FINE_WGS), T, 1, G, 1).total;
 }
 
+extern "C" int qs_paged_attention_walk_pages(int B, int T, int NQ, int NKV, int max_blocks, int pages_per_split,
+                                             int mixer) {
+    if (B <= 0 || T <= 0 || NKV <= 0 || NQ <= 0 || NQ % NKV || max_blocks <= 0 || pages_per_split <= 0 ||
+        pages_per_split > 64 || nsplit_of(max_blocks, pages_per_split) > MAX_SPLITS)
+        return pages_per_split;  // not a call that qs_paged_gqa_decode takes: it says so
+    return walk_pages(B, T, NKV, NQ / NKV, max_blocks, pages_per_split, mixer);
+}
+
 static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const char *who, void *stream) {
     const int B = a.B, T = a.T, NQ = a.NQ, NKV = a.NKV, max_blocks = a.max_blocks;
-    int pages_per_split = a.pps;
+    const int pages_per_split = a.pps;
     QS_REQUIRE(a.q && a.k_cache && a.v_cache && a.block_table && a.seq_lens && a.o, "%s: null pointer", who);
     QS_REQUIRE((a.k_new == nullptr) == (a.v_new == nullptr), "%s: give both k_new and v_new or neither", who);
     QS_REQUIRE(HDa == HD, "%s: HD must be %d (got %d)", who, HD, HDa);
@@ -1372,19 +1380,15 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
     QS_REQUIRE(pages_per_split > 0 && pages_per_split <= 64, "%s: pages_per_split must be in [1, 64] (got %d)", who,
                pages_per_split);
     const int G = NQ / NKV;
-    int ns = nsplit_of(max_blocks, pages_per_split);
+    const int ns = nsplit_of(max_blocks, pages_per_split);
     QS_REQUIRE(ns == 1 || workspace, "%s: %d splits need a workspace", who, ns);
     QS_REQUIRE(ns <= MAX_SPLITS, "%s: %d splits exceed %d (raise pages_per_split)", who, ns, MAX_SPLITS);
     QS_REQUIRE((long)B * NKV * ns < (1L << 31), "%s: grid too large", who);
     QS_REQUIRE((size_t)B * NKV * sizeof(int) <= CNT_BYTES, "%s: B NKV = %d exceeds %d", who, B * NKV,
                (int)(CNT_BYTES / sizeof(int)));
-    if (workspace) {
-        pages_per_split = a.pps = walk_pages(B, T, NKV, G, max_blocks, pages_per_split, a.wq);
-        ns = nsplit_of(max_blocks, pages_per_split);
-    }
     a.nsplit = ns;
     a.merge = ns > 1 && T * G <= 16 && (ns <= MERGE_ANY || (ns <= MERGE_MAX && T * G <= 8 * attn_wpp(pages_per_split)));
-    if (workspace) {
+    if (ns > 1) {  // one split leaves the workspace alone
         const WsLayout L = ws_layout(B, T, NKV, G, ns);
         char *ws = static_cast<char *>(workspace);
         a.cnt = reinterpret_cast<int *>(ws + L.cnt);

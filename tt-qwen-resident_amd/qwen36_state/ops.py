@@ -5,6 +5,8 @@ shapes, dtypes, devices and contiguity (ValueError on a mismatch, like the refer
 enqueues HIP kernels on the current torch stream. Tensors are caller-owned; state arguments are updated in
 place as in the reference. Nothing here computes on the CPU.
 """
+import functools
+
 import torch
 
 from ._lib import call, lib
@@ -440,6 +442,22 @@ def paged_fill_cache(cache, x, page_table, batch_idx=0):
 # ------------------------------------------------------------------------------------------- a6
 
 
+@functools.lru_cache(maxsize=1024, typed=True)
+def _walk(B, T, nq, nkv, max_blocks, pages_per_split, mixer):
+    """The pages a workgroup is best given to walk, at most the caller's, and the bytes of a workspace for them."""
+    pages = lib().qs_paged_attention_walk_pages(B, T, nq, nkv, max_blocks, pages_per_split, mixer)
+    return pages, lib().qs_paged_attention_workspace_bytes(B, T, nq, nkv, HD, max_blocks, pages_per_split)
+
+
+def _pages(B, T, nq, nkv, max_blocks, pages_per_split, mixer, ws):
+    """Pages per split of a launch: the best ones where ``ws`` holds their partials, else as the caller says (a buffer
+    too small for them may be given where the caller's own split needs none)."""
+    if ws is None:
+        return pages_per_split
+    pages, nbytes = _walk(B, T, nq, nkv, max_blocks, pages_per_split, mixer)
+    return pages if ws.nbytes >= nbytes else pages_per_split
+
+
 def attention_workspace(B, T, nq, nkv, max_blocks, pages_per_split, device):
     nbytes = lib().qs_paged_attention_workspace_bytes(B, T, nq, nkv, HD, max_blocks, pages_per_split)
     return workspace(("attn", pages_per_split), nbytes, device)
@@ -472,8 +490,9 @@ def paged_gqa_decode(q, k_cache, v_cache, block_table, seq_lens, scale, k_new=No
     _chk(o, "out", torch.bfloat16, (B, T, nq, hd), dev)
     if ws is None and (mb + pages_per_split - 1) // pages_per_split > 1:
         ws = attention_workspace(B, T, nq, nkv, mb, pages_per_split, dev)
+    pps = _pages(B, T, nq, nkv, mb, int(pages_per_split), False, ws)
     call("qs_paged_gqa_decode", _p(q), _p(k_new), _p(v_new), _p(k_cache), _p(v_cache), _p(block_table),
-         _p(seq_lens), _p(o), _p(ws), B, T, nq, nkv, hd, block, mb, nb, int(pages_per_split), float(scale),
+         _p(seq_lens), _p(o), _p(ws), B, T, nq, nkv, hd, block, mb, nb, pps, float(scale),
          _p(status), _stream(dev))  # fmt: skip
     return o
 
@@ -626,9 +645,10 @@ def attn_mixer_decode(q, k_new, v_new, gate, wq, wk, cos, sin, k_cache, v_cache,
     o = torch.empty(B, T, nq, hd, dtype=torch.bfloat16, device=dev) if out is None else out
     if ws is None:
         ws = attention_workspace(B, T, nq, nkv, mb, pages_per_split, dev)
+    pps = _pages(B, T, nq, nkv, mb, pages_per_split, True, ws)
     call("qs_attn_mixer_decode", _p(q), _p(k_new), _p(v_new), _p(gate), _p(wq), _p(wk),
          _p(cos if rot else None), _p(sin if rot else None), rot, _p(k_cache), _p(v_cache), _p(block_table),
-         _p(seq_lens), _p(o), _p(ws), B, T, nq, nkv, hd, block, mb, nb, pages_per_split, float(eps), _p(status),
+         _p(seq_lens), _p(o), _p(ws), B, T, nq, nkv, hd, block, mb, nb, pps, float(eps), _p(status),
          _stream(dev))  # fmt: skip
     return o
 
