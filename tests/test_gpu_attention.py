@@ -75,6 +75,8 @@ def run_case(dev, d, pps, fused=True):
         (2, 3000, 6, 4),  # 36 query rows per KV head: three tiles of the rows kernel
         (1, 700, 7, 64),  # three tiles, odd token count, one split
         (3, 900, 2, 4),  # 12 query rows per KV head: two tokens on the one-tile MFMA kernel
+        (2, 60, 1, 8),  # a one-page table without a workspace: one page per workgroup, one token
+        (2, 60, 3, 8),  # and three
     ],
 )
 def test_attention(dev, B, ctx, T, pps):

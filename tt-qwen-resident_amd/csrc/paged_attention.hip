@@ -1345,7 +1345,9 @@ int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps, bool mixer
     return std::min(pps, p > 1 ? (p + 1) & ~1 : 1);
 }
 // Pages a workgroup of the independent-wave kernel walks at once (4 waves each): two when the split has more
-// than one page (batch 8 at 4096 positions: 26.8 against 27.7 us; batch 1 at 32768: 29.8 against 30.4).
+// than one page (batch 8 at 4096 positions: 26.8 against 27.7 us; batch 1 at 32768: 29.8 against 30.4). pps is at most the
+// table's width: a one-page table is walked by 4 waves whatever the caller allows (batch 1 at 60 positions, three tokens
+// 9.0 -> 7.5 us, one 7.4 -> 6.5).
 int attn_wpp(int pps) { return pps >= 2 ? 2 : 1; }
 
 }  // namespace
@@ -1369,7 +1371,7 @@ extern "C" int qs_paged_attention_walk_pages(int B, int T, int NQ, int NKV, int 
 
 static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const char *who, void *stream) {
     const int B = a.B, T = a.T, NQ = a.NQ, NKV = a.NKV, max_blocks = a.max_blocks;
-    const int pages_per_split = a.pps;
+    int pages_per_split = a.pps;
     QS_REQUIRE(a.q && a.k_cache && a.v_cache && a.block_table && a.seq_lens && a.o, "%s: null pointer", who);
     QS_REQUIRE((a.k_new == nullptr) == (a.v_new == nullptr), "%s: give both k_new and v_new or neither", who);
     QS_REQUIRE(HDa == HD, "%s: HD must be %d (got %d)", who, HD, HDa);
@@ -1387,6 +1389,7 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
     QS_REQUIRE((size_t)B * NKV * sizeof(int) <= CNT_BYTES, "%s: B NKV = %d exceeds %d", who, B * NKV,
                (int)(CNT_BYTES / sizeof(int)));
     a.nsplit = ns;
+    pages_per_split = a.pps = std::min(pages_per_split, max_blocks);
     a.merge = ns > 1 && T * G <= 16 && (ns <= MERGE_ANY || (ns <= MERGE_MAX && T * G <= 8 * attn_wpp(pages_per_split)));
     if (ns > 1) {  // one split leaves the workspace alone
         const WsLayout L = ws_layout(B, T, NKV, G, ns);
