@@ -32,7 +32,10 @@ def plan(B, T, G, width, pps, mixer=False, nkv=4):
     p = -(-width // most) if most else pps
     p = min(pps, p if p <= 1 or not most else p + p % 2)
     ns = -(-width // p)
-    return p, ns, 1 < ns and R <= 16 and (ns <= 4 or ns <= 8 and R <= (16 if p > 1 else 8))
+    wpp = 2 if p > 1 else 1
+    rows, wgs = -(-R // (4 * wpp)), B * nkv * ns
+    few = wgs * rows * rows <= 192 or rows == 1 and (T > 2 or wpp == 1 and wgs > 256)
+    return p, ns, 1 < ns and R <= 16 and (ns <= 4 or R <= 8 * wpp and (ns <= 8 or ns <= 16 and few))
 
 
 def split_rows(ws):
@@ -222,12 +225,16 @@ def test_in_launch_merge_counters_rearm(dev):
         assert_attn_output(o, O.bf16(ref))
 
 
-# Where the merge moves between the launches: 4 and 5 splits of 12 rows and 8 and 9 of 6 on one page per workgroup, 8 and
-# 9 of 12 rows on two pages, 2 splits of 16 rows (group size 8) and of 18; and where a table stays whole: 2 and 3 pages of
-# 6 rows at batch 4, 2 but not 3 at batch 5, 4 but not 5 of 12 rows at batch 4, 3 but not 4 at batch 5, 2 but not 3 of 24.
-# The partials written show the split count.
+# Where the merge moves between the launches: 4 and 5 splits of 12 rows and 8 and 9 of 6 on one page per workgroup (9 at
+# batch 1 in the launch), 8 and 9 of 12 rows on two pages, 2 splits of 16 rows (group size 8) and of 18; 16 splits in the
+# launch for 4 rows at batch 1, one row at batch 3 and, past a workgroup per CU, 5, but not 4, and 4 tokens of one head, or
+# 8 of them on two pages, at batch 4, not for 8 rows. And where a table stays whole: 2 and 3 pages of 6 rows at batch 4, 2
+# but not 3 at batch 5, 4 but not 5 of 12 rows at batch 4, 3 but not 4 at batch 5, 2 but not 3 of 24. The partials written
+# show the split count.
 @pytest.mark.parametrize("B,G,T,width,pps,splits,merged", [
     (6, 6, 2, 4, 2, 4, True), (2, 6, 2, 5, 2, 5, False), (2, 6, 1, 8, 8, 8, True), (2, 6, 1, 9, 8, 9, False),
+    (1, 6, 1, 9, 8, 9, True), (1, 4, 1, 16, 8, 16, True), (3, 1, 1, 16, 1, 16, True), (4, 1, 1, 16, 8, 16, False),
+    (5, 1, 1, 16, 1, 16, True), (1, 8, 1, 16, 8, 16, False), (4, 1, 4, 16, 8, 16, True), (4, 1, 8, 64, 8, 16, True),
     (8, 6, 2, 16, 2, 8, True), (7, 6, 2, 18, 8, 9, False), (64, 8, 2, 5, 4, 2, True), (64, 6, 3, 5, 4, 2, False),
     (4, 6, 1, 1, 8, 1, False), (4, 6, 1, 2, 2, 1, False), (4, 6, 1, 3, 8, 1, False), (4, 6, 1, 3, 2, 3, True),
     (5, 6, 1, 2, 8, 1, False), (5, 6, 1, 3, 8, 3, True), (4, 6, 2, 4, 8, 1, False), (4, 6, 2, 5, 8, 5, False),
@@ -469,7 +476,7 @@ def test_verify_token_forms(dev, G, T, width, mixer):
 # A table wider than its users: the splits past a user's pages write no partial, and the merges read none of theirs (the
 # workspace holds NaNs); table entries past a user's pages are not looked at. Merged in the launch (4 and 8 splits) and in
 # one of their own (16 to 24, and 65, past one load of every split's maximum); users of one page, of all, idle.
-@pytest.mark.parametrize("B,T,width,pps,merged", [(16, 1, 16, 4, True), (8, 2, 16, 2, True), (3, 1, 128, 8, False),
+@pytest.mark.parametrize("B,T,width,pps,merged", [(16, 1, 16, 4, True), (8, 2, 16, 2, True), (3, 1, 144, 8, False),
                                                   (5, 2, 24, 1, False), (4, 4, 64, 8, False), (3, 8, 130, 2, False),
                                                   (3, 11, 40, 2, False)])  # fmt: skip
 @pytest.mark.parametrize("mixer", [False, True])

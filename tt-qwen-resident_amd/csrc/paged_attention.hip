@@ -19,6 +19,7 @@
 // 86-106 and kernels/attn_leader_compute.cpp:42-79) by the last workgroup of the (user, KV head) to finish
 // when there are few (AttnArgs::merge), else by a separate merge launch, so results are identical run to run.
 #include <algorithm>
+#include <type_traits>
 
 #include "qs_common.h"
 
@@ -245,12 +246,8 @@ constexpr int VPAD = HD + 16;  // K / V slice row pitch (bf16): 32-byte skew bet
 // in split order, so the result does not depend on which workgroup finished last. No L2-wide writeback or
 // invalidate is needed because only sc1 accesses touch the shared data. (The leader side of the
 // reference: kernels/attn_leader_writer.cpp:86-106, kernels/attn_leader_compute.cpp:42-79.)
-// Up to 4 splits, or 8 where 2 rows per wave cover the user's query rows, are merged there; more, and every verify step
-// of the rows kernel, in a launch of their own. Per layer, in the launch against in its own: one token (6 rows), a page
-// per workgroup (4 waves), 2 / 4 / 8 / 16 splits at batch 1 8.8, 9.0, 9.5, 10.3 against 9.7, 9.7, 10.0, 10.0 us and at
-// batch 4 9.2, 9.4, 10.5, 12.8 against 10.2, 10.1, 10.3, 10.6; two tokens (12 rows) at batch 1 9.8, 10.1, 10.8, 12.3
-// against 9.9, 9.9, 10.0, 10.0 and 4 splits at batch 8 10.5 against 10.9; two pages (8 waves), 8 splits 11.2 against 11.2.
-constexpr int MERGE_MAX = 8, MERGE_ANY = 4;
+// merge_here says which calls are merged so; the others, and every step of the rows kernel, in a launch of their own.
+constexpr int MERGE_ANY = 4, MERGE_MAX = 8, MERGE_MOST = 16;
 template <int NWV>
 __device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b, int g, int tid, int n) {
     __shared__ int s_last;
@@ -273,49 +270,57 @@ __device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b,
                                                       (short)0, ns * R * HD * 4, 0x00020000);
     const auto rm = __builtin_amdgcn_make_buffer_rsrc(qs::uniform_ptr(a.part_ml + prow(a, G, b, g, 0, 0) * 2),
                                                       (short)0, ns * R * 8, 0x00020000);
-    for (int r0 = w; r0 < R; r0 += 2 * NWV) {
-        f32x4_t x[2][MERGE_MAX];
-        float2 ml[2];
-        uint2 gw[2];
+    // ROWS query rows of a wave at a time, MOST splits
+    auto merge = [&](auto rows, auto most) {
+        constexpr int ROWS = decltype(rows)::value, MOST = decltype(most)::value;
+        for (int r0 = w; r0 < R; r0 += ROWS * NWV) {
+            f32x4_t x[ROWS][MOST];
+            float2 ml[ROWS];
+            uint2 gw[ROWS];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int qr = r0 + NWV * j;
-            if (qr >= R) continue;
+            for (int j = 0; j < ROWS; ++j) {
+                const int qr = r0 + NWV * j;
+                if (qr >= R) continue;
 #pragma unroll
-            for (int sp = 0; sp < MERGE_MAX; ++sp)
-                if (sp < ns)
-                    x[j][sp] = __builtin_bit_cast(
-                        f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ro, ((sp * R + qr) * HD + 4 * lane) * 4, 0,
-                                                                        qs::CP_SC1));
-            ml[j] = make_float2(-INFINITY, 0.f);
-            if (lane < ns) {
-                const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(rm, (lane * R + qr) * 8, 0, qs::CP_SC1);
-                ml[j] = make_float2(__uint_as_float(u[0]), __uint_as_float(u[1]));
+                for (int sp = 0; sp < MOST; ++sp)
+                    if (sp < ns)
+                        x[j][sp] = __builtin_bit_cast(
+                            f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ro, ((sp * R + qr) * HD + 4 * lane) * 4, 0,
+                                                                            qs::CP_SC1));
+                ml[j] = make_float2(-INFINITY, 0.f);
+                if (lane < ns) {
+                    const u32x2 u = __builtin_amdgcn_raw_buffer_load_b64(rm, (lane * R + qr) * 8, 0, qs::CP_SC1);
+                    ml[j] = make_float2(__uint_as_float(u[0]), __uint_as_float(u[1]));
+                }
+                if (a.gate)
+                    gw[j] = *reinterpret_cast<const uint2 *>(
+                        a.gate + (((size_t)b * T + qr / G) * a.NQ + g * G + qr % G) * HD + 4 * lane);
             }
-            if (a.gate)
-                gw[j] = *reinterpret_cast<const uint2 *>(
-                    a.gate + (((size_t)b * T + qr / G) * a.NQ + g * G + qr % G) * HD + 4 * lane);
-        }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int qr = r0 + NWV * j;
-            if (qr >= R) continue;
-            const float M = qs::wave_max_bcast(ml[j].x);
-            const float e = ml[j].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[j].x - M);
-            const float L = qs::wave_sum_dpp(e * ml[j].y);
-            f32x4_t O = {0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < ROWS; ++j) {
+                const int qr = r0 + NWV * j;
+                if (qr >= R) continue;
+                const float M = qs::wave_max_bcast(ml[j].x);
+                const float e = ml[j].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[j].x - M);
+                const float L = qs::wave_sum_dpp(e * ml[j].y);
+                f32x4_t O = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int sp = 0; sp < MERGE_MAX; ++sp)
-                if (sp < ns) O += qs::lane_val(e, sp) * x[j][sp];
-            O *= 1.0f / L;
-            if (a.gate) {
-                O[0] *= sigm(qs::bf_lo(gw[j].x)), O[1] *= sigm(qs::bf_hi(gw[j].x));
-                O[2] *= sigm(qs::bf_lo(gw[j].y)), O[3] *= sigm(qs::bf_hi(gw[j].y));
+                for (int sp = 0; sp < MOST; ++sp)
+                    if (sp < ns) O += qs::lane_val(e, sp) * x[j][sp];
+                O *= 1.0f / L;
+                if (a.gate) {
+                    O[0] *= sigm(qs::bf_lo(gw[j].x)), O[1] *= sigm(qs::bf_hi(gw[j].x));
+                    O[2] *= sigm(qs::bf_lo(gw[j].y)), O[3] *= sigm(qs::bf_hi(gw[j].y));
+                }
+                *reinterpret_cast<uint2 *>(a.o + (((size_t)b * T + qr / G) * a.NQ + g * G + qr % G) * HD + 4 * lane) =
+                    make_uint2(qs::cvt_pk_bf16(O[0], O[1]), qs::cvt_pk_bf16(O[2], O[3]));
             }
-            *reinterpret_cast<uint2 *>(a.o + (((size_t)b * T + qr / G) * a.NQ + g * G + qr % G) * HD + 4 * lane) =
-                make_uint2(qs::cvt_pk_bf16(O[0], O[1]), qs::cvt_pk_bf16(O[2], O[3]));
         }
-    }
+    };
+    if (ns <= MERGE_MAX)
+        merge(std::integral_constant<int, 2>{}, std::integral_constant<int, MERGE_MAX>{});
+    else
+        merge(std::integral_constant<int, 1>{}, std::integral_constant<int, MERGE_MOST>{});
 }
 
 // ------------------------------------------------------------------------------ MFMA kernel (verify rows)
@@ -1349,6 +1354,22 @@ int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps, bool mixer
 // table's width: a one-page table is walked by 4 waves whatever the caller allows (batch 1 at 60 positions, three tokens
 // 9.0 -> 7.5 us, one 7.4 -> 6.5).
 int attn_wpp(int pps) { return pps >= 2 ? 2 : 1; }
+// Whether the splits of a call of R <= 16 query rows per KV head, wgs workgroups of 4 wpp waves, are merged inside the
+// launch. Up to 4 splits, or 8 where 2 rows per wave cover the rows, always: one token (6 rows), a page per workgroup (4
+// waves), in the launch against in its own, us a layer, 2 / 4 / 8 splits at batch 1 8.8, 9.0, 9.5 against 9.7, 9.7, 10.0 and
+// at batch 4 9.2, 9.4, 10.5 against 10.2, 10.1, 10.3; two tokens (12 rows) at batch 1 9.8, 10.1, 10.8 against 9.9, 9.9, 10.0
+// and 4 splits at batch 8 10.5 against 10.9; two pages (8 waves), 8 splits 11.2 against 11.2. 9 to 16 splits where few
+// workgroups do so at a time: 4 rows, batch 1, 9 / 16 splits 9.2, 9.6 against 10.4, 10.6, batch 2 16 splits 10.5 against
+// 10.7, batch 4 9 / 12 / 16 splits 10.4, 11.1, 12.1 against 10.7, 10.9, 11.1; 6 rows (two to a wave, one after the other)
+// batch 1 9 / 12 / 16 splits 9.7, 10.1, 10.8 against 10.3, 10.3, 10.4. And with one row per wave, where the calls are longer:
+// three or more tokens, which store their rows first (4 tokens of one head, batch 4, 9 / 16 splits 12.5, 13.6 against 13.7,
+// 14.2), and more than one workgroup per CU (4 rows, batch 8, 16 splits 13.6 against 14.8).
+bool merge_here(int T, int R, int wpp, int ns, long wgs) {
+    if (ns <= MERGE_ANY) return true;
+    if (R > 8 * wpp || ns > MERGE_MOST) return false;
+    const int rows = (R + 4 * wpp - 1) / (4 * wpp);  // rows per wave of the merging workgroup
+    return ns <= MERGE_MAX || wgs * rows * rows <= 192 || (rows == 1 && (T > 2 || (wpp == 1 && wgs > 256)));
+}
 
 }  // namespace
 
@@ -1390,7 +1411,8 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
                (int)(CNT_BYTES / sizeof(int)));
     a.nsplit = ns;
     pages_per_split = a.pps = std::min(pages_per_split, max_blocks);
-    a.merge = ns > 1 && T * G <= 16 && (ns <= MERGE_ANY || (ns <= MERGE_MAX && T * G <= 8 * attn_wpp(pages_per_split)));
+    const int wpp = attn_wpp(pages_per_split), R = T * G;
+    a.merge = ns > 1 && R <= 16 && merge_here(T, R, wpp, ns, (long)B * NKV * ns);
     if (ns > 1) {  // one split leaves the workspace alone
         const WsLayout L = ws_layout(B, T, NKV, G, ns);
         char *ws = static_cast<char *>(workspace);
@@ -1401,9 +1423,7 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
     const dim3 grid(B * NKV * ns);
     hipStream_t st = QS_STREAM(stream);
     QS_REQUIRE(G == 1 || G == 2 || G == 4 || G == 6 || G == 8, "%s: group size NQ/NKV = %d not in {1, 2, 4, 6, 8}", who, G);
-    const int R = T * G;
     if (R <= 16) {  // every one-token decode
-        const int wpp = attn_wpp(pages_per_split);
 #define QS_WAVE(GG)                                                              \
     if (a.wq) {                                                                  \
         if (wpp == 1) attn_wave_kernel<GG, 1, true><<<grid, 256, 0, st>>>(a);    \
