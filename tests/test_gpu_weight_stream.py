@@ -90,13 +90,15 @@ def _rel(a, b):
 # the last workgroup of a block applying silu after K splits: (16, 5120, 1024) gate | up in 4 splits,
 # (4, 5120, 2048) in 2; (1, 10240, 512): one row too long for the gate | up workgroups to normalise, through the
 # rmsnorm kernel's two passes over 8192-value chunks
-# column blocks and K splits: (2, 128, 64) one group for 8 waves; (16, 5120, 10240) 4 tiles per block, 3 splits in both
-# projections; (2, 2560, 17088) 2 tiles per block, 512 blocks whole and 22 in 2 splits, down 4 tiles in 6 splits;
-# (1, 6144, 1024) the longest row gate | up workgroups normalise, (1, 6272, 512) the first past it
+# column blocks and K splits: (2, 128, 64) one group for 8 waves; (16, 5120, 10240) 4 tiles per block, gate | up whole,
+# down in 3 splits; (2, 2560, 17088) 2 tiles per block, 512 blocks whole and 22 in 2 splits, down 4 tiles in 6 splits;
+# (3, 4096, 16448) 4 tiles per block, 256 blocks whole and one in 4 splits; (2, 2176, 4224) 1 tile per block, 256 whole
+# and 8 in 2 splits; (1, 6144, 1024) the longest row gate | up workgroups normalise, (1, 6272, 512) the first past it
 @pytest.mark.parametrize("B,H,I,fmt", [(2, 128, 64, 9), (1, 128, 64, 9), (16, 5120, 10240, 9), (2, 2560, 17088, 8),
                                        (1, 6144, 1024, 9), (1, 6272, 512, 9), (1, 256, 512, 9), (8, 512, 1024, 9), (16, 256, 256, 9), (1, 5120, 17408, 9),
                                        (16, 5120, 1024, 9), (5, 1024, 2048, 9), (4, 5120, 2048, 9), (1, 10240, 512, 9),
-                                       (1, 5120, 17408, 8), (16, 256, 256, 8), (4, 5120, 2048, 8)])  # fmt: skip
+                                       (1, 5120, 17408, 8), (16, 256, 256, 8), (4, 5120, 2048, 8),
+                                       (3, 4096, 16448, 9), (2, 2176, 4224, 8)])  # fmt: skip
 def test_mlp_decode(dev, B, H, I, fmt):
     x, gamma, gate, up, down = _mlp(dev, B, H, I, down_fmt=fmt)
     out = ops.mlp_decode(x.to(dev), gamma.to(dev), gate, up, down).cpu().double()

@@ -613,9 +613,14 @@ __global__ __launch_bounds__(64 * ROWS_WAVES, 4) void rows_kernel(Proj a) {
 // of 8 waves (H 3456 / I 9920, 16 rows: 29.7 us at 3 groups and 32.7 at 2, where too little overlaps the stream's
 // start and end; 37.5 at 6, where one tile per wave reads the rows too often).
 // Splits: a launch's time follows the most workgroups any CU holds, so the blocks past the last multiple of 256
-// are cut along K into s parts, s minimising ceil(rest s / 256) / s plus 1% of a block's time per part for the
-// partials' way through memory (0.4% and 2.5% measured alike, except 33.9 against 30.7 us at H 3456 / I 9920
-// at 0.4%).
+// are cut along K into s parts, s minimising the time of the CU with the most of them: ceil(rest s / 256) parts, each 1 / s
+// of a block's time and its own fill and drain (that of 2 K groups per wave of gate | up, half a group of the 8-bit
+// formats), plus 1% of a block's time per part for the partials' way through memory (0.4% and 2.5% measured alike, except
+// 33.9 against 30.7 us at H 3456 / I 9920 at 0.4%). Without the fill and drain many blocks were cut until a wave had one
+// group left and nothing in flight behind it: H 4096 / I 12288, 192 blocks of gate | up in 4 parts each 35.2 us at 2 rows
+// and 38.8 at 16, uncut 29.7 and 32.5; H 5120 / I 25600, 144 of 400 in 5 parts 62.4 and 69.9, uncut 61.1 and 66.5; H 2176 /
+// I 4224, one row, 136 blocks of down in 7 parts 15.2, in 3 13.7. Over 41 shapes of H 512 to 7168 and I 1536 to 25600 at 1 to 16 rows no plan measured
+// more than 0.4 us slower for it, also with twice the gate | up's term.
 struct RowsPlan {
     int nt;             // column tiles per block
     int units;          // column blocks
@@ -630,9 +635,10 @@ RowsPlan rows_plan(int K, int N, int fmt, int nt = 4) {
     p.units = (ntile + p.nt - 1) / p.nt;
     const int whole = p.units / 256 * 256, rest = p.units - whole;
     p.nsplit = 1;
+    const double fill = (fmt == FMT_FP4 ? 2.0 : 0.5) * ROWS_WAVES / nq;  // in block times
     double cost = 1e30;
     for (int s = 1; s <= 16 && nq / s >= ROWS_WAVES; ++s) {
-        const double c = (double)((rest * s + 255) / 256) / s + (s - 1) * 0.01;
+        const double c = (rest * s + 255) / 256 * (1.0 / s + fill) + (s - 1) * 0.01;
         if (c < cost) cost = c, p.nsplit = s;
     }
     p.nwhole = p.nsplit == 1 ? p.units : whole;
