@@ -79,6 +79,21 @@ def test_conv_prefill_pieces_equal_the_whole(dev):
     assert torch.equal(b[3], whole)
 
 
+def test_conv_prefill_blocks_by_channels(dev):
+    """The line between the two lies at tokens times channels: 40960 channels, 769 tokens (8 per thread) equal, bit for
+    bit, their pieces of 767 and 2 (4 per thread)."""
+    nk, nv, T = 64, 192, 769
+    c = (2 * nk + nv) * 128
+    gen = torch.Generator().manual_seed(8)
+    xg = torch.randn(T, c, generator=gen).bfloat16().to(dev)
+    csg, tg = (torch.randn(c, n, generator=gen).bfloat16().to(dev) for n in (3, 4))
+    *whole, st = ops.causal_conv1d_prefill(xg, tg, csg, nk=nk, nv=nv)
+    *a, mid = ops.causal_conv1d_prefill(xg[:767], tg, csg, nk=nk, nv=nv)
+    *b, end = ops.causal_conv1d_prefill(xg[767:], tg, mid, nk=nk, nv=nv)
+    assert all(torch.equal(torch.cat([x, y]), z) for x, y, z in zip(a, b, whole))
+    assert torch.equal(st, end)
+
+
 def test_conv_prefill_8192_tokens(dev):
     """The prompt length of the prefill workload: 8192 tokens of the 10240 q | k | v channels."""
     T = 8192

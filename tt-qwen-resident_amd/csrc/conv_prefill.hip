@@ -7,8 +7,8 @@
 // fp32), so y equals T successive decode conv steps bit for bit, and the carry is the decode conv state
 // those steps leave.
 //
-// One thread per 8 adjacent channels (16-byte rows) and R = 8 tokens: it loads the 11 window rows it needs
-// (the 3 before its block from x, or from the carry for the first block), then writes 8 output rows into
+// One thread per 8 adjacent channels (16-byte rows) and R = 4 or 8 tokens: it loads the R + 3 window rows it needs
+// (the 3 before its block from x, or from the carry for the first block), then writes R output rows into
 // the q, k or v plane its channels belong to (channels [0, CQ) -> q, [CQ, 2 CQ) -> k, [2 CQ, 2 CQ + CV) -> v).
 // The threads of the first token block also write the new carry; they are the only readers of the carry
 // in, so the carry may be updated in place. Lanes run over channel groups, so every row access is a
@@ -161,11 +161,12 @@ extern "C" int qs_conv1d_prefill(const uint16_t *x, int ldx, const uint16_t *con
     ConvPrefillArgs a{};
     a.x = x, a.st_in = conv_state_in, a.taps = taps, a.q = q, a.k = k, a.v = v, a.st_out = conv_state_out;
     a.ldx = ldx, a.T = T, a.CQ = CQ, a.CV = CV, a.ngroups = C / 8;
-    // tokens per thread: 8, or 4 for prompts too short to fill the chip with blocks of 8 (the carry's rows reach 3
-    // tokens into the prompt and only the first block may read them, so not fewer). 10240 channels, 8 -> 4: 16 tokens
-    // 8.8 -> 6.0 us, 200 9.2 -> 6.4, 1000 13.5 -> 13.0, 3000 30.0 -> 28.1, 4096 37.6 -> 37.5, 8192 67.2 -> 68.8
-    // (16, 24, 32 and 4 blocks of 16 in sequence measured slower than 8 there)
-    const int R = T <= 3072 ? 4 : 8;
+    // tokens per thread: 8, or 4 for prompts too short for their channels to fill the chip with blocks of 8 (the carry's
+    // rows reach 3 tokens into the prompt and only the first block may read them, so not fewer). 10240 channels, 8 -> 4: 16
+    // tokens 8.8 -> 6.0 us, 200 9.2 -> 6.4, 1000 13.5 -> 13.0, 3000 30.0 -> 28.1, 4096 37.6 -> 37.5, 8192 67.2 -> 68.8
+    // (16, 24, 32 and 4 blocks of 16 in sequence measured slower than 8 there); 2048 channels, 4096 12.8 -> 11.2, 8192 18.9 ->
+    // 18.2; 40960 channels, 500 23.0 -> 20.5, 1000 40.2 -> 40.2, 2500 87.2 -> 92.5
+    const int R = (long)T * C <= 3072L * 10240 ? 4 : 8;
     a.ntb = T > 0 ? (T + R - 1) / R : 1;
     const long wgs = (long)((a.ngroups + 63) / 64) * ((a.ntb + 3) / 4);
     QS_REQUIRE(wgs < (1L << 31), "qs_conv1d_prefill: T = %d tokens are too many for one launch", T);
