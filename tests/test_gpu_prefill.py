@@ -116,6 +116,15 @@ def test_prefill_fresh_prompts_start_from_zero(dev):
         S1.fill_(7.0), S2.fill_(7.0)  # the outputs are the caller's
 
 
+def test_prefill_row_forms(dev):
+    """k and v in any form whose rows are the tokens' in order: [2 T, heads / 2, 128] counts as [T, heads, 128]."""
+    d = {k: v.to(dev) for k, v in W.prefill(66, "cpu", seed=12).items()}
+    o, S = run(dev, d, 66)
+    o1, S1 = ops.chunk_gated_delta_rule(d["q"], d["k"].view(132, 8, 128), d["v"].view(132, 24, 128), d["g"], d["beta"],
+                                        initial_state=d["S0"])  # fmt: skip
+    assert torch.equal(o1, o) and torch.equal(S1, S)
+
+
 def test_prefill_repeatable(dev):
     d = W.prefill(300, "cpu", seed=7)
     a = run(dev, d, 300)

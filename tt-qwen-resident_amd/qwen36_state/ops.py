@@ -580,7 +580,7 @@ def chunk_gated_delta_rule(q, k, v, g, beta, *, scale=None, initial_state=None, 
     dev = q.device
     T = q.shape[0]
     nv = g.shape[1]
-    heads = lambda t, d: t if t.dim() == 3 and t.shape[2] == d else t.reshape(T, -1, d)  # noqa: E731
+    heads = lambda t, d: t if t.dim() == 3 and t.shape[0] == T and t.shape[2] == d else t.reshape(T, -1, d)  # noqa: E731
     q3 = heads(q, DK)
     nk = q3.shape[1]
     _chk(q3, "q", torch.bfloat16, (T, nk, DK), dev)
