@@ -259,8 +259,8 @@ int qs_attn_mixer_decode(const uint16_t *q, const uint16_t *k_new, const uint16_
 /* ---------------------------------------------------------------------------------------- a8: prefill
  * Chunked gated delta rule over one sequence (WY/UT form, bf16 MFMA, fp32 state carry), L2-norm of q
  * (times scale) and k inside:
- *   q, k [T, NK, DK] bf16; v [T, NV, DV] bf16; g, beta [T, NV] fp32; initial_state [NV, DK, DV] fp32
- *   -> o [T, NV, DV] bf16 (token-major), final_state [NV, DK, DV] fp32 (may alias initial_state).
+ *   q, k [T, NK, DK] bf16; v [T, NV, DV] bf16; g, beta [T, NV] fp32; initial_state [NV, DK, DV] fp32, or
+ *   null for a fresh prompt (zeros) -> o [T, NV, DV] bf16 (token-major), final_state [NV, DK, DV] fp32 (may alias initial_state).
  * chunk: 32 (the reference prefill's chunk_size, prefill/pp_prefill.py:56, :801) or 64. The chunked form
  * equals the token-by-token recurrence for every chunk size, so both run the kernels' 64-token chunks;
  * any other value is rejected.

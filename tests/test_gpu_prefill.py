@@ -114,6 +114,7 @@ def test_prefill_fresh_prompts_start_from_zero(dev):
         o2, S2 = ops.chunk_gated_delta_rule(*few)
         assert torch.equal(o1, o) and torch.equal(S1, S) and torch.equal(o2, o4) and torch.equal(S2, S4)
         S1.fill_(7.0), S2.fill_(7.0)  # the outputs are the caller's
+    assert not any("zero" in str(kind) for kind, *_ in ops._WS)  # and nothing is kept for it
 
 
 def test_prefill_row_forms(dev):

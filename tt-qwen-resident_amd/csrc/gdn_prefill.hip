@@ -81,7 +81,7 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, void *lds, int o
 struct PrefillArgs {
     const uint16_t *q, *k, *v;  // [T, NK, DK], [T, NK, DK], [T, NV, DV]
     const float *g, *beta;      // [T, NV]
-    const float *S0;            // [NV, DK, DV]
+    const float *S0;            // [NV, DK, DV], or null: zeros
     float *ST;                  // [NV, DK, DV]
     uint16_t *o;                // [T, NV, DV]
     uint16_t *Tm;               // workspace [nch, NV, 2, 64 x 64] bf16: hi and lo planes of Tm, fragment order
@@ -455,11 +455,13 @@ __global__ __launch_bounds__(WALK_THREADS) void chunk_walk_kernel(PrefillArgs a)
         *reinterpret_cast<uint2 *>(&sS[0][v][d]) = hi;
         *reinterpret_cast<uint2 *>(&sS[1][v][d]) = lo;
     };
+    const auto r0 = rsrc(a.S0 + (size_t)h * DK * DV, a.S0 ? DK * DV * 4 : 0);  // without one an empty range: zeros
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            S[mt][i] = a.S0[((size_t)h * DK + 32 * w + 16 * mt + fq + i) * DV + SLAB * slab + 16 * role + fr];
+            S[mt][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                r0, ((32 * w + 16 * mt + fq + i) * DV + SLAB * slab + 16 * role + fr) * 4, 0, 0));
         mirror(mt);
     }
 
@@ -730,7 +732,7 @@ extern "C" int qs_gdn_chunk_prefill(const uint16_t *q, const uint16_t *k, const 
                                     const float *beta, const float *initial_state, uint16_t *o, float *final_state,
                                     void *workspace, int T, int NK, int NV, int DKa, int DVa, int chunk, float scale,
                                     float eps, void *stream) {
-    QS_REQUIRE(q && k && v && g && beta && initial_state && o && final_state && workspace,
+    QS_REQUIRE(q && k && v && g && beta && o && final_state && workspace,
                "qs_gdn_chunk_prefill: null pointer");
     QS_REQUIRE(T > 0, "qs_gdn_chunk_prefill: T must be positive (got %d)", T);
     QS_REQUIRE(DKa == DK && DVa == DV, "qs_gdn_chunk_prefill: DK and DV must be 128 (got %d, %d)", DKa, DVa);

@@ -531,15 +531,6 @@ def causal_conv1d_prefill(x, taps, conv_state=None, conv_state_out=None, nk=NK, 
     return q, k, v, conv_state_out
 
 
-def _zero_state(nv, dev):
-    """The zero start state of a fresh prompt, only ever read: a workspace of its own size, cleared once per stream
-    instead of by a launch per call (3 MB at 48 heads; a 200-token prompt's conv, rule and fill 38.3 -> 36.1 us). A
-    captured call clears one inside its graph, which then depends on no buffer kept here."""
-    if torch.cuda.is_current_stream_capturing():
-        return torch.zeros(nv, DK, DV, dtype=torch.float32, device=dev)
-    return workspace(("zero state", nv), 4 * nv * DK * DV, dev).view(torch.float32).view(nv, DK, DV)
-
-
 def chunk_gated_delta_rule(q, k, v, g, beta, *, scale=None, initial_state=None, output_final_state=True,
                            chunk_size=64, output_head_major=False, memory_config=None, eye=None, tril=None,
                            ones=None, masks=None, eps=EPS, ws=None, final_state=None):  # fmt: skip
@@ -548,7 +539,7 @@ def chunk_gated_delta_rule(q, k, v, g, beta, *, scale=None, initial_state=None, 
     (prefill/pp_prefill.py:791-807).
 
     q, k [T, NK*DK] or [T, NK, DK] bf16 token-major (L2-normalised inside, q times scale), v [T, NV*DV] or
-    [T, NV, DV] bf16, g, beta [T, NV] fp32, initial_state [NV, DK, DV] fp32. The reference's per-device
+    [T, NV, DV] bf16, g, beta [T, NV] fp32, initial_state [NV, DK, DV] fp32 or None (zeros). The reference's per-device
     tensors carry a leading batch dimension of 1 (q [1, T, NK*DK], g [1, T, NV], initial_state
     [1, NV, DK, DV]); that form is accepted too and keeps the dimension on the outputs.
     Returns (o, final_state): o [T, NV, DV] bf16 ([NV, T, DV] with output_head_major), final_state
@@ -588,9 +579,8 @@ def chunk_gated_delta_rule(q, k, v, g, beta, *, scale=None, initial_state=None, 
     _chk(heads(v, DV), "v", torch.bfloat16, (T, nv, DV), dev)
     _chk(g, "g", torch.float32, (T, nv), dev)
     _chk(beta, "beta", torch.float32, (T, nv), dev)
-    if initial_state is None:
-        initial_state = _zero_state(nv, dev)
-    _chk(initial_state, "initial_state", torch.float32, (nv, DK, DV), dev)
+    if initial_state is not None:
+        _chk(initial_state, "initial_state", torch.float32, (nv, DK, DV), dev)
     scale = DK**-0.5 if scale is None else scale
     o = torch.empty(T, nv, DV, dtype=torch.bfloat16, device=dev)
     S = torch.empty(nv, DK, DV, dtype=torch.float32, device=dev) if final_state is None else final_state
