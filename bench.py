@@ -671,7 +671,7 @@ def bench_mlp_layer(args, torch, tel):
     layers = [W.mlp_layer(B, "cuda:0", seed=i, keep_fp32=(i == 0 and not args.no_cpu)) for i in range(3)]
     for d in layers:
         d["out"] = torch.empty_like(d["x"])
-    ws = torch.empty(ops.lib().qs_mlp_decode_workspace_bytes(B, H, I), dtype=torch.uint8, device="cuda:0")
+    ws = torch.zeros(ops.lib().qs_mlp_decode_workspace_bytes(B, H, I), dtype=torch.uint8, device="cuda:0")
     R = 2
 
     def calls(st):

@@ -23,3 +23,11 @@ def test_launcher_world_size_refused():
     r = run_bench(["--gpus", "1"], {"WORLD_SIZE": "8"})
     assert r.returncode == 2
     assert "one GPU" in r.stderr
+
+
+def test_workspaces_are_zeroed():
+    """The kernels' workspaces hold arrival counters and must be zero before their first use: every one the bench
+    allocates is."""
+    src = open(os.path.join(ROOT, "bench.py")).read()
+    lines = [l for l in src.split("\n") if "_workspace_bytes(" in l and "torch." in l]
+    assert lines and all("torch.zeros(" in l for l in lines), lines
