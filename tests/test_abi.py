@@ -117,6 +117,17 @@ def test_attention_walk_pages():
         assert L.qs_paged_attention_walk_pages(1, 1, nq, 4, mb, pps, 0) == pps
 
 
+@pytest.mark.parametrize("name,raw", [("cuda:0", False), ("cuda", True)])
+def test_stream_handle_falls_back_to_the_public_call(monkeypatch, name, raw):
+    """A torch without the raw stream call, or a device without an index: the stream object's handle."""
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: Stream)
+    monkeypatch.setattr(ops, "_raw_stream", (lambda index: 1 + index) if raw else None)
+    assert ops._stream(torch.device(name)) == 77
+
+
 def test_ops_validate_before_calling():
     cpu = torch.zeros(1, 16, 128, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="GPU"):

@@ -27,9 +27,15 @@ def _p(t):
     return None if t is None else t.data_ptr()
 
 
+# the current stream's handle without a Stream object around it, where torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev):
-    """The current stream's handle on ``dev`` (a tensor's device), without a Stream object around it."""
-    return torch._C._cuda_getCurrentRawStream(dev.index)
+    """The current stream's handle on ``dev``."""
+    if _raw_stream is None or dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return _raw_stream(dev.index)
 
 
 def _chk(t, name, dtype, shape=None, dev=None):
