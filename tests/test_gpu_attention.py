@@ -529,3 +529,25 @@ def test_one_split_leaves_the_workspace(dev, T):
     assert torch.equal(o2, o) and torch.equal(none, o)
     check_mixer(dev, d, 8, 64, torch.Generator().manual_seed(T), ws=ws[:256])
     assert int((ws != 0xFF).sum()) == 0
+
+
+# 70 users x 4 KV heads, past a workgroup per CU, walk the caller's pages. One page group against two in the rows kernel, by
+# its tiles, the pages and the mixer, for up to 8 new tokens and more: 2 tiles at 4 and 5 pages, 3 and 4 tiles at 2 and 3,
+# with the mixer 2 tiles at 2 (in 2 splits, whole) and 3, 3 at 2.
+@pytest.mark.parametrize("G,T,width,pps,mixer", [
+    (6, 4, 8, 4, False), (6, 4, 10, 5, False), (2, 9, 10, 5, False), (6, 8, 4, 2, False), (6, 8, 6, 3, False),
+    (4, 9, 6, 3, False), (8, 8, 6, 3, False), (4, 13, 6, 3, False), (6, 4, 4, 2, True), (6, 4, 2, 2, True), (6, 4, 6, 3, True),
+    (2, 9, 6, 3, True), (6, 8, 4, 2, True),
+])  # fmt: skip
+def test_page_groups(dev, G, T, width, pps, mixer):
+    B = 70
+    assert plan(B, T, G, width, pps, mixer)[0] == pps
+    d = W.attn_layer(B, width * 64, "cpu", seed=G + T + width, T=T, num_blocks=B * width + 8)
+    gen = torch.Generator().manual_seed(G + T)
+    d["q"] = torch.randn(B, T, G * 4, 256, generator=gen).bfloat16()
+    d["seq_lens"] = torch.randint(T, width * 64 + 1, (B,), generator=gen).to(torch.int32)
+    if mixer:
+        return check_mixer(dev, d, pps, 64, gen)
+    o, ref, same = run_case(dev, d, pps)
+    assert same
+    assert_attn_output(o, ref)

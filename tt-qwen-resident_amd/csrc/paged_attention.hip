@@ -1349,6 +1349,15 @@ int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps, bool mixer
     const int p = (int)((max_blocks + most - 1) / most);
     return std::min(pps, p > 1 ? (p + 1) & ~1 : 1);
 }
+// Whether the rows kernel walks a few pages one at a time though it could two: its workgroups then share a CU by twos, one's
+// loads and merge of waves beside the other's pages, where the pair of groups is alone on it. One against two groups, us a
+// layer: 4 tokens (24 rows, 2 tiles) at 2 pages a split, batch 1 / 8192 15.9 against 17.3, batch 8 / 4000 42.8, 51.6, at 4
+// pages batch 8 / 4000 36.1, 39.1; 8 tokens (3 tiles) at 2 pages, batch 4 / 4000 35.7, 37.4, at 4 batch 4 / 8000 46.7, 46.5, at
+// 8 38.8, 37.4; with the mixer, 4 tokens at 2 pages, batch 4 / 8000 55.7, 57.6, batch 16 / 2000 60.2, 59.0, a whole table of 2
+// 14.7, 12.5, 4 pages batch 4 / 8000 43.0, 42.2, 8 tokens at 2 pages batch 8 / 4000 74.6, 73.4.
+bool rows_one(int tiles, int pps, int ns, bool mixer) {
+    return mixer ? tiles == 2 && pps == 2 && ns > 1 : pps <= 2 || (tiles == 2 && pps <= 4);
+}
 // Pages a workgroup of the independent-wave kernel walks at once (4 waves each): two when the split has more
 // than one page (batch 8 at 4096 positions: 26.8 against 27.7 us; batch 1 at 32768: 29.8 against 30.4). pps is at most the
 // table's width: a one-page table is walked by 4 waves whatever the caller allows (batch 1 at 60 positions, three tokens
@@ -1444,7 +1453,7 @@ static int attn_launch(AttnArgs a, void *workspace, int HDa, int block, const ch
         const int nrb = (R + 63) / 64, QT = rows_tiles(R);  // query rows in blocks of 16 QT
         QS_REQUIRE((long)grid.x * nrb < (1L << 31), "%s: grid too large", who);
         const dim3 rgrid(grid.x * nrb);
-        const bool two = pages_per_split >= 2 && rows_pairs(R, T, a.wq);
+        const bool two = pages_per_split >= 2 && rows_pairs(R, T, a.wq) && !rows_one(QT, pages_per_split, ns, a.wq);
         // A call is given the form for up to 8 new tokens where it can be (batch 1 / 3 tokens / 60 positions 7.7 -> 7.5 us,
         // 4 tokens with the mixer 13.2 -> 12.8)
 #define QS_ROWS(Q, MX, W, TN) attn_rows_kernel<Q, MX, W, TN><<<rgrid, 256 * W, 0, st>>>(a, G, nrb)
