@@ -686,7 +686,7 @@ def bench_mlp_layer(args, torch, tel):
     stats = {k: (v / n if k.endswith("_ms") else v) for k, v in stats.items()}
     nbytes = mlp_bytes(B, H, I)
     out = entry("MLP half of one decoder layer, 1 row: rmsnorm (weight folded into gate | up) + gate | up 5120 x "
-                "17408 MXFP4 with silu, down 17408 x 5120 MXINT8 in 4 K splits + residual (2 launches)", nbytes, ms,
+                "17408 MXFP4 with silu, down 17408 x 5120 MXINT8 in 3 K splits + residual (2 launches)", nbytes, ms,
                 stats,
                 roofline("mlp_decode", nbytes, ms))  # fmt: skip
     out["us_per_layer"] = out["us_per_step"]

@@ -274,8 +274,9 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     constexpr int RPL = RW / RG;   // rows per lane
     static_assert(RPL >= 1 && RW % RG == 0 && (VERIFY || TM == 1), "slab shape");
     static_assert(!NORM || (!VERIFY && WPG == NSLAB && CG <= 16), "the epilogue needs whole heads per workgroup");
-    // conv roles by wave of the workgroup (SPLITC below: otherwise): q channels on wave 0, k on wave 1 (when there is one; NW = 2: wave 2), the
-    // slab's v channels on wave 2 (NW = 4), each slab's wave 1 (NW = 2) or every wave for its own slab (NW = 1)
+    // conv roles by wave of the workgroup (SPLITC below: otherwise): q channels on wave 0, k on wave 1 (when there is one;
+    // NW = 2: wave 2), the slab's v channels on wave 2 (NW = 4), each slab's wave 1 (NW = 2) or every wave for its own slab
+    // (NW = 1)
     constexpr int WK = NW == 2 && WPG >= 2 ? 2 : (NW >= 4 || WPG >= 2) ? 1 : 0;
     constexpr int WV = NW >= 4 ? 2 : NW - 1;
     // the wave that writes o (and forms each token's q . k for it): the slab's last wave, which reaches each
@@ -399,7 +400,7 @@ __global__ __launch_bounds__(64 * NW * WPG) void gdn_kernel(GdnArgs a) {
     }
     // NORM: the epilogue's z and norm_w of the lane's 4 columns. Requested and read before any store leaves (read
     // after the last token they waited for the state stores too: 271 against 281 us for the 48 layers below), ahead of
-    // the state with several waves per slab (250 us), behind it with one (batch 8, 12 layers: 130.0 us behind, 137.6
+    // the state with several waves per slab (259 us), behind it with one (batch 8, 12 layers: 130.0 us behind, 137.6
     // ahead, 136.5 read after the token)
     uint2 z4 = make_uint2(0, 0);
     float4 w4 = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -805,7 +806,7 @@ void launch_gdn_tm(const GdnArgs &a, hipStream_t st) {
     const int per_key_head = (a.NV / a.NK) * (DV / 32);  // consecutive slab units sharing one key head
     if constexpr (!VERIFY) {
         // with the gated RMSNorm epilogue a workgroup holds one value head: its 4 slabs on one wave each at
-        // large batch, on 2 waves each below (batch 1, 48 layers: 250 us, with 4 waves each 293; batch 8, where 2
+        // large batch, on 2 waves each below (batch 1, 48 layers: 259 us, with 4 waves each 293; batch 8, where 2
         // waves each take 148 us for 12 layers, 137 with one)
         if (a.z) {
             if (units >= 1024)

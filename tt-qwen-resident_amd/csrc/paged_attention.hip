@@ -17,7 +17,8 @@
 // The splits' partials (m, l, unnormalised O per query row) go to the workspace and are merged in split order
 // (the leader side of the reference: global max, rescale, sum, normalise, kernels/attn_leader_writer.cpp:
 // 86-106 and kernels/attn_leader_compute.cpp:42-79) by the last workgroup of the (user, KV head) to finish
-// when there are few (AttnArgs::merge), else by a separate merge launch, so results are identical run to run.
+// when the one-token kernel's splits are few (merge_here), else by a separate merge launch, so results are identical run
+// to run. Splits past a user's pages take no part (split_live).
 #include <algorithm>
 #include <type_traits>
 
@@ -31,15 +32,9 @@ constexpr int BLK = 64;
 // than the default policy at batch 8 / 4096 positions and at batch 1 / 32768)
 constexpr int NT = 2;
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c,
-                                           false);
-}
 
 struct AttnArgs {
     const uint16_t *q;                  // [B, T, NQ, HD]
@@ -343,9 +338,10 @@ __device__ __forceinline__ void merge_in_launch(const AttnArgs &a, int G, int b,
 // and the second product costs 3% (B 4 / 4100 positions / T 8 / pps 8: 33.7 against 32.5 us a layer).
 // Bound by the chain of a page: about 7000 cycles a page pair (stamps: K requests and scores 2000, maxima and
 // barrier 1500, V and P into LDS 2000, P V 1400), both waves of a SIMD in the same phase; the scores of pages
-// without new rows skip the masks. Measured per layer, G 6: B 4 / 4100 positions ragged / T 8 / pps 8 163 -> 35 us
-// against VALU dot products with two tokens a pass; B 1 / 8192 / T 4 / pps 2 with the mixer 24.9 -> 21.7 us against
-// the pages one at a time with a scaled product per 16-row slice (17.4 us without the mixer either way).
+// without new rows skip the masks. Measured per layer, G 6, with the pages a workgroup walks and their groups as they
+// are now chosen: B 4 / 4100 positions ragged / T 8 / pps 8 163 -> 30 us against VALU dot products with two tokens a
+// pass; B 1 / 8192 / T 4 / pps 2 24.9 -> 18.8 us with the mixer, 17.4 -> 15.9 without, against the pages one at a time with
+// a scaled product per 16-row slice.
 // The step's new rows (mixer: k normalised and rotated) are requested with the query rows and staged in LDS by
 // the workgroups whose split holds their pages; they take the place of the pool's rows as the page is used (K in
 // the score operand's registers, V as it is staged) and go to the pool after the page loop, so nothing waits for
@@ -716,8 +712,7 @@ __global__ __launch_bounds__(256 * WPP, 2) void attn_rows_kernel(AttnArgs a, int
     if constexpr (WPP == 2) __syncthreads();
 
     // this wave's head dims of the group's tiles of the split's partial (or of the output); the partials are
-    // written through to the agent-coherent level (sc1), where another workgroup of this launch or the merge
-    // launch reads them
+    // written through to the agent-coherent level (sc1), where the merge launch reads them
     const auto rpo = __builtin_amdgcn_make_buffer_rsrc(a.part_o + prow(a, G, b, g, split, 0) * HD, (short)0,
                                                        R * HD * 4, 0x00020000);
     const auto rpm = __builtin_amdgcn_make_buffer_rsrc(a.part_ml + prow(a, G, b, g, split, 0) * 2, (short)0,
