@@ -33,9 +33,10 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 def _stream(dev):
     """The current stream's handle on ``dev``."""
-    if _raw_stream is None or dev.index is None:
+    try:
+        return _raw_stream(dev.index)
+    except TypeError:  # no such call, or a device without an index
         return torch.cuda.current_stream(dev).cuda_stream
-    return _raw_stream(dev.index)
 
 
 def _chk(t, name, dtype, shape=None, dev=None):
@@ -449,19 +450,12 @@ def paged_fill_cache(cache, x, page_table, batch_idx=0):
 
 
 @functools.lru_cache(maxsize=1024, typed=True)
-def _walk(B, T, nq, nkv, max_blocks, pages_per_split, mixer):
-    """The pages a workgroup is best given to walk, at most the caller's, and the bytes of a workspace for them."""
+def _pages(B, T, nq, nkv, max_blocks, pages_per_split, mixer, ws_bytes):
+    """Pages per split of a launch: the best ones, at most the caller's, where the workspace holds their partials, else the
+    caller's (a buffer too small for them may be given where the caller's own split needs none)."""
     pages = lib().qs_paged_attention_walk_pages(B, T, nq, nkv, max_blocks, pages_per_split, mixer)
-    return pages, lib().qs_paged_attention_workspace_bytes(B, T, nq, nkv, HD, max_blocks, pages_per_split)
-
-
-def _pages(B, T, nq, nkv, max_blocks, pages_per_split, mixer, ws):
-    """Pages per split of a launch: the best ones where ``ws`` holds their partials, else as the caller says (a buffer
-    too small for them may be given where the caller's own split needs none)."""
-    if ws is None:
-        return pages_per_split
-    pages, nbytes = _walk(B, T, nq, nkv, max_blocks, pages_per_split, mixer)
-    return pages if ws.nbytes >= nbytes else pages_per_split
+    nbytes = lib().qs_paged_attention_workspace_bytes(B, T, nq, nkv, HD, max_blocks, pages_per_split)
+    return pages if ws_bytes >= nbytes else pages_per_split
 
 
 def attention_workspace(B, T, nq, nkv, max_blocks, pages_per_split, device):
@@ -496,7 +490,9 @@ def paged_gqa_decode(q, k_cache, v_cache, block_table, seq_lens, scale, k_new=No
     _chk(o, "out", torch.bfloat16, (B, T, nq, hd), dev)
     if ws is None and (mb + pages_per_split - 1) // pages_per_split > 1:
         ws = attention_workspace(B, T, nq, nkv, mb, pages_per_split, dev)
-    pps = _pages(B, T, nq, nkv, mb, int(pages_per_split), False, ws)
+    pps = int(pages_per_split)
+    if ws is not None:
+        pps = _pages(B, T, nq, nkv, mb, pps, False, ws.nbytes)
     call("qs_paged_gqa_decode", _p(q), _p(k_new), _p(v_new), _p(k_cache), _p(v_cache), _p(block_table),
          _p(seq_lens), _p(o), _p(ws), B, T, nq, nkv, hd, block, mb, nb, pps, float(scale),
          _p(status), _stream(dev))  # fmt: skip
@@ -641,7 +637,7 @@ def attn_mixer_decode(q, k_new, v_new, gate, wq, wk, cos, sin, k_cache, v_cache,
     o = torch.empty(B, T, nq, hd, dtype=torch.bfloat16, device=dev) if out is None else out
     if ws is None:
         ws = attention_workspace(B, T, nq, nkv, mb, pages_per_split, dev)
-    pps = _pages(B, T, nq, nkv, mb, pages_per_split, True, ws)
+    pps = _pages(B, T, nq, nkv, mb, pages_per_split, True, ws.nbytes)
     call("qs_attn_mixer_decode", _p(q), _p(k_new), _p(v_new), _p(gate), _p(wq), _p(wk),
          _p(cos if rot else None), _p(sin if rot else None), rot, _p(k_cache), _p(v_cache), _p(block_table),
          _p(seq_lens), _p(o), _p(ws), B, T, nq, nkv, hd, block, mb, nb, pps, float(eps), _p(status),
