@@ -1318,19 +1318,19 @@ int rows_tiles(int R) {
 bool rows_pairs(int R, int T, bool mixer) { return !mixer || rows_tiles(R) == 2 || (rows_tiles(R) == 3 && T <= 8); }
 
 int nsplit_of(int max_blocks, int pps) { return (max_blocks + pps - 1) / pps; }
-// Pages a workgroup is best given to walk: the caller's, or as few as keep the whole launch within one workgroup per CU (an even number
-// past one, for the two pages in flight). A page takes its waves ~2 us of dependent latency (load, scores, softmax,
-// P V), so a grid that leaves CUs idle is cut finer; past 256 workgroups the partials cost more than the shorter walks
-// save. Per layer with the mixer, the caller's pages -> the rule's: batch 1, 8 pages: 200 positions 13.0 -> 11.4 us (4
+// Pages a workgroup is best given to walk: the caller's, or as few as keep the whole launch within one workgroup per CU
+// (an even number past one, for the two pages in flight). A page takes its waves ~2 us of dependent latency (load, scores,
+// softmax, P V), so a grid that leaves CUs idle is cut finer; past 256 workgroups the partials cost more than the shorter
+// walks save. Per layer with the mixer, the caller's pages -> the rule's: batch 1, 8 pages: 200 positions 13.0 -> 11.4 us (4
 // workgroups -> 16), 1000 19.1 -> 12.3, 4096 19.7 -> 13.2; 16 pages, 2000: 26.4 -> 11.0; batch 4, 8 pages, ragged
 // 1000: 19.3 -> 13.7; batch 1 / 4 tokens, 8 pages, 1000: 29.5 -> 15.2. One step finer than the rule: batch 1 / 8192
 // 18.6 against 16.1, batch 4 / 4096 26.4 against 20.4, batch 8 / 2048 27.7 against 18.6. Only sizes known to the host
 // enter the rule, so a user's result depends on no other user's length.
-// A table of few pages stays whole (if the caller's pages allow it): two pages are walked at once, and without a second
-// split there is no merge. One split against a page per split: one token, batch 1, 2 / 3 / 4 pages 7.8, 8.7, 9.5 against
-// 8.8, 8.9, 8.8 us, 3 pages at batch 8 9.8 against 9.4, with the mixer 10.6 against 10.4; two tokens, batch 1, 2 / 3 / 4
-// pages 7.9, 8.9, 9.7 against 9.8, 9.9, 10.0, 4 pages at batch 8 10.9 against 10.5; four tokens (rows kernel) 2 / 3 pages
-// 9.7, 12.0 against 11.2, 11.2; where the rows kernel walks one page at a time (rows_pairs), 11 tokens with the mixer, 2
+// A table of few pages stays whole (if the caller's pages allow it): without a second split there is no merge. One split
+// against a page per split: one token, batch 1, 2 / 3 / 4 pages 7.8, 8.7, 9.5 against 8.8, 8.9, 8.8 us, 3 pages at batch 8
+// 9.8 against 9.4, with the mixer 10.6 against 10.4; two tokens, batch 1, 2 / 3 / 4 pages 7.9, 8.9, 9.7 against 9.8, 9.9,
+// 10.0, 4 pages at batch 8 10.9 against 10.5; the rows kernel, four tokens, 2 / 3 pages 9.2, 11.0 against 11.0, 11.1, eight
+// 12.0, 14.9 against 13.3, 13.5; where its LDS has no room for two page groups (rows_pairs), 11 tokens with the mixer, 2
 // pages 20.8 against 18.4.
 constexpr int FINE_WGS = 256;
 int walk_pages(int B, int T, int NKV, int G, int max_blocks, int pps, bool mixer) {
